@@ -93,13 +93,13 @@ constexpr ComboTables build_combo_tables()
 static constexpr ComboTables kCombos = build_combo_tables();
 static __constant__ ComboTables c_combos = build_combo_tables();
 
-__host__ __device__ inline int popcount4(unsigned m)
+__host__ __device__ constexpr int popcount4(unsigned m)
 {
     return static_cast<int>((m & 1u) + ((m >> 1) & 1u) + ((m >> 2) & 1u) + ((m >> 3) & 1u));
 }
 
 // parity of the concatenated index list (src ‖ dst): +1 even, -1 odd
-__host__ __device__ inline int concat_sign(unsigned src, unsigned dst, int n)
+__host__ __device__ constexpr int concat_sign(unsigned src, unsigned dst, int n)
 {
     int ids[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     int m = 0;
@@ -162,6 +162,12 @@ struct DevGeom {
     int64_t ext[SIL_MAX_DIM];
     const double* axis[SIL_MAX_DIM]; // device coordinates (rectilinear)
     const double* nodal;             // device [node][ndim] (general)
+    // rectilinear: edge length per node (forward, backward at the last node)
+    // and its reciprocal, device; regular: finite and far enough from zero
+    // that no node is degenerate for any degree
+    const double* spacing[SIL_MAX_DIM];
+    const double* inv_spacing[SIL_MAX_DIM];
+    bool regular;
     int metric_kind;
     const double* metric;
 };
@@ -172,4 +178,5 @@ struct sil_grid_s {
     sil::DevGeom geom;
     double* axis_storage[SIL_MAX_DIM]; // device copies of the axis coordinates
     double* spacing[SIL_MAX_DIM];      // device per-node edge lengths (rectilinear)
+    double* inv_spacing[SIL_MAX_DIM];  // device reciprocals of spacing (one allocation with it)
 };

@@ -4,7 +4,8 @@
 // diagonal / symmetric metrics.  One thread per output node; every
 // intermediate (dω, ⋆, dᵀ, δω) is re-evaluated where it is needed, so no
 // workspace is ever allocated.  The fused kernels in dec_fused.hip serve the
-// hot shapes; these serve everything else.
+// hot shapes, those of dec_rect.hip regular rectilinear grids with identity
+// or diagonal metric; these serve everything else.
 #include "dec_kernels.hpp"
 #include "geometry.hpp"
 
@@ -334,6 +335,8 @@ int launch_coboundary(int k, bool transposed, const double* in, const sil_view& 
 {
     int64_t total = view_nodes(vout) * view_batches(vout);
     if (total == 0) return SIL_OK;
+    if (!transposed && rect_views_ok(vin, vout))
+        return launch_rect(RectOp::Coboundary, k, nullptr, in, vin, out, vout, stream);
     const int block = 256;
     hipLaunchKernelGGL(k_coboundary, dim3(grid_for(total, block)), dim3(block), 0, stream, k, transposed ? 1 : 0, in,
                        to_dev(vin), out, to_dev(vout), total);
@@ -356,6 +359,8 @@ int launch_hodge_apply(const DevGeom& g, int k, const double* in, const sil_view
 {
     int64_t nodes = 1;
     for (int a = 0; a < g.ndim; ++a) nodes *= g.ext[a];
+    if (rect_geom_ok(g) && rect_views_ok(vin, vout))
+        return launch_rect(RectOp::Hodge, k, &g, in, vin, out, vout, stream);
     const int block = 128;
     hipLaunchKernelGGL(k_hodge_apply, dim3(grid_for(nodes, block)), dim3(block), 0, stream, g, k, in, to_dev(vin),
                        out, to_dev(vout), nodes);
@@ -368,6 +373,8 @@ int launch_codifferential(const DevGeom& g, int k, const double* in, const sil_v
 {
     int64_t total = view_nodes(vout);
     if (total == 0) return SIL_OK;
+    if (rect_geom_ok(g) && rect_views_ok(vin, vout))
+        return launch_rect(RectOp::Codifferential, k, &g, in, vin, out, vout, stream);
     const int block = 128;
     hipLaunchKernelGGL(k_codifferential, dim3(grid_for(total, block)), dim3(block), 0, stream, g, k, in, to_dev(vin),
                        out, to_dev(vout), total);
@@ -380,6 +387,8 @@ int launch_laplacian_generic(const DevGeom& g, int k, const double* in, const si
 {
     int64_t total = view_nodes(vout);
     if (total == 0) return SIL_OK;
+    if (rect_geom_ok(g) && rect_views_ok(vin, vout))
+        return launch_rect(RectOp::Laplacian, k, &g, in, vin, out, vout, stream);
     const int block = 128;
     hipLaunchKernelGGL(k_laplacian, dim3(grid_for(total, block)), dim3(block), 0, stream, g, k, in, to_dev(vin), out,
                        to_dev(vout), total);

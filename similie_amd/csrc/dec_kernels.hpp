@@ -15,6 +15,18 @@ int launch_codifferential(const DevGeom& g, int k, const double* in, const sil_v
 int launch_laplacian_generic(const DevGeom& g, int k, const double* in, const sil_view& vin, double* out,
                              const sil_view& vout, hipStream_t stream);
 
+// The same operators with the dimension and the degree as template constants
+// (dec_rect.hip): rectilinear grids of regular spacings with identity or
+// diagonal metric, N ≤ 3.  `g` is null for the coboundary.
+enum class RectOp { Coboundary, Hodge, Codifferential, Laplacian };
+bool rect_views_ok(const sil_view& vin, const sil_view& vout);
+inline bool rect_geom_ok(const DevGeom& g)
+{
+    return g.rectilinear && g.regular && g.metric_kind != SIL_METRIC_SYMMETRIC;
+}
+int launch_rect(RectOp op, int k, const DevGeom* g, const double* in, const sil_view& vin, double* out,
+                const sil_view& vout, hipStream_t stream);
+
 // Fused single-pass Laplacians on rectilinear grids with identity or diagonal
 // metric, index-last dense arrays.  `spacing[a]` holds the per-node edge
 // length along axis a (forward, backward at the last node).
