@@ -245,6 +245,41 @@ def test_unet_backward_on_gpu_activations(learned):
     assert max(errs) <= GRAD_TOL_GPU_ACTIVATIONS, errs
 
 
+@pytest.mark.parametrize("shape", [(1, 8, 8), (3, 8, 24), (2, 40, 16), (7, 64, 56)])
+def test_unet_end_layer_gradients(learned, shape):
+    """The weight gradients of the output and the input layer at the edges of
+    their split (one 64-pixel step, images smaller than the grid, many
+    images): the output layer's from the GPU's own c0 in FP64, every block
+    against the emulating oracle on the GPU's activations.  The output
+    layer's terms are exact products of FP32 and BF16 summed in FP32: a tree
+    of n terms is off by at most (log2 n + 8) roundings of 2^-24 of the sum
+    of magnitudes, 2e-6 for these sizes."""
+    B, H, W = shape
+    rng = np.random.default_rng(B + H + W)
+    params = make_params(rng)
+    x = rng.standard_normal((B, H, W, 2)).astype(np.float32)
+    dout = rng.standard_normal((B, H, W)).astype(np.float32)
+    net = learned.UNet(B, H, W, seed=1)
+    net.set_params(torch.from_numpy(params))
+    xt = torch.from_numpy(x).cuda()
+    net.forward(xt)
+    _, act = U.forward(params.astype(np.float64), x, emulate=True)
+    a = _layer_inputs(net, act, B)
+    g = net.backward(xt, torch.from_numpy(dout).cuda()).cpu().numpy()
+    c0 = np.pad(net.activation("c0", B).cpu().numpy().astype(np.float64), ((0, 0), (1, 1), (1, 1), (0, 0)))
+    d = dout.astype(np.float64)
+    for t in range(9):
+        dy, dx = divmod(t, 3)
+        terms = d[..., None] * c0[:, dy:dy + H, dx:dx + W, :]
+        got = g[U.OUT_BASE + t * U.C: U.OUT_BASE + (t + 1) * U.C]
+        bound = 2e-6 * np.abs(terms).sum(axis=(0, 1, 2)) + 1e-30
+        assert np.all(np.abs(got - terms.sum(axis=(0, 1, 2))) <= bound), t
+    assert abs(g[U.OUT_BASE + 9 * U.C] - d.sum()) <= 2e-6 * np.abs(d).sum()
+    g_ref = U.backward(params.astype(np.float64), a, dout, emulate=True)
+    assert rel(g[: U.N_IN], g_ref[: U.N_IN]) <= GRAD_TOL_GPU_ACTIVATIONS
+    assert rel(g[U.layer_slices(12)[0]], g_ref[U.layer_slices(12)[0]]) <= GRAD_TOL_GPU_ACTIVATIONS
+
+
 def test_unet_direction_loss_matches_oracle(learned):
     B, n = 2, 32
     rng = np.random.default_rng(31)
