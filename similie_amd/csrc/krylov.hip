@@ -3,15 +3,21 @@
 // The reference hands its matrix-free operator to Ginkgo's CG
 // (src/similie/solvers/minimize_strong_formulation_residual.hpp:1028-1304),
 // which synchronises with the host at every iteration for its ResidualNorm
-// stopping criterion.  Here one iteration is four kernels —
-//   K1 p = z + β p_old fused into q = A p with per-block ⟨p, q⟩ partials,
-//   K2 α = ⟨r, z⟩ / ⟨p, q⟩,
-//   K3 x += α p, r −= α q with per-block ⟨r, z⟩ and ⟨r, r⟩ partials,
-//   K4 β, the stopping test ‖r‖2 ≤ tol·‖b‖2 and the iteration counter —
-// every scalar stays in device memory, every kernel returns at once when the
-// device `done` flag is set, and a chunk of iterations is captured once into a
-// hipGraph and replayed; the host reads the flag once per chunk.  Partial sums
-// are reduced in a fixed order, so a solve is bit-reproducible.
+// stopping criterion.  Here an iteration is
+//   K1 p = z + β p_old and q = A p with per-block ⟨p, q⟩ partials (one kernel
+//      for the 2D Poisson operator, two for the curl-curl operator),
+//   K2 α = ⟨r, z⟩ / ⟨p, q⟩, x += α p, r −= α q with per-block ⟨r, z⟩ and ⟨r, r⟩
+//      partials,
+// and the partials of one are summed by every workgroup of the other
+// (reduce_all, cg_begin): β, the stopping test ‖r‖2 ≤ tol·‖b‖2 and the
+// iteration counter in K1 of the next iteration, α in K2.  A kernel of one
+// workgroup for each of the two (k_alpha, k_beta, still used where an
+// operator's partials are too many or K1 cannot sum them) took 4.5 µs a time,
+// more than the vectors of a small system.  Every scalar stays in device
+// memory, every kernel returns at once when the solve is over, and a chunk of
+// iterations, ended by a kernel that settles the scalars, is captured once
+// into a hipGraph and replayed; the host reads the flag once per chunk.
+// Partial sums are reduced in a fixed order, so a solve is bit-reproducible.
 //
 // Mixed precision: the recurrence (r, p, q) and every operator application
 // inside the loop run in FP32 while x, all dot products and the scalars are
@@ -24,16 +30,11 @@
 #include <cmath>
 #include <mutex>
 #include <new>
+#include <type_traits>
 
-#include "operators.hpp"
+#include "apply_epilogue.hpp"
 
 namespace sil {
-
-struct CgScalars {
-    double rz, rz_prev, pq, alpha, beta, rr, bb, tol2bb;
-    double rr_true;
-    int done, iter, max_iter, converged;
-};
 
 struct Workspace {
     int64_t n = 0;
@@ -46,6 +47,7 @@ struct Workspace {
     float *r32 = nullptr, *q32 = nullptr, *p32[2] = {nullptr, nullptr};
     float *inv_diag32 = nullptr, *xc32 = nullptr;
     double* partials = nullptr; // [3][part_stride]
+    double* upart = nullptr;    // single-pass iteration: ⟨r, z⟩, ⟨r, r⟩ partials [slot][2][kUpdBlocks]
     int64_t part_stride = 0;    // slots per partial-sum array
     CgScalars* sc = nullptr;
     CgScalars* host_sc = nullptr; // pinned
@@ -68,6 +70,16 @@ namespace {
 constexpr int kUpdBlock = 256;
 constexpr int kUpdBlocks = 2048;
 constexpr int kRedThreads = 1024;
+// most partials of an operator application that every workgroup of the update
+// sums itself
+constexpr int kMaxSharedPartials = 2048;
+
+// workgroups of an update over n rows: four rows a thread, at most 1024, so
+// that the next kernel sums few partials
+inline int update_blocks(int64_t n)
+{
+    return (int)std::max<int64_t>(1, std::min<int64_t>((n + 4 * kUpdBlock - 1) / (4 * kUpdBlock), 1024));
+}
 
 __device__ double block_sum(double v)
 {
@@ -182,38 +194,17 @@ __global__ void k_alpha(CgScalars* sc, const double* part, int count)
     }
 }
 
-// XC: x accumulates in the FP32 correction xc (folded into the FP64 x at
-// every residual replacement) instead of in x itself
-template <typename T, bool XC = false>
-__global__ __launch_bounds__(kUpdBlock) void k_update(const CgScalars* __restrict__ sc, double* __restrict__ x,
-                                                      const T* __restrict__ p, T* __restrict__ r,
-                                                      const T* __restrict__ q, const T* __restrict__ inv_diag,
-                                                      int64_t n, double* __restrict__ part_rz,
-                                                      double* __restrict__ part_rr, float* __restrict__ xc)
+// per-block sums of (a, b) → pa[block], pb[block]
+__device__ __forceinline__ void store_two_sums(double a, double b, double* __restrict__ pa, double* __restrict__ pb)
 {
-    if (sc->done) return;
-    const double alpha = sc->alpha;
-    const float alpha32 = (float)alpha;
-    double vz = 0.0, vr = 0.0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        if constexpr (XC)
-            xc[i] = fmaf(alpha32, (float)p[i], xc[i]);
-        else
-            x[i] += alpha * (double)p[i];
-        const T ri = (T)((double)r[i] - alpha * (double)q[i]);
-        r[i] = ri;
-        const double rd = (double)ri;
-        vr += rd * rd;
-        vz += rd * (inv_diag ? rd * (double)inv_diag[i] : rd);
-    }
     __shared__ double sh[2][kUpdBlock / 64];
     for (int off = 32; off > 0; off >>= 1) {
-        vz += __shfl_down(vz, off, 64);
-        vr += __shfl_down(vr, off, 64);
+        a += __shfl_down(a, off, 64);
+        b += __shfl_down(b, off, 64);
     }
     if ((threadIdx.x & 63) == 0) {
-        sh[0][threadIdx.x >> 6] = vz;
-        sh[1][threadIdx.x >> 6] = vr;
+        sh[0][threadIdx.x >> 6] = a;
+        sh[1][threadIdx.x >> 6] = b;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -222,9 +213,89 @@ __global__ __launch_bounds__(kUpdBlock) void k_update(const CgScalars* __restric
             s0 += sh[0][i];
             s1 += sh[1][i];
         }
-        part_rz[blockIdx.x] = s0;
-        part_rr[blockIdx.x] = s1;
+        pa[blockIdx.x] = s0;
+        pb[blockIdx.x] = s1;
     }
+}
+
+// Where an update takes α from: sc->alpha (k_alpha has formed it; part null), or
+// ⟨r, z⟩ at rz over the sum of `count` partials of ⟨p, q⟩.  Over when *stop.
+struct AlphaSource {
+    const int* stop;
+    const double* rz;
+    const double* part;
+    int count;
+};
+
+// XC: x accumulates in the FP32 correction xc (folded into the FP64 x at
+// every residual replacement) instead of in x itself.  The solver's vectors
+// move in 16-byte accesses; so does x with XVEC (in a solve without allocation
+// x is the caller's array, which need not be aligned).
+template <typename T, bool XC, bool XVEC>
+__global__ __launch_bounds__(kUpdBlock) void k_update(const CgScalars* __restrict__ sc, AlphaSource as,
+                                                      double* __restrict__ x, const T* __restrict__ p,
+                                                      T* __restrict__ r, const T* __restrict__ q,
+                                                      const T* __restrict__ inv_diag, int64_t n,
+                                                      double* __restrict__ part_rz, double* __restrict__ part_rr,
+                                                      float* __restrict__ xc)
+{
+    if (*as.stop) return;
+    double alpha;
+    if (as.part) {
+        double pq[1];
+        reduce_all<kUpdBlock, 1>({as.part}, {as.count}, pq);
+        alpha = *as.rz / pq[0];
+    } else {
+        alpha = sc->alpha;
+    }
+    const float alpha32 = (float)alpha;
+    double vz = 0.0, vr = 0.0;
+    auto row = [&](T& ri, T qi, T di) {
+        ri = (T)((double)ri - alpha * (double)qi);
+        const double rd = (double)ri;
+        vr += rd * rd;
+        vz += rd * (inv_diag ? rd * (double)di : rd);
+    };
+    constexpr int V = 16 / (int)sizeof(T);
+    typedef T Vec __attribute__((ext_vector_type(V)));
+    const int64_t stride = (int64_t)gridDim.x * kUpdBlock, t = blockIdx.x * (int64_t)kUpdBlock + threadIdx.x;
+    const int64_t nv = n / V;
+    for (int64_t i = t; i < nv; i += stride) {
+        const Vec pv = reinterpret_cast<const Vec*>(p)[i], qv = reinterpret_cast<const Vec*>(q)[i];
+        Vec rv = reinterpret_cast<Vec*>(r)[i], dv = rv;
+        if (inv_diag) dv = reinterpret_cast<const Vec*>(inv_diag)[i];
+        if constexpr (XC) {
+            Vec xv = reinterpret_cast<Vec*>(xc)[i];
+#pragma unroll
+            for (int u = 0; u < V; ++u) xv[u] = fmaf(alpha32, (float)pv[u], xv[u]);
+            reinterpret_cast<Vec*>(xc)[i] = xv;
+        } else if constexpr (XVEC) {
+            Vec xv = reinterpret_cast<Vec*>(x)[i];
+#pragma unroll
+            for (int u = 0; u < V; ++u) xv[u] += alpha * (double)pv[u];
+            reinterpret_cast<Vec*>(x)[i] = xv;
+        } else {
+#pragma unroll
+            for (int u = 0; u < V; ++u) x[i * V + u] += alpha * (double)pv[u];
+        }
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            T ri = rv[u];
+            row(ri, qv[u], dv[u]);
+            rv[u] = ri;
+        }
+        reinterpret_cast<Vec*>(r)[i] = rv;
+    }
+    for (int64_t i = nv * V + t; i < n; i += stride) {
+        if constexpr (XC)
+            xc[i] = fmaf(alpha32, (float)p[i], xc[i]);
+        else
+            x[i] += alpha * (double)p[i];
+        T ri = r[i];
+        row(ri, q[i], inv_diag ? inv_diag[i] : T(1));
+        r[i] = ri;
+    }
+    store_two_sums(vz, vr, part_rz, part_rr);
 }
 
 __global__ void k_beta(CgScalars* sc, const double* part_rz, int count_rz, const double* part_rr, int count_rr)
@@ -247,90 +318,21 @@ __global__ void k_beta(CgScalars* sc, const double* part_rz, int count_rz, const
     }
 }
 
-// ---- single-pass FP32 iteration (3D curl-curl operator) ----
-//
-// The march that forms q = A p also sums ⟨q, z⟩ and ⟨q, D⁻¹ q⟩ (z = D⁻¹ r), so
-// the next ⟨r, z⟩ is known before r is updated:
-//   γ' = ⟨r − αq, D⁻¹(r − αq)⟩ = γ − 2α⟨q, z⟩ + α²⟨q, D⁻¹ q⟩,  β' = γ'/γ,
-// and one streaming pass updates r, the iterate and the next direction
-// p' = D⁻¹ r' + β' p together; it also sums the exact ⟨r', z'⟩ (the next α
-// uses it) and ⟨r', r'⟩.  Per iteration: the march and one vector pass, where
-// the standard iteration has the march, the update and the direction pass.
-
-// α = γ / ⟨p, q⟩ and β' from the expansion; three partial arrays at stride
-__global__ void k_alpha_expand(CgScalars* sc, const double* part, int64_t stride, int count)
+// The end of a chunk whose kernels finish each other's iterations: the last
+// iteration's partials, as k_beta; `slot` is that iteration's.
+__global__ void k_settle(CgScalars* sc, int slot, const double* part_rz, const double* part_rr, int count,
+                         bool keep_beta)
 {
-    if (sc->done) return;
-    const double pq = reduce_partials(part, count);
-    const double qz = reduce_partials(part + stride, count);
-    const double qq = reduce_partials(part + 2 * stride, count);
+    if (sc->stops[slot]) return;
+    const double rz = reduce_partials(part_rz, count);
+    const double rr = reduce_partials(part_rr, count);
     if (threadIdx.x == 0) {
-        const double g = sc->rz;
-        const double alpha = g / pq;
-        const double gn = g - 2.0 * alpha * qz + alpha * alpha * qq;
-        sc->pq = pq;
-        sc->alpha = alpha;
-        sc->beta = gn / g;
-    }
-}
-
-// r' = r − αq; xc += αp; p' = D⁻¹ r' + β' p (arithmetic of p_value); partials
-// of ⟨r', z'⟩ and ⟨r', r'⟩
-__global__ __launch_bounds__(kUpdBlock) void k_update_dir(const CgScalars* __restrict__ sc,
-                                                          const float* __restrict__ p, float* __restrict__ pn,
-                                                          float* __restrict__ r, const float* __restrict__ q,
-                                                          const float* __restrict__ inv_diag, int64_t n,
-                                                          double* __restrict__ part_rz, double* __restrict__ part_rr,
-                                                          float* __restrict__ xc)
-{
-    if (sc->done) return;
-    const double alpha = sc->alpha, beta = sc->beta;
-    const float alpha32 = (float)alpha;
-    double vz = 0.0, vr = 0.0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float pi = p[i];
-        xc[i] = fmaf(alpha32, pi, xc[i]);
-        const float ri = (float)((double)r[i] - alpha * (double)q[i]);
-        r[i] = ri;
-        const double rd = (double)ri;
-        const double z = inv_diag ? rd * (double)inv_diag[i] : rd;
-        pn[i] = (float)(z + beta * (double)pi);
-        vr += rd * rd;
-        vz += rd * z;
-    }
-    __shared__ double sh[2][kUpdBlock / 64];
-    for (int off = 32; off > 0; off >>= 1) {
-        vz += __shfl_down(vz, off, 64);
-        vr += __shfl_down(vr, off, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        sh[0][threadIdx.x >> 6] = vz;
-        sh[1][threadIdx.x >> 6] = vr;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s0 = 0.0, s1 = 0.0;
-        for (int i = 0; i < kUpdBlock / 64; ++i) {
-            s0 += sh[0][i];
-            s1 += sh[1][i];
-        }
-        part_rz[blockIdx.x] = s0;
-        part_rr[blockIdx.x] = s1;
-    }
-}
-
-// the exact ⟨r', z'⟩ and ⟨r', r'⟩: the next α, the stopping test (β' was
-// taken from the expansion)
-__global__ void k_gamma(CgScalars* sc, const double* part_rz, int count_rz, const double* part_rr, int count_rr)
-{
-    if (sc->done) return;
-    const double rz = reduce_partials(part_rz, count_rz);
-    const double rr = reduce_partials(part_rr, count_rr);
-    if (threadIdx.x == 0) {
-        sc->rz_prev = sc->rz;
+        const double prev = sc->rzs[slot];
+        if (!keep_beta) sc->beta = rz / prev;
+        sc->rz_prev = prev;
         sc->rz = rz;
         sc->rr = rr;
-        sc->iter += 1;
+        sc->iter = sc->iters[slot] + 1;
         if (rr <= sc->tol2bb) {
             sc->done = 1;
             sc->converged = 1;
@@ -338,6 +340,115 @@ __global__ void k_gamma(CgScalars* sc, const double* part_rz, int count_rz, cons
             sc->done = 1;
         }
     }
+}
+
+// ---- single-pass FP32 iteration (3D curl-curl operator) ----
+//
+// The march that forms q = A p also sums ⟨q, z⟩ and ⟨q, D⁻¹ q⟩ (z = D⁻¹ r), so
+// the next ⟨r, z⟩ is known before r is updated:
+//   γ' = ⟨r − αq, D⁻¹(r − αq)⟩ = γ − 2α⟨q, z⟩ + α²⟨q, D⁻¹ q⟩,  β' = γ'/γ,
+// and one streaming pass updates r, the iterate and the next direction
+// p' = D⁻¹ r' + β' p together; it also sums the exact ⟨r', z'⟩ (the next α
+// uses it) and ⟨r', r'⟩.  Per iteration: the march and one vector pass (which
+// also finishes the iteration before), where the standard iteration has the
+// march, the update and the direction pass.
+
+// One iteration after its march: γ, ⟨r, r⟩ and the stopping test of the
+// iteration before from its partials (first: the chunk starts from settled
+// scalars), α = γ / ⟨p, q⟩ and β' from the march's three partial arrays (at
+// mstride), then r' = r − αq; xc += αp; p' = D⁻¹ r' + β' p (arithmetic of
+// p_value) and the partials of ⟨r', z'⟩ and ⟨r', r'⟩ into the iteration's own
+// slot.  Every workgroup sums the partials; workgroup 0 records the scalars.
+__global__ __launch_bounds__(kUpdBlock) void k_update_dir(CgScalars* __restrict__ sc, int slot, bool first,
+                                                          const double* __restrict__ prev_parts, int prev_count,
+                                                          const double* __restrict__ march, int64_t mstride,
+                                                          int mcount, const float* __restrict__ p,
+                                                          float* __restrict__ pn, float* __restrict__ r,
+                                                          const float* __restrict__ q,
+                                                          const float* __restrict__ inv_diag, int64_t n,
+                                                          double* __restrict__ parts, float* __restrict__ xc)
+{
+    const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+    double g, pq, qz, qq;
+    if (first) {
+        if (sc->done) {
+            if (writer) sc->stops[slot] = 1;
+            return;
+        }
+        double v[3];
+        reduce_all<kUpdBlock, 3>({march, march + mstride, march + 2 * mstride}, {mcount, mcount, mcount}, v);
+        g = sc->rz;
+        pq = v[0], qz = v[1], qq = v[2];
+        if (writer) {
+            sc->iters[slot] = sc->iter;
+            sc->stops[slot] = 0;
+            sc->rzs[slot] = g;
+        }
+    } else {
+        if (sc->stops[slot ^ 1]) {
+            if (writer) sc->stops[slot] = 1;
+            return;
+        }
+        double v[5];
+        reduce_all<kUpdBlock, 5>({march, march + mstride, march + 2 * mstride, prev_parts, prev_parts + kUpdBlocks},
+                                 {mcount, mcount, mcount, prev_count, prev_count}, v);
+        pq = v[0], qz = v[1], qq = v[2], g = v[3];
+        const double rr = v[4];
+        const int it = sc->iters[slot ^ 1] + 1;
+        const bool conv = rr <= sc->tol2bb, stop = conv || it >= sc->max_iter;
+        if (writer) {
+            sc->iters[slot] = it;
+            sc->stops[slot] = stop ? 1 : 0;
+            sc->rzs[slot] = g;
+            sc->rz_prev = sc->rzs[slot ^ 1];
+            sc->rz = g;
+            sc->rr = rr;
+            sc->iter = it;
+            if (stop) {
+                sc->done = 1;
+                if (conv) sc->converged = 1;
+            }
+        }
+        if (stop) return;
+    }
+    const double alpha = g / pq;
+    const double beta = (g - 2.0 * alpha * qz + alpha * alpha * qq) / g;
+    const float alpha32 = (float)alpha;
+    double vz = 0.0, vr = 0.0;
+    auto row = [&](float pi, float& ri, float qi, float di) -> float {
+        ri = (float)((double)ri - alpha * (double)qi);
+        const double rd = (double)ri;
+        const double z = inv_diag ? rd * (double)di : rd;
+        vr += rd * rd;
+        vz += rd * z;
+        return (float)(z + beta * (double)pi);
+    };
+    typedef float F4 __attribute__((ext_vector_type(4)));
+    const int64_t stride = (int64_t)gridDim.x * kUpdBlock, t = blockIdx.x * (int64_t)kUpdBlock + threadIdx.x;
+    const int64_t nv = n / 4;
+    for (int64_t i = t; i < nv; i += stride) {
+        const F4 pv = reinterpret_cast<const F4*>(p)[i], qv = reinterpret_cast<const F4*>(q)[i];
+        F4 rv = reinterpret_cast<F4*>(r)[i], xv = reinterpret_cast<F4*>(xc)[i], dv = rv, nvv;
+        if (inv_diag) dv = reinterpret_cast<const F4*>(inv_diag)[i];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            xv[u] = fmaf(alpha32, pv[u], xv[u]);
+            float ri = rv[u];
+            nvv[u] = row(pv[u], ri, qv[u], dv[u]);
+            rv[u] = ri;
+        }
+        reinterpret_cast<F4*>(xc)[i] = xv;
+        reinterpret_cast<F4*>(r)[i] = rv;
+        reinterpret_cast<F4*>(pn)[i] = nvv;
+    }
+    for (int64_t i = nv * 4 + t; i < n; i += stride) {
+        const float pi = p[i];
+        xc[i] = fmaf(alpha32, pi, xc[i]);
+        float ri = r[i];
+        pn[i] = row(pi, ri, q[i], inv_diag ? inv_diag[i] : 1.0f);
+        r[i] = ri;
+    }
+    store_two_sums(vz, vr, parts, parts + kUpdBlocks);
 }
 
 // FP64 residual replacement: r64 = b − Ax (tmp = Ax) → r (T), partials of
@@ -546,7 +657,7 @@ int ensure_workspace(sil_operator op, bool mixed, hipStream_t s)
     }
     if (mixed && !w.r32) {
         if ((rc = alloc(&w.r32, n)) || (rc = alloc(&w.q32, n)) || (rc = alloc(&w.p32[0], n)) ||
-            (rc = alloc(&w.p32[1], n)) || (rc = alloc(&w.xc32, n)))
+            (rc = alloc(&w.p32[1], n)) || (rc = alloc(&w.xc32, n)) || (rc = alloc(&w.upart, 4 * kUpdBlocks)))
             return rc;
     }
     return SIL_OK;
@@ -554,11 +665,12 @@ int ensure_workspace(sil_operator op, bool mixed, hipStream_t s)
 
 enum Precond { PC_IDENTITY = 0, PC_JACOBI = 1, PC_ISAI = 2 };
 
-// enqueue one CG iteration; pold / pnew are the p ping-pong buffers.  With
-// SpdIsai the direction is formed from z (not from r) and the update's
-// ⟨r, z⟩ partials are replaced by those of the preconditioner application.
+// Enqueues iterations 0 … chunk − 1 (an even number) of CG on the ping-pong
+// direction buffers p[0], p[1] and leaves the scalars settled.  With SpdIsai
+// the direction is formed from z (not from r) and the update's ⟨r, z⟩ partials
+// are replaced by those of the preconditioner application.
 template <typename T>
-int enqueue_iteration(sil_operator op, Workspace& w, T* r, T* q, T* pold, T* pnew, int pc, hipStream_t s)
+int enqueue_chunk(sil_operator op, Workspace& w, T* r, T* q, T* const* p, int pc, int chunk, hipStream_t s)
 {
     double* part0 = w.partials;
     double* part1 = w.partials + w.part_stride;
@@ -570,43 +682,73 @@ int enqueue_iteration(sil_operator op, Workspace& w, T* r, T* q, T* pold, T* pne
         else
             invd = w.inv_diag32;
     }
-    const T* zsrc = r;
-    if constexpr (sizeof(T) == 8)
-        if (pc == PC_ISAI) zsrc = w.isai_z;
+    const int ub = update_blocks(op->n);
+    int rc, nb = 0;
     if constexpr (sizeof(T) == 4) {
         if (w.single_pass) {
-            // pold holds the current direction p, pnew receives the next one
-            int nb = 0;
+            // p[slot] holds the current direction, p[slot ^ 1] receives the next one
             const NlData* nl = op->kind == OP_MS3D_JACOBIAN ? &op->nl : nullptr;
-            int rc = ms3d_qdots32(op->ms, nl, pold, q, r, invd, part0, w.part_stride, &w.sc->done, &nb, s);
-            if (rc) return rc;
-            hipLaunchKernelGGL(k_alpha_expand, dim3(1), dim3(kRedThreads), 0, s, w.sc, part0, w.part_stride, nb);
-            hipLaunchKernelGGL(k_update_dir, dim3(kUpdBlocks), dim3(kUpdBlock), 0, s, w.sc, pold, pnew, r, q, invd,
-                               op->n, part1, part2, w.xc32);
-            hipLaunchKernelGGL(k_gamma, dim3(1), dim3(kRedThreads), 0, s, w.sc, part1, kUpdBlocks, part2, kUpdBlocks);
+            for (int it = 0; it < chunk; ++it) {
+                const int slot = it & 1;
+                double* mine = w.upart + slot * 2 * kUpdBlocks;
+                const double* prev = w.upart + (slot ^ 1) * 2 * kUpdBlocks;
+                const int* over = it == 0 ? &w.sc->done : &w.sc->stops[slot ^ 1];
+                if ((rc = ms3d_qdots32(op->ms, nl, p[slot], q, r, invd, part0, w.part_stride, over, &nb, s))) return rc;
+                hipLaunchKernelGGL(k_update_dir, dim3(ub), dim3(kUpdBlock), 0, s, w.sc, slot, it == 0, prev, ub, part0,
+                                   w.part_stride, nb, p[slot], p[slot ^ 1], r, q, invd, op->n, mine, w.xc32);
+            }
+            const double* last = w.upart + ((chunk - 1) & 1) * 2 * kUpdBlocks;
+            // β' of the last iteration came with its direction
+            hipLaunchKernelGGL(k_settle, dim3(1), dim3(kRedThreads), 0, s, w.sc, (chunk - 1) & 1, last,
+                               last + kUpdBlocks, ub, true);
             SIL_LAUNCH_CHECK();
             return SIL_OK;
         }
     }
-    PUpdate<T> pu{zsrc, pold, pnew, &w.sc->beta, invd, &w.sc->done};
-    int nb = 0;
-    int rc;
+    const T* zsrc = r;
     if constexpr (sizeof(T) == 8)
-        rc = apply64(op, nullptr, q, DotEpilogue{part0}, &pu, &nb, s);
-    else
-        rc = apply32(op, nullptr, q, DotEpilogue{part0}, &pu, &nb, s);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_alpha, dim3(1), dim3(kRedThreads), 0, s, w.sc, part0, nb);
-    if constexpr (sizeof(T) == 4)
-        hipLaunchKernelGGL((k_update<T, true>), dim3(kUpdBlocks), dim3(kUpdBlock), 0, s, w.sc, w.x, pnew, r, q, invd,
-                           op->n, part1, part2, w.xc32);
-    else
-        hipLaunchKernelGGL((k_update<T, false>), dim3(kUpdBlocks), dim3(kUpdBlock), 0, s, w.sc, w.x, pnew, r, q, invd,
-                           op->n, part1, part2, nullptr);
-    int nb_rz = kUpdBlocks;
-    if constexpr (sizeof(T) == 8)
-        if (pc == PC_ISAI && (rc = isai_apply(w, r, part1, &nb_rz, &w.sc->done, s))) return rc;
-    hipLaunchKernelGGL(k_beta, dim3(1), dim3(kRedThreads), 0, s, w.sc, part1, nb_rz, part2, kUpdBlocks);
+        if (pc == PC_ISAI) zsrc = w.isai_z;
+    // operators whose first kernel (the direction pass, or the Poisson
+    // product) finishes the iteration before; FP32 marches form the direction
+    // in every workgroup's halo and leave it to k_beta
+    const bool joined = pc != PC_ISAI && (op->kind == OP_POISSON2D ||
+                                          (sizeof(T) == 8 && (op->kind == OP_MAGNETOSTATICS3D ||
+                                                              op->kind == OP_MS3D_JACOBIAN)));
+    const bool aligned = (reinterpret_cast<uintptr_t>(w.x) & 15) == 0;
+    for (int it = 0; it < chunk; ++it) {
+        const int slot = it & 1;
+        T* pnew = p[slot ^ 1];
+        PUpdate<T> pu{zsrc, p[slot], pnew, &w.sc->beta, invd, joined ? &w.sc->stops[slot] : &w.sc->done, {}};
+        if (joined) pu.step = CgStep{w.sc, it == 0 ? nullptr : part1, it == 0 ? nullptr : part2, ub, slot};
+        if constexpr (sizeof(T) == 8)
+            rc = apply64(op, nullptr, q, DotEpilogue{part0}, &pu, &nb, s);
+        else
+            rc = apply32(op, nullptr, q, DotEpilogue{part0}, &pu, &nb, s);
+        if (rc) return rc;
+        AlphaSource as{pu.done, joined ? &w.sc->rzs[slot] : &w.sc->rz, part0, nb};
+        if (nb > kMaxSharedPartials) {
+            // ⟨r, z⟩ of the iteration is in sc->rz either way
+            hipLaunchKernelGGL(k_alpha, dim3(1), dim3(kRedThreads), 0, s, w.sc, part0, nb);
+            as.part = nullptr;
+        }
+        auto update = [&](auto V) {
+            constexpr bool v = decltype(V)::value;
+            hipLaunchKernelGGL((k_update<T, sizeof(T) == 4, v>), dim3(ub), dim3(kUpdBlock), 0, s, w.sc, as, w.x, pnew, r,
+                               q, invd, op->n, part1, part2, w.xc32);
+        };
+        if (aligned)
+            update(std::true_type{});
+        else
+            update(std::false_type{});
+        if (!joined) {
+            int nb_rz = ub;
+            if constexpr (sizeof(T) == 8)
+                if (pc == PC_ISAI && (rc = isai_apply(w, r, part1, &nb_rz, &w.sc->done, s))) return rc;
+            hipLaunchKernelGGL(k_beta, dim3(1), dim3(kRedThreads), 0, s, w.sc, part1, nb_rz, part2, ub);
+        }
+    }
+    if (joined)
+        hipLaunchKernelGGL(k_settle, dim3(1), dim3(kRedThreads), 0, s, w.sc, (chunk - 1) & 1, part1, part2, ub, false);
     SIL_LAUNCH_CHECK();
     return SIL_OK;
 }
@@ -629,9 +771,7 @@ int get_graph(sil_operator op, int prec, int pc, int chunk, T* r, T* q, T* const
     SIL_CHECK_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
     hipGraph_t graph;
     SIL_CHECK_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    int rc = SIL_OK;
-    for (int it = 0; it < chunk && rc == SIL_OK; ++it)
-        rc = enqueue_iteration<T>(op, w, r, q, p[it & 1], p[(it + 1) & 1], pc, cs);
+    const int rc = enqueue_chunk<T>(op, w, r, q, p, pc, chunk, cs);
     hipError_t e = hipStreamEndCapture(cs, &graph);
     if (rc != SIL_OK) {
         (void)hipStreamDestroy(cs);
@@ -691,7 +831,7 @@ void invalidate_isai(sil_operator op)
 void destroy_workspace(Workspace* w)
 {
     if (!w) return;
-    for (double* p : {w->x, w->b, w->r, w->q, w->p[0], w->p[1], w->inv_diag, w->tmp, w->partials, w->isai_t,
+    for (double* p : {w->x, w->b, w->r, w->q, w->p[0], w->p[1], w->inv_diag, w->tmp, w->partials, w->upart, w->isai_t,
                       w->isai_z, w->fb_r, w->fb_d})
         if (p) (void)hipFree(p);
     csr_free(w->isai_g);
@@ -1041,8 +1181,7 @@ int cg_solve_noalloc(sil_operator op, const double* rhs, double* solution, const
     if ((rc = read_scalars(w, s))) return rc;
     dg.initial_residual_l2 = std::sqrt(host.bb);
     while (!host.done) {
-        for (int it = 0; it < chunk; ++it)
-            if ((rc = enqueue_iteration<double>(op, w, w.r, w.q, w.p[it & 1], w.p[(it + 1) & 1], pc, s))) return rc;
+        if ((rc = enqueue_chunk<double>(op, w, w.r, w.q, w.p, pc, chunk, s))) return rc;
         if ((rc = read_scalars(w, s))) return rc;
     }
     if ((rc = true_residual(op, w, s))) return rc;

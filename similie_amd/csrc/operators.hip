@@ -55,13 +55,46 @@ struct MsArgs {
 enum MsResponse { RESP_LINEAR = 0, RESP_SCALED = 1, RESP_JACOBIAN = 2 };
 
 // p_new = z + β p_old with z = D⁻¹ r (Jacobi) or r: the CG direction, in
-// the arithmetic of p_value
+// the arithmetic of p_value.  The arrays are the solver's own (16-byte
+// aligned): 16-byte accesses, the last rows one by one.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_direction(PUpdate<T> pu, int64_t n)
 {
-    if (*pu.done) return;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        pu.p_new[i] = p_value<T>(&pu, nullptr, i);
+    double beta;
+    if (pu.step.sc) {
+        if (!cg_begin<kBlock>(pu.step, beta)) return;
+    } else {
+        if (*pu.done) return;
+        beta = *pu.beta;
+    }
+    constexpr int V = 16 / sizeof(T);
+    typedef T Vec __attribute__((ext_vector_type(V)));
+    const int64_t nv = n / V, stride = (int64_t)gridDim.x * kBlock, t = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+    const Vec* r = reinterpret_cast<const Vec*>(pu.r);
+    const Vec* d = reinterpret_cast<const Vec*>(pu.inv_diag);
+    const Vec* po = reinterpret_cast<const Vec*>(pu.p_old);
+    Vec* pn = reinterpret_cast<Vec*>(pu.p_new);
+    for (int64_t i = t; i < nv; i += stride) {
+        const Vec rv = r[i], pv = po[i];
+        Vec o;
+        if (d) {
+            const Vec dv = d[i];
+#pragma unroll
+            for (int q = 0; q < V; ++q) o[q] = (T)((double)rv[q] * (double)dv[q] + beta * (double)pv[q]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < V; ++q) o[q] = (T)((double)rv[q] + beta * (double)pv[q]);
+        }
+        pn[i] = o;
+    }
+    for (int64_t i = nv * V + t; i < n; i += stride) pu.p_new[i] = p_value_of<T>(pu, beta, i);
+}
+
+// workgroups of k_direction: four rows a thread or more, and few enough that
+// each summing the partials of the iteration before costs little
+inline unsigned direction_grid(int64_t n)
+{
+    return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 4 * kBlock - 1) / (4 * kBlock), 2048));
 }
 
 template <typename T, bool PU>
@@ -763,20 +796,40 @@ __global__ __launch_bounds__(kBlock) void k_p2d_apply(int64_t nx, int64_t ny, co
                                                       const T* __restrict__ wy, const T* __restrict__ x,
                                                       T* __restrict__ out, double* __restrict__ partials, PUpdate<T> pu)
 {
-    if (PU && *pu.done) return;
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    double beta = 0.0;
+    if constexpr (PU) {
+        if (pu.step.sc) {
+            if (!cg_begin<kBlock>(pu.step, beta)) return;
+        } else {
+            if (*pu.done) return;
+            beta = *pu.beta;
+        }
+    }
+    const int64_t t = blockIdx.x * (int64_t)kBlock + threadIdx.x;
     double dot = 0.0;
     if (t < nx * ny) {
-        const int64_t j = t % ny, i = t / ny;
-        const PUpdate<T>* pp = PU ? &pu : nullptr;
+        int64_t i, j;
+        if (nx * ny <= UINT32_MAX) { // uniform: a 32-bit division
+            i = (uint32_t)t / (uint32_t)ny;
+            j = (uint32_t)t % (uint32_t)ny;
+        } else {
+            i = t / ny;
+            j = t % ny;
+        }
+        auto value = [&](int64_t q) -> T {
+            if constexpr (PU)
+                return p_value_of<T>(pu, beta, q);
+            else
+                return x[q];
+        };
         const bool inner = i > 0 && j > 0 && i + 1 < nx && j + 1 < ny;
-        T pv = inner ? p_value<T>(pp, x, t) : T(0);
+        T pv = inner ? value(t) : T(0);
         T o = T(0);
         if (inner) {
-            const T ue = (i + 2 < nx) ? p_value<T>(pp, x, t + ny) : T(0);
-            const T uw = (i > 1) ? p_value<T>(pp, x, t - ny) : T(0);
-            const T un = (j + 2 < ny) ? p_value<T>(pp, x, t + 1) : T(0);
-            const T us = (j > 1) ? p_value<T>(pp, x, t - 1) : T(0);
+            const T ue = (i + 2 < nx) ? value(t + ny) : T(0);
+            const T uw = (i > 1) ? value(t - ny) : T(0);
+            const T un = (j + 2 < ny) ? value(t + 1) : T(0);
+            const T us = (j > 1) ? value(t - 1) : T(0);
             o = wx[t] * (pv - ue) + wx[t - ny] * (pv - uw) + wy[t] * (pv - un) + wy[t - 1] * (pv - us);
         }
         out[t] = o;
@@ -866,18 +919,31 @@ MsArgs<float> ms_args<float>(const Ms3dData& d)
     return a;
 }
 
-// pipelined-march shape: rows per tile (16 or 8; 0 selects the earlier
-// march) and planes per chunk, from SIL_MS3D_PIPE="ty,chunk"
+// Shape of the pipelined march: rows per tile (16 or 8; 0 selects the
+// earlier march) and planes per chunk; SIL_MS3D_PIPE="ty,chunk" fixes it.
+//
+// A workgroup walks chunk + 2 planes one after the other, each a round trip to
+// memory, so on a grid that gives fewer workgroups than the chip holds the
+// walk's length is the time: 16 × 24 tiles on 57 × 49 × 65 nodes are 12
+// workgroups of 26 steps, 28 µs for 4 MB.  The rule takes the shape with the
+// least (workgroups per compute unit, rounded up) · (chunk + 2) · weight; the
+// weight of 16 rows, 2.2, is the measured time of their step against that of
+// 8 rows.  FP64 product, 16 × 24 → the rule's shape: 25³ 27 → 8 µs, 97³ 33 →
+// 14 (8 × 8), 129 × 113 × 97 34 → 21 (8 × 8), 193³ 79 → 79 (16 × 24).  FP32
+// follows the same line (20 → 10, 21 → 12, 50 → 50).
 struct MsPipeShape {
     int ty, chunk;
 };
 
-MsPipeShape ms_pipe_shape()
+constexpr int64_t kComputeUnits = 256;
+constexpr int kMsPipeChunkDefault = 24;
+
+MsPipeShape ms_pipe_shape(const Ms3dData& d)
 {
-    static const MsPipeShape shape = [] {
-        MsPipeShape p{16, 24};
+    static const MsPipeShape fixed = [] {
+        MsPipeShape p{-1, 0};
         if (const char* e = std::getenv("SIL_MS3D_PIPE")) {
-            int ty = 16, ch = 24;
+            int ty = 16, ch = kMsPipeChunkDefault;
             if (std::sscanf(e, "%d,%d", &ty, &ch) >= 1) {
                 p.ty = (ty == 0 || ty == 8) ? ty : 16;
                 p.chunk = std::min(std::max(ch, 1), kMsPipeChunkMax);
@@ -885,7 +951,21 @@ MsPipeShape ms_pipe_shape()
         }
         return p;
     }();
-    return shape;
+    if (fixed.ty >= 0) return fixed;
+    MsPipeShape best{16, kMsPipeChunkDefault};
+    double least = 0.0;
+    for (const int ty : {16, 8}) {
+        const int64_t tiles = ((d.nx + 61) / 62) * ((d.ny + ty - 3) / (ty - 2));
+        for (int c = kMsPipeChunkDefault; c >= 2; --c) {
+            const int64_t nb = tiles * ((d.nz + c - 1) / c);
+            const double cost = (double)((nb + kComputeUnits - 1) / kComputeUnits) * (c + 2) * (ty == 16 ? 2.2 : 1.0);
+            if (least == 0.0 || cost < least) {
+                least = cost;
+                best = {ty, c};
+            }
+        }
+    }
+    return best;
 }
 
 template <typename T, int RESP = RESP_LINEAR>
@@ -956,7 +1036,7 @@ int ms_apply_curl(const Ms3dData& d, const T* in, T* out, DotEpilogue dot, const
             const char* e = std::getenv("SIL_MS3D_NT");
             return !(e && e[0] == '0');
         }();
-        const MsPipeShape ps = ms_pipe_shape();
+        const MsPipeShape ps = ms_pipe_shape(d);
         const int64_t chunk_bytes = (int64_t)(ps.chunk + 2) * d.nx * d.ny * 4 * (int64_t)sizeof(T);
         if (ps.ty > 0 && chunk_bytes <= kMaxBufferBytes) {
             const int pty = ps.ty - 2;
@@ -971,9 +1051,7 @@ int ms_apply_curl(const Ms3dData& d, const T* in, T* out, DotEpilogue dot, const
             // march's FP64 registers)
             const bool fused = pu && sizeof(T) == 4;
             if (pu && !fused) {
-                const int64_t ndof = 3 * nn;
-                const unsigned gd = (unsigned)std::min<int64_t>((ndof + kBlock - 1) / kBlock, 8192);
-                hipLaunchKernelGGL((k_direction<T>), dim3(gd), dim3(kBlock), 0, s, *pu, ndof);
+                hipLaunchKernelGGL((k_direction<T>), dim3(direction_grid(3 * nn)), dim3(kBlock), 0, s, *pu, 3 * nn);
             }
             PUpdate<T> pp{};
             if (pu) pp = *pu;
@@ -1001,9 +1079,7 @@ int ms_apply_curl(const Ms3dData& d, const T* in, T* out, DotEpilogue dot, const
             // the CG direction in its own streaming pass (forming it while the
             // earlier march stages its tile reads three strided arrays per
             // node and is slower than the pass)
-            const int64_t ndof = 3 * nn;
-            const unsigned g = (unsigned)std::min<int64_t>((ndof + kBlock - 1) / kBlock, 8192);
-            hipLaunchKernelGGL((k_direction<T>), dim3(g), dim3(kBlock), 0, s, *pu, ndof);
+            hipLaunchKernelGGL((k_direction<T>), dim3(direction_grid(3 * nn)), dim3(kBlock), 0, s, *pu, 3 * nn);
             src = pu->p_new;
             skip.done = pu->done;
         }
@@ -1017,9 +1093,7 @@ int ms_apply_curl(const Ms3dData& d, const T* in, T* out, DotEpilogue dot, const
         // the direction is formed in its own pass: formed inside the
         // direct kernel, every one of the ~40 neighbour reads of a node would
         // read r, D⁻¹ and p_old instead of p
-        const int64_t ndof = 3 * nn;
-        const unsigned g = (unsigned)std::min<int64_t>((ndof + kBlock - 1) / kBlock, 8192);
-        hipLaunchKernelGGL((k_direction<T>), dim3(g), dim3(kBlock), 0, s, *pu, ndof);
+        hipLaunchKernelGGL((k_direction<T>), dim3(direction_grid(3 * nn)), dim3(kBlock), 0, s, *pu, 3 * nn);
         PUpdate<T> skip{};
         skip.done = pu->done;
         hipLaunchKernelGGL((k_ms3d_apply<T, false>), dim3(nb), dim3(kBlock), 0, s, a, pu->p_new, out, dot.partials,
@@ -1076,16 +1150,14 @@ int ms3d_jacobian_apply32(const Ms3dData& d, const NlData& nl, const float* in, 
 
 int direction_pass32(const PUpdate<float>& pu, int64_t n, hipStream_t s)
 {
-    const unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + kBlock - 1) / kBlock, 8192));
-    hipLaunchKernelGGL((k_direction<float>), dim3(g), dim3(kBlock), 0, s, pu, n);
+    hipLaunchKernelGGL((k_direction<float>), dim3(direction_grid(n)), dim3(kBlock), 0, s, pu, n);
     SIL_LAUNCH_CHECK();
     return SIL_OK;
 }
 
 int direction_pass64(const PUpdate<double>& pu, int64_t n, hipStream_t s)
 {
-    const unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + kBlock - 1) / kBlock, 8192));
-    hipLaunchKernelGGL((k_direction<double>), dim3(g), dim3(kBlock), 0, s, pu, n);
+    hipLaunchKernelGGL((k_direction<double>), dim3(direction_grid(n)), dim3(kBlock), 0, s, pu, n);
     SIL_LAUNCH_CHECK();
     return SIL_OK;
 }
@@ -1107,7 +1179,7 @@ template <int RESP>
 int ms_qdots32(const Ms3dData& d, const NlData* nl, const float* p, float* q, const float* r, const float* inv_diag,
                double* partials, int64_t pstride, const int* done, int* nb_out, hipStream_t s)
 {
-    const MsPipeShape ps = ms_pipe_shape();
+    const MsPipeShape ps = ms_pipe_shape(d);
     const int pty = ps.ty - 2;
     const int ptx = (int)((d.nx + 61) / 62), pny = (int)((d.ny + pty - 1) / pty);
     const int pkc = (int)((d.nz + ps.chunk - 1) / ps.chunk);
@@ -1140,7 +1212,7 @@ int ms_qdots32(const Ms3dData& d, const NlData* nl, const float* p, float* q, co
 
 bool ms3d_single_pass_ok(const Ms3dData& d)
 {
-    const MsPipeShape ps = ms_pipe_shape();
+    const MsPipeShape ps = ms_pipe_shape(d);
     const int64_t chunk_bytes = (int64_t)(ps.chunk + 2) * d.nx * d.ny * 4 * (int64_t)sizeof(float);
     return !d.divg && ps.ty > 0 && d.nx >= 3 && d.ny >= 3 && d.nz >= 3 && chunk_bytes <= kMaxBufferBytes;
 }

@@ -102,6 +102,32 @@ struct DotEpilogue {
     double* partials; // null: no dot
 };
 
+// The CG scalars on the device.  Between chunks of iterations rz, beta, iter,
+// done and converged describe the last finished iteration.  Inside a chunk
+// iteration i keeps its ⟨r, z⟩, its number and whether it stops the solve in
+// slot i & 1 of the pairs below, so that a kernel which reduces the previous
+// iteration's partial sums in every workgroup never reads a value that
+// another workgroup of the same kernel is writing.
+struct CgScalars {
+    double rz, rz_prev, pq, alpha, beta, rr, bb, tol2bb;
+    double rr_true;
+    int done, iter, max_iter, converged;
+    double rzs[2];
+    int iters[2], stops[2];
+};
+
+// What the first kernel of a CG iteration needs to finish the previous one:
+// the partial sums of ⟨r, z⟩ and ⟨r, r⟩ (null in the first iteration of a
+// chunk, whose scalars are already settled) and the iteration's slot.  sc
+// null: β is read from PUpdate::beta, a kernel of its own has settled it.
+struct CgStep {
+    CgScalars* sc = nullptr;
+    const double* part_rz = nullptr;
+    const double* part_rr = nullptr;
+    int count = 0;
+    int slot = 0;
+};
+
 // CG "p = z + β p_old" prologue fused into an application: when enabled the
 // kernel forms p from (r, p_old, β, diag) for every node it reads, writes p
 // for its own rows, and applies the operator to the new p.
@@ -113,6 +139,7 @@ struct PUpdate {
     const double* beta;  // device scalar
     const T* inv_diag;   // Jacobi, in the recurrence's arithmetic, or null
     const int* done;     // device flag: skip when set
+    CgStep step;         // with sc set: the first kernel finishes the previous iteration
 };
 
 int ms3d_apply64(const Ms3dData& d, const double* in, double* out, DotEpilogue dot, const PUpdate<double>* pu,

@@ -144,3 +144,79 @@ def test_cg_zero_rhs_and_iteration_cap(S):
     st = S.StrongFormulationSolverSettings(max_iterations=5, relative_tolerance=1e-14, preconditioner="identity")
     x, dg = S.minimize_strong_formulation_residual(op, cuda(b).reshape(-1), settings=st)
     assert dg["iterations"] == 5 and dg["converged"] == 0
+
+
+def _numpy_cg(apply, diag, b, iterations):
+    """Jacobi CG, a fixed number of iterations"""
+    x, r = np.zeros_like(b), b.copy()
+    z = r / diag
+    p, rz = z.copy(), float(np.dot(r, z))
+    for _ in range(iterations):
+        q = apply(p)
+        if rz == 0.0:  # solved exactly: the iterates stay
+            break
+        alpha = rz / float(np.dot(p, q))
+        x += alpha * p
+        r -= alpha * q
+        z = r / diag
+        new = float(np.dot(r, z))
+        p, rz = z + (new / rz) * p, new
+    return x
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("shape", [(3, 3), (5, 4), (33, 17), (61, 64, 1), (4, 3, 5), (9, 16, 7), (65, 9, 30)])
+def test_cg_stops_at_the_iteration_limit(shape, precision):
+    """The iterates after 1, 2, 3, 31, 32, 33 and 35 iterations (the first and
+    last of a chunk, the first of the next) against plain CG: every kernel of
+    an iteration finishes the one before, so a limit inside a chunk, at its
+    end and just after it takes different paths.  Rows that are no multiple
+    of the vector width, fewer rows than one workgroup's, one direction
+    kernel (3D) and none (2D).  Stretched axes of a small 3D grid keep 35
+    iterations below convergence."""
+    from similie_amd import solvers as S
+
+    rng = np.random.default_rng(sum(shape))
+    if len(shape) == 2:
+        hx = [np.cumsum(np.concatenate([[0.0], rng.uniform(0.5, 1.5, n - 1)])) for n in shape]
+        kappa = np.exp(rng.standard_normal(shape))
+        op = S.Poisson2D(*hx, kappa=torch.from_numpy(kappa.reshape(-1)).cuda())
+    else:
+        shape = tuple(max(s, 3) for s in shape)
+        axes = [np.cumsum(np.concatenate([[0.0], rng.uniform(0.5, 1.5, n - 1)])) for n in shape]
+        mu = np.exp(rng.standard_normal(int(np.prod(shape))))
+        op = S.MagnetostaticsOperator3D(*axes, torch.from_numpy(mu).cuda(), gauge_penalty=0.5)
+    n = op.size()
+    dense = torch.stack([op.apply(e) for e in torch.eye(n, dtype=torch.float64, device="cuda")]).cpu().numpy().T \
+        if n <= 600 else None
+    diag = op.diagonal().cpu().numpy()
+
+    def apply(v):
+        return dense @ v if dense is not None else op.apply(torch.from_numpy(v).cuda()).cpu().numpy()
+
+    b = rng.standard_normal(n)
+    if len(shape) == 2:
+        b = b.reshape(shape)
+        b[0, :] = b[-1, :] = 0.0
+        b[:, 0] = b[:, -1] = 0.0
+        b = b.reshape(-1)
+    bt = torch.from_numpy(b).cuda()
+    # k steps of a recurrence rounded to u amplify by at most the operator's
+    # condition (below 1e3 here): 35 · 1e3 · u, 4e-12 in FP64 and 2e-3 in FP32;
+    # a reduction in another order counts as one more rounding
+    for limit in (1, 2, 3, 31, 32, 33, 35):
+        x, dg = S.minimize_strong_formulation_residual(
+            op, bt, settings=S.StrongFormulationSolverSettings(max_iterations=limit, relative_tolerance=1e-9,
+                                                               precision=precision, check_interval=32))
+        assert dg["iterations"] <= limit
+        if not dg["converged"]:
+            assert dg["iterations"] == limit
+        r = b - apply(x.cpu().numpy())
+        rel_true = np.linalg.norm(r) / max(np.linalg.norm(b), 1e-300)
+        assert abs(rel_true - dg["true_relative_residual"]) <= 1e-9 + 1e-6 * rel_true
+        if dg["converged"]:
+            assert rel_true <= 1e-9 * (1 + 1e-3)
+        else:
+            ref = _numpy_cg(apply, diag, b, limit)
+            tol = 1e-10 if precision == "fp64" else 2e-3
+            assert np.linalg.norm(x.cpu().numpy() - ref) <= tol * np.linalg.norm(ref), limit
