@@ -3,8 +3,6 @@
 // the per-block partial sums of ⟨in, out⟩.
 #pragma once
 
-#include <hipcub/hipcub.hpp>
-
 #include "operators.hpp"
 
 namespace sil {
@@ -28,36 +26,65 @@ __device__ __forceinline__ T p_value_of(const PUpdate<T>& pu, double beta, int64
     return (T)(z + beta * (double)pu.p_old[idx]);
 }
 
+// v of the lane N places round its row of 16
+template <int N>
+__device__ __forceinline__ double row_rotate(double v)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x120 + N, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x120 + N, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, (uint64_t)(uint32_t)lo | ((uint64_t)(uint32_t)hi << 32));
+}
+
+__device__ __forceinline__ double read_lane(double v, int lane)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, lane);
+    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(u >> 32), lane);
+    return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
+}
+
+// the wavefront's sum in every lane, all lanes active: rotations within the
+// rows of 16 (DPP, no LDS round trips as a shuffle makes), then the four rows
+__device__ __forceinline__ double wave_sum(double v)
+{
+    v += row_rotate<8>(v);
+    v += row_rotate<4>(v);
+    v += row_rotate<2>(v);
+    v += row_rotate<1>(v);
+    return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
+}
+
 // Sums of K partial-sum arrays in every thread of a workgroup of THREADS, in a
-// fixed order (the same bits in every workgroup).  Up to 4 · THREADS values
-// are in flight per array.
+// fixed order (the same bits in every workgroup).  Each array goes to one
+// wavefront (K ≥ 3), or to half or all of them, sixteen loads a lane in flight.
 template <int THREADS, int K>
 __device__ __forceinline__ void reduce_all(const double* const (&p)[K], const int (&count)[K], double (&out)[K])
 {
-    __shared__ double sh[K][THREADS / 64];
+    constexpr int W = THREADS / 64, parts = K == 1 ? W : (K == 2 ? W / 2 : 1), U = 16;
+    __shared__ double sh[K][parts];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part = wave % parts;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
+        if (wave / parts != k % (W / parts)) continue;
         double v = 0.0;
-        for (int i = threadIdx.x; i < count[k]; i += 4 * THREADS) {
-            double q[4];
+        for (int i = part * 64 + lane; i < count[k]; i += U * 64 * parts) {
+            double q[U];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) q[u] = i + u * THREADS < count[k] ? p[k][i + u * THREADS] : 0.0;
-            v += (q[0] + q[1]) + (q[2] + q[3]);
+            for (int u = 0; u < U; ++u) q[u] = i + u * 64 * parts < count[k] ? p[k][i + u * 64 * parts] : 0.0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) v += q[u];
         }
-        out[k] = v;
+        v = wave_sum(v);
+        if (lane == 0) sh[k][part] = v;
     }
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-        for (int off = 32; off > 0; off >>= 1) out[k] += __shfl_xor(out[k], off, 64);
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int k = 0; k < K; ++k) sh[k][threadIdx.x >> 6] = out[k];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         out[k] = sh[k][0];
 #pragma unroll
-        for (int w = 1; w < THREADS / 64; ++w) out[k] += sh[k][w];
+        for (int w = 1; w < parts; ++w) out[k] += sh[k][w];
     }
 }
 
@@ -80,15 +107,17 @@ __device__ __forceinline__ bool cg_begin(const CgStep& st, double& beta)
         }
         return !sc.done;
     }
-    if (sc.stops[s ^ 1]) {
+    // (read before the sums, tested after: one round trip)
+    const int over = sc.stops[s ^ 1], it = sc.iters[s ^ 1] + 1;
+    const double prev = sc.rzs[s ^ 1], tol2bb = sc.tol2bb;
+    const int max_iter = sc.max_iter;
+    double v[2];
+    reduce_all<THREADS, 2>({st.part_rz, st.part_rr}, {st.count, st.count}, v);
+    if (over) {
         if (first) sc.stops[s] = 1;
         return false;
     }
-    double v[2];
-    reduce_all<THREADS, 2>({st.part_rz, st.part_rr}, {st.count, st.count}, v);
-    const double prev = sc.rzs[s ^ 1];
-    const int it = sc.iters[s ^ 1] + 1;
-    const bool conv = v[1] <= sc.tol2bb, stop = conv || it >= sc.max_iter;
+    const bool conv = v[1] <= tol2bb, stop = conv || it >= max_iter;
     beta = v[0] / prev;
     if (first) {
         sc.rzs[s] = v[0];
@@ -111,10 +140,16 @@ __device__ __forceinline__ bool cg_begin(const CgStep& st, double& beta)
 template <typename T>
 __device__ __forceinline__ void block_dot_store(double v, double* partials)
 {
-    using BR = hipcub::BlockReduce<double, kApplyBlock>;
-    __shared__ typename BR::TempStorage tmp;
-    double s = BR(tmp).Sum(v);
-    if (threadIdx.x == 0) partials[blockIdx.x] = s;
+    __shared__ double sh[kApplyBlock / 64];
+    const double s = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = sh[0];
+#pragma unroll
+        for (int w = 1; w < kApplyBlock / 64; ++w) t += sh[w];
+        partials[blockIdx.x] = t;
+    }
 }
 
 }  // namespace sil

@@ -74,11 +74,12 @@ constexpr int kRedThreads = 1024;
 // sums itself
 constexpr int kMaxSharedPartials = 2048;
 
-// workgroups of an update over n rows: four rows a thread, at most 1024, so
-// that the next kernel sums few partials
-inline int update_blocks(int64_t n)
+// workgroups of an update over n rows of `width` bytes: one 16-byte vector a
+// thread, at most 1024 (the next kernel sums their partials)
+inline int update_blocks(int64_t n, int width)
 {
-    return (int)std::max<int64_t>(1, std::min<int64_t>((n + 4 * kUpdBlock - 1) / (4 * kUpdBlock), 1024));
+    const int64_t rows = kUpdBlock * (16 / width);
+    return (int)std::max<int64_t>(1, std::min<int64_t>((n + rows - 1) / rows, 1024));
 }
 
 __device__ double block_sum(double v)
@@ -198,23 +199,17 @@ __global__ void k_alpha(CgScalars* sc, const double* part, int count)
 __device__ __forceinline__ void store_two_sums(double a, double b, double* __restrict__ pa, double* __restrict__ pb)
 {
     __shared__ double sh[2][kUpdBlock / 64];
-    for (int off = 32; off > 0; off >>= 1) {
-        a += __shfl_down(a, off, 64);
-        b += __shfl_down(b, off, 64);
-    }
+    a = wave_sum(a);
+    b = wave_sum(b);
     if ((threadIdx.x & 63) == 0) {
         sh[0][threadIdx.x >> 6] = a;
         sh[1][threadIdx.x >> 6] = b;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double s0 = 0.0, s1 = 0.0;
-        for (int i = 0; i < kUpdBlock / 64; ++i) {
-            s0 += sh[0][i];
-            s1 += sh[1][i];
-        }
-        pa[blockIdx.x] = s0;
-        pb[blockIdx.x] = s1;
+    if (threadIdx.x < 2) {
+        double v = sh[threadIdx.x][0];
+        for (int i = 1; i < kUpdBlock / 64; ++i) v += sh[threadIdx.x][i];
+        (threadIdx.x == 0 ? pa : pb)[blockIdx.x] = v;
     }
 }
 
@@ -239,15 +234,40 @@ __global__ __launch_bounds__(kUpdBlock) void k_update(const CgScalars* __restric
                                                       double* __restrict__ part_rz, double* __restrict__ part_rr,
                                                       float* __restrict__ xc)
 {
-    if (*as.stop) return;
+    constexpr int V = 16 / (int)sizeof(T);
+    typedef T Vec __attribute__((ext_vector_type(V)));
+    const int64_t stride = (int64_t)gridDim.x * kUpdBlock, t = blockIdx.x * (int64_t)kUpdBlock + threadIdx.x;
+    const int64_t nv = n / V;
+    // the first rows are requested before the scalars they wait for
+    struct Rows {
+        Vec p, q, r, d, x;
+    } next = {};
+    auto load = [&](int64_t i) {
+        next.p = reinterpret_cast<const Vec*>(p)[i];
+        next.q = reinterpret_cast<const Vec*>(q)[i];
+        next.r = reinterpret_cast<Vec*>(r)[i];
+        if (inv_diag) next.d = reinterpret_cast<const Vec*>(inv_diag)[i];
+        if constexpr (XC) {
+            next.x = reinterpret_cast<Vec*>(xc)[i];
+        } else if constexpr (XVEC) {
+            next.x = reinterpret_cast<Vec*>(x)[i];
+        } else {
+#pragma unroll
+            for (int u = 0; u < V; ++u) next.x[u] = x[i * V + u];
+        }
+    };
+    if (t < nv) load(t);
+    const int stop = *as.stop;
     double alpha;
     if (as.part) {
+        const double rz = *as.rz;
         double pq[1];
         reduce_all<kUpdBlock, 1>({as.part}, {as.count}, pq);
-        alpha = *as.rz / pq[0];
+        alpha = rz / pq[0];
     } else {
         alpha = sc->alpha;
     }
+    if (stop) return;
     const float alpha32 = (float)alpha;
     double vz = 0.0, vr = 0.0;
     auto row = [&](T& ri, T qi, T di) {
@@ -256,35 +276,30 @@ __global__ __launch_bounds__(kUpdBlock) void k_update(const CgScalars* __restric
         vr += rd * rd;
         vz += rd * (inv_diag ? rd * (double)di : rd);
     };
-    constexpr int V = 16 / (int)sizeof(T);
-    typedef T Vec __attribute__((ext_vector_type(V)));
-    const int64_t stride = (int64_t)gridDim.x * kUpdBlock, t = blockIdx.x * (int64_t)kUpdBlock + threadIdx.x;
-    const int64_t nv = n / V;
-    for (int64_t i = t; i < nv; i += stride) {
-        const Vec pv = reinterpret_cast<const Vec*>(p)[i], qv = reinterpret_cast<const Vec*>(q)[i];
-        Vec rv = reinterpret_cast<Vec*>(r)[i], dv = rv;
-        if (inv_diag) dv = reinterpret_cast<const Vec*>(inv_diag)[i];
-        if constexpr (XC) {
-            Vec xv = reinterpret_cast<Vec*>(xc)[i];
-#pragma unroll
-            for (int u = 0; u < V; ++u) xv[u] = fmaf(alpha32, (float)pv[u], xv[u]);
-            reinterpret_cast<Vec*>(xc)[i] = xv;
-        } else if constexpr (XVEC) {
-            Vec xv = reinterpret_cast<Vec*>(x)[i];
-#pragma unroll
-            for (int u = 0; u < V; ++u) xv[u] += alpha * (double)pv[u];
-            reinterpret_cast<Vec*>(x)[i] = xv;
-        } else {
-#pragma unroll
-            for (int u = 0; u < V; ++u) x[i * V + u] += alpha * (double)pv[u];
-        }
+    for (int64_t i = t; i < nv;) {
+        Rows c = next;
+        const int64_t at = i;
+        i += stride;
+        if (i < nv) load(i);
 #pragma unroll
         for (int u = 0; u < V; ++u) {
-            T ri = rv[u];
-            row(ri, qv[u], dv[u]);
-            rv[u] = ri;
+            if constexpr (XC)
+                c.x[u] = fmaf(alpha32, (float)c.p[u], c.x[u]);
+            else
+                c.x[u] += alpha * (double)c.p[u];
+            T ri = c.r[u];
+            row(ri, c.q[u], c.d[u]);
+            c.r[u] = ri;
         }
-        reinterpret_cast<Vec*>(r)[i] = rv;
+        if constexpr (XC) {
+            reinterpret_cast<Vec*>(xc)[at] = c.x;
+        } else if constexpr (XVEC) {
+            reinterpret_cast<Vec*>(x)[at] = c.x;
+        } else {
+#pragma unroll
+            for (int u = 0; u < V; ++u) x[at * V + u] = c.x[u];
+        }
+        reinterpret_cast<Vec*>(r)[at] = c.r;
     }
     for (int64_t i = nv * V + t; i < n; i += stride) {
         if constexpr (XC)
@@ -368,39 +383,53 @@ __global__ __launch_bounds__(kUpdBlock) void k_update_dir(CgScalars* __restrict_
                                                           const float* __restrict__ inv_diag, int64_t n,
                                                           double* __restrict__ parts, float* __restrict__ xc)
 {
+    typedef float F4 __attribute__((ext_vector_type(4)));
+    const int64_t stride = (int64_t)gridDim.x * kUpdBlock, t = blockIdx.x * (int64_t)kUpdBlock + threadIdx.x;
+    const int64_t nv = n / 4;
+    // the first rows are requested before the scalars they wait for
+    struct Rows {
+        F4 p, q, r, x, d;
+    } next = {};
+    auto load = [&](int64_t i) {
+        next.p = reinterpret_cast<const F4*>(p)[i];
+        next.q = reinterpret_cast<const F4*>(q)[i];
+        next.r = reinterpret_cast<F4*>(r)[i];
+        next.x = reinterpret_cast<F4*>(xc)[i];
+        if (inv_diag) next.d = reinterpret_cast<const F4*>(inv_diag)[i];
+    };
+    if (t < nv) load(t);
     const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
     double g, pq, qz, qq;
     if (first) {
-        if (sc->done) {
-            if (writer) sc->stops[slot] = 1;
-            return;
-        }
+        const int over = sc->done, iter = sc->iter;
+        g = sc->rz;
         double v[3];
         reduce_all<kUpdBlock, 3>({march, march + mstride, march + 2 * mstride}, {mcount, mcount, mcount}, v);
-        g = sc->rz;
         pq = v[0], qz = v[1], qq = v[2];
         if (writer) {
-            sc->iters[slot] = sc->iter;
-            sc->stops[slot] = 0;
+            sc->iters[slot] = iter;
+            sc->stops[slot] = over;
             sc->rzs[slot] = g;
         }
+        if (over) return;
     } else {
-        if (sc->stops[slot ^ 1]) {
-            if (writer) sc->stops[slot] = 1;
-            return;
-        }
+        const int over = sc->stops[slot ^ 1], it = sc->iters[slot ^ 1] + 1, max_iter = sc->max_iter;
+        const double g_prev = sc->rzs[slot ^ 1], tol2bb = sc->tol2bb;
         double v[5];
         reduce_all<kUpdBlock, 5>({march, march + mstride, march + 2 * mstride, prev_parts, prev_parts + kUpdBlocks},
                                  {mcount, mcount, mcount, prev_count, prev_count}, v);
+        if (over) {
+            if (writer) sc->stops[slot] = 1;
+            return;
+        }
         pq = v[0], qz = v[1], qq = v[2], g = v[3];
         const double rr = v[4];
-        const int it = sc->iters[slot ^ 1] + 1;
-        const bool conv = rr <= sc->tol2bb, stop = conv || it >= sc->max_iter;
+        const bool conv = rr <= tol2bb, stop = conv || it >= max_iter;
         if (writer) {
             sc->iters[slot] = it;
             sc->stops[slot] = stop ? 1 : 0;
             sc->rzs[slot] = g;
-            sc->rz_prev = sc->rzs[slot ^ 1];
+            sc->rz_prev = g_prev;
             sc->rz = g;
             sc->rr = rr;
             sc->iter = it;
@@ -423,23 +452,22 @@ __global__ __launch_bounds__(kUpdBlock) void k_update_dir(CgScalars* __restrict_
         vz += rd * z;
         return (float)(z + beta * (double)pi);
     };
-    typedef float F4 __attribute__((ext_vector_type(4)));
-    const int64_t stride = (int64_t)gridDim.x * kUpdBlock, t = blockIdx.x * (int64_t)kUpdBlock + threadIdx.x;
-    const int64_t nv = n / 4;
-    for (int64_t i = t; i < nv; i += stride) {
-        const F4 pv = reinterpret_cast<const F4*>(p)[i], qv = reinterpret_cast<const F4*>(q)[i];
-        F4 rv = reinterpret_cast<F4*>(r)[i], xv = reinterpret_cast<F4*>(xc)[i], dv = rv, nvv;
-        if (inv_diag) dv = reinterpret_cast<const F4*>(inv_diag)[i];
+    for (int64_t i = t; i < nv;) {
+        Rows c = next;
+        const int64_t at = i;
+        i += stride;
+        if (i < nv) load(i);
+        F4 np;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            xv[u] = fmaf(alpha32, pv[u], xv[u]);
-            float ri = rv[u];
-            nvv[u] = row(pv[u], ri, qv[u], dv[u]);
-            rv[u] = ri;
+            c.x[u] = fmaf(alpha32, c.p[u], c.x[u]);
+            float ri = c.r[u];
+            np[u] = row(c.p[u], ri, c.q[u], c.d[u]);
+            c.r[u] = ri;
         }
-        reinterpret_cast<F4*>(xc)[i] = xv;
-        reinterpret_cast<F4*>(r)[i] = rv;
-        reinterpret_cast<F4*>(pn)[i] = nvv;
+        reinterpret_cast<F4*>(xc)[at] = c.x;
+        reinterpret_cast<F4*>(r)[at] = c.r;
+        reinterpret_cast<F4*>(pn)[at] = np;
     }
     for (int64_t i = nv * 4 + t; i < n; i += stride) {
         const float pi = p[i];
@@ -682,7 +710,7 @@ int enqueue_chunk(sil_operator op, Workspace& w, T* r, T* q, T* const* p, int pc
         else
             invd = w.inv_diag32;
     }
-    const int ub = update_blocks(op->n);
+    const int ub = update_blocks(op->n, sizeof(T));
     int rc, nb = 0;
     if constexpr (sizeof(T) == 4) {
         if (w.single_pass) {

@@ -14,8 +14,6 @@
 //
 // Both come in FP64 and FP32 and can (a) emit per-block partial sums of
 // ⟨in, out⟩ and (b) form the CG direction p = z + β p_old on the fly.
-#include <hipcub/hipcub.hpp>
-
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -60,13 +58,6 @@ enum MsResponse { RESP_LINEAR = 0, RESP_SCALED = 1, RESP_JACOBIAN = 2 };
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_direction(PUpdate<T> pu, int64_t n)
 {
-    double beta;
-    if (pu.step.sc) {
-        if (!cg_begin<kBlock>(pu.step, beta)) return;
-    } else {
-        if (*pu.done) return;
-        beta = *pu.beta;
-    }
     constexpr int V = 16 / sizeof(T);
     typedef T Vec __attribute__((ext_vector_type(V)));
     const int64_t nv = n / V, stride = (int64_t)gridDim.x * kBlock, t = blockIdx.x * (int64_t)kBlock + threadIdx.x;
@@ -74,18 +65,33 @@ __global__ __launch_bounds__(kBlock) void k_direction(PUpdate<T> pu, int64_t n)
     const Vec* d = reinterpret_cast<const Vec*>(pu.inv_diag);
     const Vec* po = reinterpret_cast<const Vec*>(pu.p_old);
     Vec* pn = reinterpret_cast<Vec*>(pu.p_new);
-    for (int64_t i = t; i < nv; i += stride) {
-        const Vec rv = r[i], pv = po[i];
+    // the first rows are requested before the scalars they wait for
+    Vec rv = {}, pv = {}, dv = {};
+    auto load = [&](int64_t i) {
+        rv = r[i];
+        pv = po[i];
+        if (d) dv = d[i];
+    };
+    if (t < nv) load(t);
+    double beta;
+    if (pu.step.sc) {
+        if (!cg_begin<kBlock>(pu.step, beta)) return;
+    } else {
+        if (*pu.done) return;
+        beta = *pu.beta;
+    }
+    for (int64_t i = t; i < nv;) {
+        const Vec r0 = rv, p0 = pv, d0 = dv;
+        const int64_t at = i;
+        i += stride;
+        if (i < nv) load(i);
         Vec o;
-        if (d) {
-            const Vec dv = d[i];
 #pragma unroll
-            for (int q = 0; q < V; ++q) o[q] = (T)((double)rv[q] * (double)dv[q] + beta * (double)pv[q]);
-        } else {
-#pragma unroll
-            for (int q = 0; q < V; ++q) o[q] = (T)((double)rv[q] + beta * (double)pv[q]);
+        for (int q = 0; q < V; ++q) {
+            const double z = d ? (double)r0[q] * (double)d0[q] : (double)r0[q];
+            o[q] = (T)(z + beta * (double)p0[q]);
         }
-        pn[i] = o;
+        pn[at] = o;
     }
     for (int64_t i = nv * V + t; i < n; i += stride) pu.p_new[i] = p_value_of<T>(pu, beta, i);
 }
@@ -796,47 +802,67 @@ __global__ __launch_bounds__(kBlock) void k_p2d_apply(int64_t nx, int64_t ny, co
                                                       const T* __restrict__ wy, const T* __restrict__ x,
                                                       T* __restrict__ out, double* __restrict__ partials, PUpdate<T> pu)
 {
-    double beta = 0.0;
+    const int64_t t = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+    const bool in = t < nx * ny;
+    int64_t i = 0, j = 0;
+    if (nx * ny <= UINT32_MAX) { // uniform: a 32-bit division
+        i = (uint32_t)t / (uint32_t)ny;
+        j = (uint32_t)t % (uint32_t)ny;
+    } else {
+        i = t / ny;
+        j = t % ny;
+    }
+    // node, east, west, north, south: their values' ingredients are requested
+    // before the scalar β that PU waits for; zero outside the interior
+    const bool inner = in && i > 0 && j > 0 && i + 1 < nx && j + 1 < ny;
+    const bool have[5] = {inner, inner && i + 2 < nx, inner && i > 1, inner && j + 2 < ny, inner && j > 1};
+    const int64_t at[5] = {t, t + ny, t - ny, t + 1, t - 1};
+    T a[5], d[5], po[5], w[4] = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+        a[q] = d[q] = po[q] = T(0);
+        if (have[q]) {
+            if constexpr (PU) {
+                a[q] = pu.r[at[q]];
+                po[q] = pu.p_old[at[q]];
+                if (pu.inv_diag) d[q] = pu.inv_diag[at[q]];
+            } else {
+                a[q] = x[at[q]];
+            }
+        }
+    }
+    if (inner) {
+        w[0] = wx[t];
+        w[1] = wx[t - ny];
+        w[2] = wy[t];
+        w[3] = wy[t - 1];
+    }
+    T v[5];
     if constexpr (PU) {
+        double beta;
         if (pu.step.sc) {
             if (!cg_begin<kBlock>(pu.step, beta)) return;
         } else {
             if (*pu.done) return;
             beta = *pu.beta;
         }
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            // arithmetic of p_value
+            const double z = pu.inv_diag ? (double)a[q] * (double)d[q] : (double)a[q];
+            v[q] = have[q] ? (T)(z + beta * (double)po[q]) : T(0);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) v[q] = a[q];
     }
-    const int64_t t = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-    double dot = 0.0;
-    if (t < nx * ny) {
-        int64_t i, j;
-        if (nx * ny <= UINT32_MAX) { // uniform: a 32-bit division
-            i = (uint32_t)t / (uint32_t)ny;
-            j = (uint32_t)t % (uint32_t)ny;
-        } else {
-            i = t / ny;
-            j = t % ny;
-        }
-        auto value = [&](int64_t q) -> T {
-            if constexpr (PU)
-                return p_value_of<T>(pu, beta, q);
-            else
-                return x[q];
-        };
-        const bool inner = i > 0 && j > 0 && i + 1 < nx && j + 1 < ny;
-        T pv = inner ? value(t) : T(0);
-        T o = T(0);
-        if (inner) {
-            const T ue = (i + 2 < nx) ? value(t + ny) : T(0);
-            const T uw = (i > 1) ? value(t - ny) : T(0);
-            const T un = (j + 2 < ny) ? value(t + 1) : T(0);
-            const T us = (j > 1) ? value(t - 1) : T(0);
-            o = wx[t] * (pv - ue) + wx[t - ny] * (pv - uw) + wy[t] * (pv - un) + wy[t - 1] * (pv - us);
-        }
+    T o = T(0);
+    if (inner) o = w[0] * (v[0] - v[1]) + w[1] * (v[0] - v[2]) + w[2] * (v[0] - v[3]) + w[3] * (v[0] - v[4]);
+    if (in) {
         out[t] = o;
-        if (PU) pu.p_new[t] = pv;
-        dot = (double)pv * (double)o;
+        if (PU) pu.p_new[t] = v[0];
     }
-    if (partials) block_dot_store<T>(dot, partials);
+    if (partials) block_dot_store<T>((double)v[0] * (double)o, partials);
 }
 
 __global__ void k_p2d_weights(int64_t nx, int64_t ny, const double* __restrict__ hx, const double* __restrict__ hy,
