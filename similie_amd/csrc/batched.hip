@@ -18,6 +18,7 @@
 #include <numeric>
 #include <vector>
 
+#include "apply_epilogue.hpp"
 #include "batched.hpp"
 
 namespace sil {
@@ -294,246 +295,357 @@ __global__ __launch_bounds__(BLOCK) void k_batched_cg(BatchArgs a)
 }
 
 // ------------------------------------------------------------- wide path ---
+//
+// A step of every wide problem is two kernels; `s` is the step's parity.
+//   A  sums the previous step's partials (every workgroup of the problem
+//      itself, so no kernel of one wavefront per problem stands between),
+//      decides what this step is, and then either
+//        CG       p = z + β p_old and q = A p, partials of ⟨p, q⟩, or
+//        REPLACE  r = b − A x in FP64, partials of ⟨r, r⟩ and ⟨r, z⟩;
+//   B  (CG steps) α from the partials of ⟨p, q⟩, x += α p, r −= α q, partials of
+//      ⟨r, z⟩ and ⟨r, r⟩.
+// A replacement is a step of its own of the problem that needs it, where it
+// used to be two further kernels of every iteration that nearly always
+// returned at once.  128 problems of sides 32–512: seven kernels, 73 µs an
+// iteration for the 45 problems of sides over 192, and the persistent kernel
+// after them, 291 ms in all; two kernels, 54 µs for the 76 over 96, and the
+// persistent kernel beside them, 146 ms.  The scalars of a
+// step go to state[s], so nothing a workgroup reads is written in the same
+// kernel.  Workgroups are mapped to the problems still running (L.map, rebuilt
+// by the host as problems finish).
 
 constexpr int kWideNT = 256;
+constexpr int kWU = 4; // nodes per thread per pass
+static_assert(kWideNT * kWU == kWideNodes, "a workgroup's nodes per pass");
 
-enum WidePhase { W_INIT = 0, W_ALPHA, W_BETA, W_REPLACED, W_FINAL };
+enum WideMode { W_START = 0, W_CG, W_REPLACE };
 
-// block sums of two values into part[0], part[1]
+// sums of `count` (≤ kWideNT) pairs in every thread, fixed order
+__device__ __forceinline__ void wide_sums(const double* __restrict__ part, int count, double& a, double& b)
+{
+    __shared__ double sh[2][kWideNT / 64];
+    double v0 = 0.0, v1 = 0.0;
+    if ((int)threadIdx.x < count) {
+        v0 = part[2 * threadIdx.x];
+        v1 = part[2 * threadIdx.x + 1];
+    }
+    v0 = wave_sum(v0);
+    v1 = wave_sum(v1);
+    if ((threadIdx.x & 63) == 0) {
+        sh[0][threadIdx.x >> 6] = v0;
+        sh[1][threadIdx.x >> 6] = v1;
+    }
+    __syncthreads();
+    a = sh[0][0];
+    b = sh[1][0];
+#pragma unroll
+    for (int w = 1; w < kWideNT / 64; ++w) {
+        a += sh[0][w];
+        b += sh[1][w];
+    }
+}
+
+// workgroup sums of two values into part[0], part[1]
 __device__ __forceinline__ void wide_partials(double v0, double v1, double* __restrict__ part)
 {
     __shared__ double sh[2][kWideNT / 64];
-    for (int off = 32; off > 0; off >>= 1) {
-        v0 += __shfl_down(v0, off, 64);
-        v1 += __shfl_down(v1, off, 64);
-    }
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) {
-        sh[0][w] = v0;
-        sh[1][w] = v1;
+    v0 = wave_sum(v0);
+    v1 = wave_sum(v1);
+    if ((threadIdx.x & 63) == 0) {
+        sh[0][threadIdx.x >> 6] = v0;
+        sh[1][threadIdx.x >> 6] = v1;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double s0 = 0.0, s1 = 0.0;
+    if (threadIdx.x < 2) {
+        double t = sh[threadIdx.x][0];
 #pragma unroll
-        for (int i = 0; i < kWideNT / 64; ++i) {
-            s0 += sh[0][i];
-            s1 += sh[1][i];
-        }
-        part[0] = s0;
-        part[1] = s1;
+        for (int w = 1; w < kWideNT / 64; ++w) t += sh[threadIdx.x][w];
+        part[threadIdx.x] = t;
     }
 }
-
-// the problem of wide slot blockIdx.y and its arrays
-struct WideView {
-    int n, nn;
-    int64_t off;
-    double* part;
-};
-
-__device__ __forceinline__ WideView wide_view(const WideLaunch& L)
-{
-    const BatchProblem P = L.problems[L.ids[blockIdx.y]];
-    WideView v;
-    v.n = P.side;
-    v.nn = P.side * P.side;
-    v.off = P.offset;
-    v.part = L.part + ((size_t)blockIdx.y * L.nbx + blockIdx.x) * 2;
-    return v;
-}
-
-#define WIDE_NODES(v) for (int t = blockIdx.x * kWideNT + threadIdx.x; t < (v).nn; t += L.nbx * kWideNT)
 
 __global__ __launch_bounds__(kWideNT) void k_wide_init(WideLaunch L)
 {
-    const WideView v = wide_view(L);
-    const double* b = L.b + v.off;
-    double* x = L.x + v.off;
-    float* r = L.r + v.off;
-    float* p = L.p + v.off;
-    const float* dinv = L.dinv32 + v.off;
+    const WideBlock m = L.full_map[blockIdx.x];
+    const WideSlot W = L.slots[m.slot];
+    const unsigned nn = (unsigned)W.n * W.n;
+    const double* b = L.b + W.offset;
+    double* x = L.x + W.offset;
+    float* r = L.r + W.offset;
+    float* p = L.p[0] + W.offset;
+    const float* dinv = L.dinv32 + W.offset;
     double bb = 0.0, rz = 0.0;
-    WIDE_NODES(v)
-    {
-        const double bi = b[t];
-        x[t] = 0.0;
-        const float rf = (float)bi;
-        r[t] = rf;
-        const float zf = L.jacobi ? rf * dinv[t] : rf;
-        p[t] = zf;
-        bb += bi * bi;
-        rz += (double)rf * (double)zf;
-    }
-    wide_partials(bb, rz, v.part);
-}
-
-__global__ __launch_bounds__(kWideNT) void k_wide_apply(WideLaunch L)
-{
-    if (L.state[blockIdx.y].done) return; // uniform per workgroup
-    const WideView v = wide_view(L);
-    const int n = v.n;
-    const float* wx = L.wx32 + v.off;
-    const float* wy = L.wy32 + v.off;
-    const float* p = L.p + v.off;
-    float* q = L.q + v.off;
-    double pq = 0.0;
-    WIDE_NODES(v)
-    {
-        const int i = t / n, j = t - i * n;
-        float qv = 0.f;
-        if (i > 0 && j > 0 && i + 1 < n && j + 1 < n) qv = apply_row<float>(wx, wy, p, n, i, j, t);
-        q[t] = qv;
-        pq += (double)p[t] * (double)qv;
-    }
-    wide_partials(pq, 0.0, v.part);
-}
-
-__global__ __launch_bounds__(kWideNT) void k_wide_update(WideLaunch L)
-{
-    const WideState& S = L.state[blockIdx.y];
-    if (S.done) return;
-    const double alpha = S.alpha;
-    const WideView v = wide_view(L);
-    double* x = L.x + v.off;
-    const float* p = L.p + v.off;
-    float* r = L.r + v.off;
-    const float* q = L.q + v.off;
-    const float* dinv = L.dinv32 + v.off;
-    double rz = 0.0, rr = 0.0;
-    WIDE_NODES(v)
-    {
-        x[t] += alpha * (double)p[t];
-        const float rf = (float)((double)r[t] - alpha * (double)q[t]);
-        r[t] = rf;
-        rz += (double)rf * (double)(L.jacobi ? rf * dinv[t] : rf);
-        rr += (double)rf * (double)rf;
-    }
-    wide_partials(rz, rr, v.part);
-}
-
-// FP64 residual b − A x: replaces r (FP32) when the problem's scalar phase
-// asked for it; with `report`, only its square norm, for problems that did
-// not converge
-__global__ __launch_bounds__(kWideNT) void k_wide_residual(WideLaunch L, int report)
-{
-    const WideState& S = L.state[blockIdx.y];
-    if (report ? S.converged != 0 : (S.done || !S.replace_now)) return;
-    const WideView v = wide_view(L);
-    const int n = v.n;
-    const double* b = L.b + v.off;
-    const double* x = L.x + v.off;
-    const double* wx = L.wx64 + v.off;
-    const double* wy = L.wy64 + v.off;
-    float* r = L.r + v.off;
-    const float* dinv = L.dinv32 + v.off;
-    double rr = 0.0, rz = 0.0;
-    WIDE_NODES(v)
-    {
-        const int i = t / n, j = t - i * n;
-        double res = 0.0;
-        if (i > 0 && j > 0 && i + 1 < n && j + 1 < n) res = b[t] - apply_row<double>(wx, wy, x, n, i, j, t);
-        rr += res * res;
-        if (!report) {
-            const float rf = (float)res;
-            r[t] = rf;
-            rz += (double)rf * (double)(L.jacobi ? rf * dinv[t] : rf);
+    for (unsigned t = m.index * kWideNodes + threadIdx.x; t < nn; t += W.nb * kWideNodes)
+#pragma unroll
+        for (int u = 0; u < kWU; ++u) {
+            const unsigned q = t + u * kWideNT;
+            if (q >= nn) break;
+            const double bi = b[q];
+            x[q] = 0.0;
+            const float rf = (float)bi;
+            r[q] = rf;
+            p[q] = 0.f;
+            const float zf = L.jacobi ? rf * dinv[q] : rf;
+            bb += bi * bi;
+            rz += (double)rf * (double)zf;
         }
-    }
-    wide_partials(rr, rz, v.part);
+    wide_partials(bb, rz, L.part2[1] + 2 * (size_t)(W.part + m.index));
 }
 
-__global__ __launch_bounds__(kWideNT) void k_wide_direction(WideLaunch L)
-{
-    const WideState& S = L.state[blockIdx.y];
-    if (S.done) return;
-    const float beta = (float)S.beta;
-    const WideView v = wide_view(L);
-    float* p = L.p + v.off;
-    const float* r = L.r + v.off;
-    const float* dinv = L.dinv32 + v.off;
-    WIDE_NODES(v) p[t] = (L.jacobi ? r[t] * dinv[t] : r[t]) + beta * p[t];
-}
-
-// one wavefront per problem: the block partials in a fixed order, then the
-// scalar recurrence of the persistent kernel
-__global__ __launch_bounds__(64) void k_wide_scalars(WideLaunch L, int phase)
+// the scalars before step 0 (one workgroup per wide problem)
+__global__ __launch_bounds__(kWideNT) void k_wide_start(WideLaunch L)
 {
     const int slot = blockIdx.x;
-    WideState& S = L.state[slot];
-    if (phase == W_FINAL ? S.converged != 0 : (phase != W_INIT && S.done)) return; // uniform
-    if (phase == W_REPLACED && !S.replace_now) return;
-    double v0 = 0.0, v1 = 0.0;
-    for (int q = threadIdx.x; q < L.nbx; q += 64) {
-        v0 += L.part[((size_t)slot * L.nbx + q) * 2];
-        v1 += L.part[((size_t)slot * L.nbx + q) * 2 + 1];
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        v0 += __shfl_down(v0, off, 64);
-        v1 += __shfl_down(v1, off, 64);
-    }
+    const WideSlot W = L.slots[slot];
+    double bb, rz;
+    wide_sums(L.part2[1] + 2 * (size_t)W.part, W.nb, bb, rz);
     if (threadIdx.x != 0) return;
-    switch (phase) {
-    case W_INIT:
-        S.bb = v0;
-        S.rz = v1;
-        S.tol2bb = L.tol * L.tol * v0;
-        S.rr_ref = v0;
-        S.rr_true = v0;
-        S.it = 0;
-        S.since = 0;
-        S.replace_now = 0;
-        S.converged = v0 == 0.0 ? 1 : 0;
-        S.done = (S.converged || L.max_it <= 0) ? 1 : 0;
-        break;
-    case W_ALPHA:
-        S.pq = v0;
-        S.alpha = S.rz / v0;
-        break;
-    case W_BETA:
-        S.it += 1;
-        S.since += 1;
-        S.rz_old = S.rz;
-        S.rz_new = v0;
-        S.rr_new = v1;
-        S.beta = v0 / S.rz_old;
-        S.rz = v0;
-        // replace when the recurrence claims convergence, when its residual
-        // fell 100-fold since the last replacement, or every `replace`
-        // iterations
-        S.replace_now = (v1 <= S.tol2bb || v1 < 1e-4 * S.rr_ref || S.since >= L.replace) ? 1 : 0;
-        if (!S.replace_now && S.it >= L.max_it) S.done = 1;
-        break;
-    case W_REPLACED:
-        S.rr_true = v0;
-        S.since = 0;
-        S.replace_now = 0;
-        if (v0 <= S.tol2bb) {
-            S.converged = 1;
-            S.done = 1;
-        } else {
-            S.beta = v1 / S.rz_old; // replaced <r,z> over the previous iteration's <r,z>
-            S.rz = v1;
-            S.rr_ref = v0;
-            if (S.it >= L.max_it) S.done = 1;
-        }
-        break;
-    case W_FINAL:
-        S.rr_true = v0;
-        break;
-    }
+    WideState S{};
+    S.bb = bb;
+    S.tol2bb = L.tol * L.tol * bb;
+    S.rz = rz;
+    S.rr_ref = bb;
+    S.rr_true = bb;
+    S.mode = W_START;
+    S.converged = bb == 0.0 ? 1 : 0;
+    S.done = (S.converged || L.max_it <= 0) ? 1 : 0;
+    L.state[L.nwide + slot] = S; // the state before step 0 has parity 1
     L.done[slot] = S.done;
 }
 
-__global__ void k_wide_results(WideLaunch L)
+__global__ __launch_bounds__(kWideNT) void k_wide_a(WideLaunch L, int s)
 {
-    const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= L.nwide) return;
-    const WideState& S = L.state[slot];
-    BatchResult& R = L.results[L.ids[slot]];
+    if ((int)blockIdx.x >= *L.nactive) return;
+    const WideBlock m = L.map[blockIdx.x];
+    const WideSlot W = L.slots[m.slot];
+    const WideState S = L.state[(s ^ 1) * L.nwide + m.slot];
+    WideState& out = L.state[s * L.nwide + m.slot];
+    const bool writer = m.index == 0 && threadIdx.x == 0;
+    if (S.done) {
+        if (writer) out = S;
+        return;
+    }
+    const int n = W.n;
+    const unsigned nn = (unsigned)n * n;
+    float* r = L.r + W.offset;
+    const float* dinv = L.dinv32 + W.offset;
+    const float* po = L.p[S.pcur] + W.offset;
+    const float* wx = L.wx32 + W.offset;
+    const float* wy = L.wy32 + W.offset;
+    const bool jac = L.jacobi != 0;
+    // the values of a node and its four neighbours, of up to kWU nodes: the
+    // first pass's are requested before the scalars they wait for
+    float rv[kWU][5], dv[kWU][5], pv[kWU][5], w[kWU][4];
+    bool in[kWU], have[kWU][5];
+    auto load = [&](unsigned t0) {
+#pragma unroll
+        for (int u = 0; u < kWU; ++u) {
+            const unsigned t = t0 + u * kWideNT;
+            const int i = t / (unsigned)n, j = t - (unsigned)i * n;
+            in[u] = t < nn && i > 0 && j > 0 && i + 1 < n && j + 1 < n;
+            have[u][0] = in[u];
+            have[u][1] = in[u] && i + 2 < n;
+            have[u][2] = in[u] && i > 1;
+            have[u][3] = in[u] && j + 2 < n;
+            have[u][4] = in[u] && j > 1;
+            const int c = in[u] ? (int)t : n + 1; // node n + 1 is interior: a safe address (n ≥ 3)
+            const int at[5] = {c, c + n, c - n, c + 1, c - 1};
+#pragma unroll
+            for (int q = 0; q < 5; ++q) {
+                rv[u][q] = r[at[q]];
+                pv[u][q] = po[at[q]];
+                dv[u][q] = jac ? dinv[at[q]] : 1.f;
+            }
+            w[u][0] = wx[c];
+            w[u][1] = wx[c - n];
+            w[u][2] = wy[c];
+            w[u][3] = wy[c - 1];
+        }
+    };
+    const unsigned t_first = m.index * kWideNodes + threadIdx.x;
+    load(t_first);
+
+    WideState N = S;
+    if (S.mode != W_START) {
+        double v0, v1;
+        wide_sums(L.part2[s ^ 1] + 2 * (size_t)W.part, W.nb, v0, v1);
+        if (S.mode == W_CG) {
+            N.it += 1;
+            N.since += 1;
+            N.rz_old = S.rz;
+            N.beta = v0 / S.rz;
+            N.rz = v0;
+            // replace when the recurrence claims convergence, when its
+            // residual fell 100-fold since the last replacement (FP32 drift
+            // grows with that ratio), or every `replace` iterations
+            if (v1 <= S.tol2bb || v1 < 1e-4 * S.rr_ref || N.since >= L.replace)
+                N.mode = W_REPLACE;
+            else if (N.it >= L.max_it)
+                N.done = 1;
+        } else {
+            N.rr_true = v0;
+            N.since = 0;
+            N.mode = W_CG;
+            if (v0 <= S.tol2bb) {
+                N.converged = 1;
+                N.done = 1;
+            } else {
+                N.beta = v1 / S.rz_old; // replaced <r,z> over the previous iteration's <r,z>
+                N.rz = v1;
+                N.rr_ref = v0;
+                if (N.it >= L.max_it) N.done = 1;
+            }
+        }
+    } else {
+        N.mode = W_CG;
+        N.beta = 0.0;
+    }
+    if (!N.done && N.mode == W_CG) N.pcur = S.pcur ^ 1;
+    if (writer) {
+        out = N;
+        if (N.done) L.done[m.slot] = 1;
+    }
+    if (N.done) return;
+
+    if (N.mode == W_REPLACE) {
+        const double* b = L.b + W.offset;
+        const double* x = L.x + W.offset;
+        const double* wx64 = L.wx64 + W.offset;
+        const double* wy64 = L.wy64 + W.offset;
+        double rr = 0.0, rz = 0.0;
+        for (unsigned t0 = t_first; t0 < nn; t0 += W.nb * kWideNodes)
+            for (int u = 0; u < kWU; ++u) {
+                const unsigned t = t0 + u * kWideNT;
+                if (t >= nn) break;
+                const int i = t / (unsigned)n, j = t - (unsigned)i * n;
+                double res = 0.0;
+                if (i > 0 && j > 0 && i + 1 < n && j + 1 < n)
+                    res = b[t] - apply_row<double>(wx64, wy64, x, n, i, j, t);
+                const float rf = (float)res;
+                r[t] = rf;
+                rr += res * res;
+                rz += (double)rf * (double)(jac ? rf * dinv[t] : rf);
+            }
+        wide_partials(rr, rz, L.part2[s] + 2 * (size_t)(W.part + m.index));
+        return;
+    }
+
+    const float beta = (float)N.beta;
+    float* pn = L.p[N.pcur] + W.offset;
+    float* q = L.q + W.offset;
+    double pq = 0.0;
+    for (unsigned t0 = t_first; t0 < nn;) {
+        float p[kWU][5];
+#pragma unroll
+        for (int u = 0; u < kWU; ++u)
+#pragma unroll
+            for (int k = 0; k < 5; ++k)
+                p[u][k] = have[u][k] ? (jac ? rv[u][k] * dv[u][k] : rv[u][k]) + beta * pv[u][k] : 0.f;
+#pragma unroll
+        for (int u = 0; u < kWU; ++u) {
+            const unsigned t = t0 + u * kWideNT;
+            float qv = 0.f;
+            if (in[u])
+                qv = w[u][0] * (p[u][0] - p[u][1]) + w[u][1] * (p[u][0] - p[u][2]) + w[u][2] * (p[u][0] - p[u][3]) +
+                     w[u][3] * (p[u][0] - p[u][4]);
+            if (t < nn) {
+                pn[t] = p[u][0];
+                q[t] = qv;
+            }
+            pq += (double)p[u][0] * (double)qv;
+        }
+        t0 += W.nb * kWideNodes;
+        if (t0 < nn) load(t0);
+    }
+    wide_partials(pq, 0.0, L.part_pq + 2 * (size_t)(W.part + m.index));
+}
+
+__global__ __launch_bounds__(kWideNT) void k_wide_b(WideLaunch L, int s)
+{
+    if ((int)blockIdx.x >= *L.nactive) return;
+    const WideBlock m = L.map[blockIdx.x];
+    const WideSlot W = L.slots[m.slot];
+    const WideState& S = L.state[s * L.nwide + m.slot];
+    if (S.done || S.mode != W_CG) return; // uniform per workgroup
+    const double rz_now = S.rz;
+    const unsigned nn = (unsigned)W.n * W.n;
+    double* x = L.x + W.offset;
+    const float* p = L.p[S.pcur] + W.offset;
+    float* r = L.r + W.offset;
+    const float* q = L.q + W.offset;
+    const float* dinv = L.dinv32 + W.offset;
+    const bool jac = L.jacobi != 0;
+    double xv[kWU];
+    float pv[kWU], rv[kWU], qv[kWU], dv[kWU];
+    auto load = [&](unsigned t0) {
+#pragma unroll
+        for (int u = 0; u < kWU; ++u) {
+            const unsigned t = t0 + u * kWideNT, c = t < nn ? t : 0u;
+            xv[u] = x[c];
+            pv[u] = p[c];
+            rv[u] = r[c];
+            qv[u] = q[c];
+            dv[u] = jac ? dinv[c] : 1.f;
+        }
+    };
+    const unsigned t_first = m.index * kWideNodes + threadIdx.x;
+    load(t_first);
+    double pq, unused;
+    wide_sums(L.part_pq + 2 * (size_t)W.part, W.nb, pq, unused);
+    const double alpha = rz_now / pq;
+    double rz = 0.0, rr = 0.0;
+    for (unsigned t0 = t_first; t0 < nn;) {
+#pragma unroll
+        for (int u = 0; u < kWU; ++u) {
+            const unsigned t = t0 + u * kWideNT;
+            if (t >= nn) continue;
+            x[t] = xv[u] + alpha * (double)pv[u];
+            const float rf = (float)((double)rv[u] - alpha * (double)qv[u]);
+            r[t] = rf;
+            rz += (double)rf * (double)(jac ? rf * dv[u] : rf);
+            rr += (double)rf * (double)rf;
+        }
+        t0 += W.nb * kWideNodes;
+        if (t0 < nn) load(t0);
+    }
+    wide_partials(rz, rr, L.part2[s] + 2 * (size_t)(W.part + m.index));
+}
+
+// ⟨r, r⟩ of the FP64 residual of the problems that did not converge
+__global__ __launch_bounds__(kWideNT) void k_wide_report(WideLaunch L, int s)
+{
+    const WideBlock m = L.full_map[blockIdx.x];
+    const WideSlot W = L.slots[m.slot];
+    if (L.state[s * L.nwide + m.slot].converged) return;
+    const int n = W.n;
+    const unsigned nn = (unsigned)n * n;
+    const double* b = L.b + W.offset;
+    const double* x = L.x + W.offset;
+    double rr = 0.0;
+    for (unsigned t0 = m.index * kWideNodes + threadIdx.x; t0 < nn; t0 += W.nb * kWideNodes)
+        for (int u = 0; u < kWU; ++u) {
+            const unsigned t = t0 + u * kWideNT;
+            if (t >= nn) break;
+            const int i = t / (unsigned)n, j = t - (unsigned)i * n;
+            double res = 0.0;
+            if (i > 0 && j > 0 && i + 1 < n && j + 1 < n)
+                res = b[t] - apply_row<double>(L.wx64 + W.offset, L.wy64 + W.offset, x, n, i, j, t);
+            rr += res * res;
+        }
+    wide_partials(rr, 0.0, L.part_pq + 2 * (size_t)(W.part + m.index));
+}
+
+__global__ __launch_bounds__(kWideNT) void k_wide_results(WideLaunch L, int s)
+{
+    const WideSlot W = L.slots[blockIdx.x];
+    const WideState& S = L.state[s * L.nwide + blockIdx.x];
+    double rr = S.rr_true, unused;
+    if (!S.converged) wide_sums(L.part_pq + 2 * (size_t)W.part, W.nb, rr, unused);
+    if (threadIdx.x != 0) return;
+    BatchResult& R = L.results[W.id];
     R.iterations = S.it;
     R.converged = S.converged;
-    R.true_relative_residual = S.bb == 0.0 ? 0.0 : sqrt(S.rr_true / S.bb);
+    R.true_relative_residual = S.bb == 0.0 ? 0.0 : sqrt(rr / S.bb);
 }
 
 __global__ void k_reset_queue(int* q) { *q = 0; }
@@ -607,31 +719,27 @@ int batched_enqueue(const BatchLaunch& L, hipStream_t s)
 
 int wide_init(const WideLaunch& L, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_wide_init, dim3(L.nbx, L.nwide), dim3(kWideNT), 0, s, L);
-    hipLaunchKernelGGL(k_wide_scalars, dim3(L.nwide), dim3(64), 0, s, L, (int)W_INIT);
+    hipLaunchKernelGGL(k_wide_init, dim3(L.full_blocks), dim3(kWideNT), 0, s, L);
+    hipLaunchKernelGGL(k_wide_start, dim3(L.nwide), dim3(kWideNT), 0, s, L);
     SIL_LAUNCH_CHECK();
     return SIL_OK;
 }
 
-int wide_iteration(const WideLaunch& L, hipStream_t s)
+int wide_steps(const WideLaunch& L, int steps, int grid, hipStream_t s)
 {
-    const dim3 g(L.nbx, L.nwide);
-    hipLaunchKernelGGL(k_wide_apply, g, dim3(kWideNT), 0, s, L);
-    hipLaunchKernelGGL(k_wide_scalars, dim3(L.nwide), dim3(64), 0, s, L, (int)W_ALPHA);
-    hipLaunchKernelGGL(k_wide_update, g, dim3(kWideNT), 0, s, L);
-    hipLaunchKernelGGL(k_wide_scalars, dim3(L.nwide), dim3(64), 0, s, L, (int)W_BETA);
-    hipLaunchKernelGGL(k_wide_residual, g, dim3(kWideNT), 0, s, L, 0);
-    hipLaunchKernelGGL(k_wide_scalars, dim3(L.nwide), dim3(64), 0, s, L, (int)W_REPLACED);
-    hipLaunchKernelGGL(k_wide_direction, g, dim3(kWideNT), 0, s, L);
+    for (int i = 0; i < steps; ++i) {
+        hipLaunchKernelGGL(k_wide_a, dim3(grid), dim3(kWideNT), 0, s, L, i & 1);
+        hipLaunchKernelGGL(k_wide_b, dim3(grid), dim3(kWideNT), 0, s, L, i & 1);
+    }
     SIL_LAUNCH_CHECK();
     return SIL_OK;
 }
 
 int wide_finish(const WideLaunch& L, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_wide_residual, dim3(L.nbx, L.nwide), dim3(kWideNT), 0, s, L, 1);
-    hipLaunchKernelGGL(k_wide_scalars, dim3(L.nwide), dim3(64), 0, s, L, (int)W_FINAL);
-    hipLaunchKernelGGL(k_wide_results, dim3((L.nwide + 255) / 256), dim3(256), 0, s, L);
+    // an even number of steps (or none) was taken: the last state has parity 1
+    hipLaunchKernelGGL(k_wide_report, dim3(L.full_blocks), dim3(kWideNT), 0, s, L, 1);
+    hipLaunchKernelGGL(k_wide_results, dim3(L.nwide), dim3(kWideNT), 0, s, L, 1);
     SIL_LAUNCH_CHECK();
     return SIL_OK;
 }

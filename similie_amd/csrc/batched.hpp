@@ -37,40 +37,62 @@ struct BatchLaunch {
     int grid;  // persistent workgroups
 };
 
-// Wide path: large problems, each spread over many workgroups.  One CG
-// iteration is a sequence of kernels (per-block partial sums, a per-problem
-// scalar kernel that reduces them in a fixed order); kernel boundaries are
-// the only synchronisation between workgroups.  Same arithmetic as the
-// persistent kernel: FP32 recurrence, FP64 x, dot products and scalars, FP64
-// residual replacement, convergence only on the FP64 residual.
+// Wide path: large problems, each spread over many workgroups.  A step of
+// every problem is two kernels (batched.hip); kernel boundaries are the only
+// synchronisation between workgroups.  Same arithmetic as the persistent
+// kernel: FP32 recurrence, FP64 x, dot products and scalars, FP64 residual
+// replacement, convergence only on the FP64 residual.
 struct WideState {
-    double bb, tol2bb, rz, rz_old, rr_ref, rr_true, alpha, beta, pq, rz_new, rr_new;
-    int32_t it, since, converged, done, replace_now, pad;
+    double bb, tol2bb, rz, rz_old, rr_ref, rr_true, beta;
+    int32_t it, since, converged, done, mode;
+    int32_t pcur; // direction buffer that holds the latest p
+};
+
+constexpr int kWideNodes = 1024;    // nodes of a workgroup per pass
+constexpr int kWideMaxBlocks = 256; // most workgroups per problem (each sums the partials of all)
+
+// a wide problem: its arrays, its workgroups and their partial sums
+struct WideSlot {
+    int64_t offset;
+    int32_t n, id;
+    int32_t nb;   // workgroups
+    int32_t part; // slot of the first one's partials
+};
+
+// workgroup `index` of wide problem `slot`
+struct WideBlock {
+    int32_t slot, index;
 };
 
 struct WideLaunch {
-    const BatchProblem* problems;
-    const int* ids;      // problem of each wide slot
+    const WideSlot* slots;
     int nwide;
-    int nbx;             // workgroups per problem
+    const WideBlock* full_map; // every workgroup of every problem
+    int full_blocks;
+    const WideBlock* map;      // the workgroups of the problems still running
+    const int* nactive;        // their number
     const float *wx32, *wy32;
     const double *wx64, *wy64;
     const double* b;
     double* x;
-    float *r, *p, *q;
+    float* r;
+    float* p[2];
+    float* q;
     const float* dinv32;
     int jacobi;
     double tol;
     int max_it;
     int replace;
-    WideState* state;
-    double* part;        // nwide · nbx · 2
-    int* done;           // nwide flags (host-visible through a copy)
+    WideState* state;  // [step parity][nwide]
+    double* part_pq;   // two values per workgroup
+    double* part2[2];  // by step parity, two values per workgroup
+    int* done;         // nwide flags (host-visible through a copy)
     BatchResult* results;
 };
 
 int wide_init(const WideLaunch& L, hipStream_t s);
-int wide_iteration(const WideLaunch& L, hipStream_t s);
+// an even number of steps on `grid` workgroups
+int wide_steps(const WideLaunch& L, int steps, int grid, hipStream_t s);
 int wide_finish(const WideLaunch& L, hipStream_t s);
 
 int batched_weights(const BatchProblem* problems_dev, int nprob, int max_side, const double* kappa, float* wx32,

@@ -5,6 +5,7 @@
 #include <cstdlib>
 #include <new>
 #include <numeric>
+#include <utility>
 #include <vector>
 
 #include "batched.hpp"
@@ -19,23 +20,35 @@ struct sil_batched_poisson_s {
     BatchProblem* problems_dev = nullptr;
     int* order_dev = nullptr;   // queue of the persistent kernel: the small problems, largest first
     int nsmall = 0;
-    // wide path: problems of side >= wide_side, each over nbx workgroups
-    int wide_side = 192;
+    // wide path: problems of side >= wide_side, each over at most nbx workgroups
+    int wide_side = 96;
     int nwide = 0, nbx = 1;
-    int nbx_max = 1; // workgroups per wide problem the partial-sum array holds
-    int* wide_ids_dev = nullptr;
+    int nbx_max = 1; // workgroups per wide problem the partial-sum arrays hold
+    std::vector<int> wide_ids;
+    std::vector<WideSlot> slots;      // host copies of the device arrays below
+    std::vector<WideBlock> full_map;
+    WideSlot* slots_dev = nullptr;
+    WideBlock *full_map_dev = nullptr, *map_dev = nullptr;
+    int* nactive_dev = nullptr;
     WideState* wide_state = nullptr;
-    double* wide_part = nullptr;
+    double* wide_part = nullptr;      // part_pq and the two part2 arrays
     int* wide_done = nullptr;
-    int* wide_done_host = nullptr; // pinned
-    hipGraphExec_t wide_graph = nullptr;
+    void* wide_host = nullptr;        // pinned: two of each of the three below
+    WideBlock* map_host[2] = {nullptr, nullptr};
+    int* nactive_host[2] = {nullptr, nullptr};
+    int* done_host[2] = {nullptr, nullptr};
+    hipEvent_t wide_event[2] = {nullptr, nullptr};
+    std::vector<std::pair<int, hipGraphExec_t>> wide_graphs; // by grid size
     int wide_max_it = -1, wide_replace = -1, wide_jacobi = -1;
     double wide_tol = -1.0;
+    float* p2 = nullptr;              // second direction buffer of the wide path
+    hipStream_t side_stream = nullptr; // the persistent kernel's, beside the wide path
+    hipEvent_t fork = nullptr, join = nullptr;
     int* queue = nullptr;
     float *wx32 = nullptr, *wy32 = nullptr, *r = nullptr, *p = nullptr, *q = nullptr, *dinv32 = nullptr;
     double *wx64 = nullptr, *wy64 = nullptr, *b = nullptr, *x = nullptr;
     BatchResult* results_dev = nullptr;
-    int block = 256;
+    int block = 512;
     int cus = 0;
     hipGraphExec_t graph = nullptr;
     int graph_block = 0;
@@ -46,18 +59,45 @@ struct sil_batched_poisson_s {
 
 namespace {
 
+void drop_wide_graphs(sil_batched_poisson h)
+{
+    for (auto& g : h->wide_graphs) (void)hipGraphExecDestroy(g.second);
+    h->wide_graphs.clear();
+}
+
+// the arrays of the current split between the two paths
+void free_split(sil_batched_poisson h)
+{
+    for (void* ptr : {(void*)h->order_dev, (void*)h->slots_dev, (void*)h->full_map_dev, (void*)h->map_dev,
+                      (void*)h->nactive_dev, (void*)h->wide_state, (void*)h->wide_part, (void*)h->wide_done})
+        if (ptr) (void)hipFree(ptr);
+    h->order_dev = nullptr;
+    h->slots_dev = nullptr;
+    h->full_map_dev = nullptr;
+    h->map_dev = nullptr;
+    h->nactive_dev = nullptr;
+    h->wide_state = nullptr;
+    h->wide_part = nullptr;
+    h->wide_done = nullptr;
+    if (h->wide_host) (void)hipHostFree(h->wide_host);
+    h->wide_host = nullptr;
+    if (h->graph) (void)hipGraphExecDestroy(h->graph);
+    h->graph = nullptr;
+    h->graph_block = 0;
+    drop_wide_graphs(h);
+}
+
 void release(sil_batched_poisson h)
 {
     if (!h) return;
-    for (void* ptr : {(void*)h->problems_dev, (void*)h->order_dev, (void*)h->queue, (void*)h->wx32, (void*)h->wy32,
-                      (void*)h->dinv32,
-                      (void*)h->r, (void*)h->p, (void*)h->q, (void*)h->wx64, (void*)h->wy64, (void*)h->b,
-                      (void*)h->x, (void*)h->results_dev, (void*)h->wide_ids_dev, (void*)h->wide_state,
-                      (void*)h->wide_part, (void*)h->wide_done})
+    free_split(h);
+    for (void* ptr : {(void*)h->problems_dev, (void*)h->queue, (void*)h->wx32, (void*)h->wy32, (void*)h->dinv32,
+                      (void*)h->r, (void*)h->p, (void*)h->p2, (void*)h->q, (void*)h->wx64, (void*)h->wy64,
+                      (void*)h->b, (void*)h->x, (void*)h->results_dev})
         if (ptr) (void)hipFree(ptr);
-    if (h->wide_done_host) (void)hipHostFree(h->wide_done_host);
-    if (h->graph) (void)hipGraphExecDestroy(h->graph);
-    if (h->wide_graph) (void)hipGraphExecDestroy(h->wide_graph);
+    for (hipEvent_t e : {h->wide_event[0], h->wide_event[1], h->fork, h->join})
+        if (e) (void)hipEventDestroy(e);
+    if (h->side_stream) (void)hipStreamDestroy(h->side_stream);
     delete h;
 }
 
@@ -144,10 +184,12 @@ int capture(sil_batched_poisson h, int block, double tol, int max_it, int replac
 WideLaunch wide_launch(sil_batched_poisson h, double tol, int max_it, int replace)
 {
     WideLaunch W{};
-    W.problems = h->problems_dev;
-    W.ids = h->wide_ids_dev;
+    W.slots = h->slots_dev;
     W.nwide = h->nwide;
-    W.nbx = h->nbx;
+    W.full_map = h->full_map_dev;
+    W.full_blocks = (int)h->full_map.size();
+    W.map = h->map_dev;
+    W.nactive = h->nactive_dev;
     W.wx32 = h->wx32;
     W.wy32 = h->wy32;
     W.wx64 = h->wx64;
@@ -155,7 +197,8 @@ WideLaunch wide_launch(sil_batched_poisson h, double tol, int max_it, int replac
     W.b = h->b;
     W.x = h->x;
     W.r = h->r;
-    W.p = h->p;
+    W.p[0] = h->p;
+    W.p[1] = h->p2;
     W.q = h->q;
     W.dinv32 = h->dinv32;
     W.jacobi = h->jacobi;
@@ -163,70 +206,149 @@ WideLaunch wide_launch(sil_batched_poisson h, double tol, int max_it, int replac
     W.max_it = max_it;
     W.replace = replace;
     W.state = h->wide_state;
-    W.part = h->wide_part;
+    const size_t parts = 2 * h->full_map.size();
+    W.part_pq = h->wide_part;
+    W.part2[0] = h->wide_part + parts;
+    W.part2[1] = h->wide_part + 2 * parts;
     W.done = h->wide_done;
     W.results = h->results_dev;
     return W;
 }
 
-// iterations of the wide path per graph launch (the host reads the done
-// flags between launches)
+// steps of the wide path per graph launch (even; the host reads the done
+// flags of one launch while the next runs)
 constexpr int kWideChunk = 8;
 
-int capture_wide(sil_batched_poisson h, double tol, int max_it, int replace)
+// the graph of kWideChunk steps on at least `blocks` workgroups: grids halve
+// from that of all problems, so few graphs serve a solve whose problems
+// finish one after the other
+int wide_graph(sil_batched_poisson h, const WideLaunch& W, int blocks, hipGraphExec_t* out)
 {
-    if (h->wide_graph && h->wide_tol == tol && h->wide_max_it == max_it && h->wide_replace == replace &&
-        h->wide_jacobi == h->jacobi)
-        return SIL_OK;
-    if (h->wide_graph) {
-        (void)hipGraphExecDestroy(h->wide_graph);
-        h->wide_graph = nullptr;
+    if (h->wide_tol != W.tol || h->wide_max_it != W.max_it || h->wide_replace != W.replace ||
+        h->wide_jacobi != W.jacobi) {
+        drop_wide_graphs(h);
+        h->wide_tol = W.tol;
+        h->wide_max_it = W.max_it;
+        h->wide_replace = W.replace;
+        h->wide_jacobi = W.jacobi;
     }
+    int grid = W.full_blocks;
+    while ((grid + 1) / 2 >= blocks && grid > 1) grid = (grid + 1) / 2;
+    for (auto& g : h->wide_graphs)
+        if (g.first == grid) {
+            *out = g.second;
+            return SIL_OK;
+        }
     hipStream_t cs;
     SIL_CHECK_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
-    hipGraph_t g;
+    hipGraph_t g = nullptr;
+    hipGraphExec_t exec = nullptr;
     hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
         (void)hipStreamDestroy(cs);
         set_error("batched: capture failed: %s", hipGetErrorString(e));
         return SIL_ERR_HIP;
     }
-    const WideLaunch W = wide_launch(h, tol, max_it, replace);
-    int rc = SIL_OK;
-    for (int i = 0; i < kWideChunk && rc == SIL_OK; ++i) rc = wide_iteration(W, cs);
+    const int rc = wide_steps(W, kWideChunk, grid, cs);
     e = hipStreamEndCapture(cs, &g);
-    if (rc == SIL_OK && e == hipSuccess) e = hipGraphInstantiate(&h->wide_graph, g, nullptr, nullptr, 0);
-    if (e == hipSuccess || rc != SIL_OK) (void)hipGraphDestroy(g);
+    if (rc == SIL_OK && e == hipSuccess) e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+    if (g) (void)hipGraphDestroy(g);
     (void)hipStreamDestroy(cs);
     if (rc) return rc;
     if (e != hipSuccess) {
         set_error("batched: graph failed: %s", hipGetErrorString(e));
         return SIL_ERR_HIP;
     }
-    h->wide_tol = tol;
-    h->wide_max_it = max_it;
-    h->wide_replace = replace;
-    h->wide_jacobi = h->jacobi;
+    h->wide_graphs.emplace_back(grid, exec);
+    *out = exec;
     return SIL_OK;
 }
 
 // the wide path to completion on stream s
 int solve_wide(sil_batched_poisson h, double tol, int max_it, int replace, hipStream_t s)
 {
-    int rc = capture_wide(h, tol, max_it, replace);
-    if (rc) return rc;
     const WideLaunch W = wide_launch(h, tol, max_it, replace);
-    if ((rc = wide_init(W, s))) return rc;
-    for (int64_t done_it = 0; done_it < max_it; done_it += kWideChunk) {
-        SIL_CHECK_HIP(hipMemcpyAsync(h->wide_done_host, h->wide_done, sizeof(int) * h->nwide,
-                                     hipMemcpyDeviceToHost, s));
-        SIL_CHECK_HIP(hipStreamSynchronize(s));
-        bool all = true;
-        for (int i = 0; i < h->nwide && all; ++i) all = h->wide_done_host[i] != 0;
-        if (all) break;
-        SIL_CHECK_HIP(hipGraphLaunch(h->wide_graph, s));
+    int rc = wide_init(W, s);
+    if (rc) return rc;
+    std::vector<char> running(h->nwide, 1);
+    int blocks = -1, buffer = 0; // workgroups of the running problems; -1: the device's map is to be written
+    // a problem takes at most one replacement step per iteration
+    const int64_t chunks = max_it <= 0 ? 0 : (2 * ((int64_t)max_it + 1) + kWideChunk - 1) / kWideChunk + 1;
+    for (int64_t c = 0; c < chunks; ++c) {
+        int active = 0;
+        for (int i = 0; i < h->nwide; ++i) active += running[i] ? h->slots[i].nb : 0;
+        if (active == 0) break;
+        // a new map when an eighth of the workgroups has nothing left to do
+        if (blocks < 0 || active <= blocks - (blocks + 7) / 8) {
+            buffer ^= 1; // the copy from the other buffer may still be under way
+            WideBlock* m = h->map_host[buffer];
+            for (const WideBlock& b : h->full_map)
+                if (running[b.slot]) *m++ = b;
+            *h->nactive_host[buffer] = active;
+            blocks = active;
+            SIL_CHECK_HIP(hipMemcpyAsync(h->map_dev, h->map_host[buffer], sizeof(WideBlock) * active,
+                                         hipMemcpyHostToDevice, s));
+            SIL_CHECK_HIP(
+                hipMemcpyAsync(h->nactive_dev, h->nactive_host[buffer], sizeof(int), hipMemcpyHostToDevice, s));
+        }
+        hipGraphExec_t g = nullptr;
+        if ((rc = wide_graph(h, W, blocks, &g))) return rc;
+        SIL_CHECK_HIP(hipGraphLaunch(g, s));
+        const int k = (int)(c & 1);
+        SIL_CHECK_HIP(
+            hipMemcpyAsync(h->done_host[k], h->wide_done, sizeof(int) * h->nwide, hipMemcpyDeviceToHost, s));
+        SIL_CHECK_HIP(hipEventRecord(h->wide_event[k], s));
+        if (c == 0) continue;
+        SIL_CHECK_HIP(hipEventSynchronize(h->wide_event[k ^ 1]));
+        for (int i = 0; i < h->nwide; ++i)
+            if (h->done_host[k ^ 1][i]) running[i] = 0;
     }
     return wide_finish(W, s);
+}
+
+// both paths on the handle's right-hand sides: the persistent kernel on its
+// own stream beside the wide path on s, which waits for it at the end.  On
+// return (errors included) the side stream has been waited for.
+int solve_both(sil_batched_poisson h, double tol, int max_it, int replace, hipStream_t s)
+{
+    int rc = SIL_OK;
+    if (h->nsmall && h->nwide) {
+        SIL_CHECK_HIP(hipEventRecord(h->fork, s));
+        SIL_CHECK_HIP(hipStreamWaitEvent(h->side_stream, h->fork, 0));
+        SIL_CHECK_HIP(hipGraphLaunch(h->graph, h->side_stream));
+        hipError_t e = hipEventRecord(h->join, h->side_stream);
+        rc = solve_wide(h, tol, max_it, replace, s);
+        if (e == hipSuccess) e = hipStreamWaitEvent(s, h->join, 0);
+        const hipError_t w = hipStreamSynchronize(h->side_stream);
+        if (rc) return rc;
+        SIL_CHECK_HIP(e);
+        SIL_CHECK_HIP(w);
+    } else if (h->nwide) {
+        rc = solve_wide(h, tol, max_it, replace, s);
+    } else {
+        SIL_CHECK_HIP(hipGraphLaunch(h->graph, s));
+    }
+    return rc;
+}
+
+// the workgroups of every wide problem for the current nbx, host and device
+int map_wide(sil_batched_poisson h)
+{
+    drop_wide_graphs(h);
+    h->slots.clear();
+    h->full_map.clear();
+    for (int i = 0; i < h->nwide; ++i) {
+        const BatchProblem& p = h->problems[h->wide_ids[i]];
+        const int64_t nn = (int64_t)p.side * p.side;
+        const int nb = (int)std::min<int64_t>(h->nbx, (nn + kWideNodes - 1) / kWideNodes);
+        h->slots.push_back(WideSlot{p.offset, p.side, h->wide_ids[i], nb, (int)h->full_map.size()});
+        for (int b = 0; b < nb; ++b) h->full_map.push_back(WideBlock{i, b});
+    }
+    if (h->nwide == 0) return SIL_OK;
+    SIL_CHECK_HIP(hipMemcpy(h->slots_dev, h->slots.data(), sizeof(WideSlot) * h->nwide, hipMemcpyHostToDevice));
+    SIL_CHECK_HIP(hipMemcpy(h->full_map_dev, h->full_map.data(), sizeof(WideBlock) * h->full_map.size(),
+                            hipMemcpyHostToDevice));
+    return SIL_OK;
 }
 
 // splits the problems between the persistent kernel (side < wide_side,
@@ -234,29 +356,18 @@ int solve_wide(sil_batched_poisson h, double tol, int max_it, int replace, hipSt
 // drops the captured graphs (they hold the previous split)
 int partition(sil_batched_poisson h, int wide_side)
 {
-    for (void* ptr : {(void*)h->order_dev, (void*)h->wide_ids_dev, (void*)h->wide_state, (void*)h->wide_part,
-                      (void*)h->wide_done})
-        if (ptr) (void)hipFree(ptr);
-    h->order_dev = nullptr;
-    h->wide_ids_dev = nullptr;
-    h->wide_state = nullptr;
-    h->wide_part = nullptr;
-    h->wide_done = nullptr;
-    if (h->wide_done_host) (void)hipHostFree(h->wide_done_host);
-    h->wide_done_host = nullptr;
-    if (h->graph) (void)hipGraphExecDestroy(h->graph);
-    if (h->wide_graph) (void)hipGraphExecDestroy(h->wide_graph);
-    h->graph = nullptr;
-    h->wide_graph = nullptr;
-    h->graph_block = 0;
+    free_split(h);
     h->wide_side = wide_side;
-    std::vector<int> order, wide;
-    int64_t max_wide_nn = 0;
+    std::vector<int> order;
+    h->wide_ids.clear();
+    int64_t max_wide_nn = 0, total_blocks = 0;
     for (int i = 0; i < h->nprob; ++i) {
         const int side = h->problems[i].side;
         if (side >= wide_side) {
-            wide.push_back(i);
-            max_wide_nn = std::max<int64_t>(max_wide_nn, (int64_t)side * side);
+            const int64_t nn = (int64_t)side * side;
+            h->wide_ids.push_back(i);
+            max_wide_nn = std::max(max_wide_nn, nn);
+            total_blocks += std::min<int64_t>(kWideMaxBlocks, (nn + kWideNodes - 1) / kWideNodes);
         } else {
             order.push_back(i);
         }
@@ -264,31 +375,31 @@ int partition(sil_batched_poisson h, int wide_side)
     std::stable_sort(order.begin(), order.end(),
                      [&](int a, int b) { return h->problems[a].side > h->problems[b].side; });
     h->nsmall = (int)order.size();
-    h->nwide = (int)wide.size();
-    // four nodes per thread of the largest wide problem, at most 256 workgroups per problem
-    h->nbx = (int)std::min<int64_t>(256, std::max<int64_t>(1, (max_wide_nn + 1023) / 1024));
+    h->nwide = (int)h->wide_ids.size();
+    // four nodes per thread, at most kWideMaxBlocks workgroups per problem
+    h->nbx = (int)std::min<int64_t>(kWideMaxBlocks, std::max<int64_t>(1, (max_wide_nn + kWideNodes - 1) / kWideNodes));
     h->nbx_max = h->nbx;
+    const int64_t nw = std::max(h->nwide, 1), nblk = std::max<int64_t>(total_blocks, 1);
     int rc;
-    if ((rc = dalloc(&h->order_dev, std::max(h->nsmall, 1))) || (rc = dalloc(&h->wide_ids_dev, std::max(h->nwide, 1))) ||
-        (rc = dalloc(&h->wide_state, std::max(h->nwide, 1))) ||
-        (rc = dalloc(&h->wide_part, (int64_t)std::max(h->nwide, 1) * h->nbx_max * 2)) ||
-        (rc = dalloc(&h->wide_done, std::max(h->nwide, 1))))
+    if ((rc = dalloc(&h->order_dev, std::max(h->nsmall, 1))) || (rc = dalloc(&h->slots_dev, nw)) ||
+        (rc = dalloc(&h->full_map_dev, nblk)) || (rc = dalloc(&h->map_dev, nblk)) ||
+        (rc = dalloc(&h->nactive_dev, 1)) || (rc = dalloc(&h->wide_state, 2 * nw)) ||
+        (rc = dalloc(&h->wide_part, 3 * 2 * nblk)) || (rc = dalloc(&h->wide_done, nw)))
         return rc;
-    if (hipHostMalloc(reinterpret_cast<void**>(&h->wide_done_host), sizeof(int) * std::max(h->nwide, 1)) !=
-        hipSuccess) {
-        h->wide_done_host = nullptr;
+    if (h->nwide && !h->p2 && (rc = dalloc(&h->p2, h->total))) return rc;
+    const size_t map_bytes = sizeof(WideBlock) * nblk, done_bytes = sizeof(int) * nw;
+    if (hipHostMalloc(&h->wide_host, 2 * (map_bytes + done_bytes + sizeof(int))) != hipSuccess) {
+        h->wide_host = nullptr;
         set_error("batched: pinned allocation failed");
         return SIL_ERR_HIP;
     }
-    hipError_t e = hipSuccess;
-    if (h->nsmall) e = hipMemcpy(h->order_dev, order.data(), sizeof(int) * h->nsmall, hipMemcpyHostToDevice);
-    if (e == hipSuccess && h->nwide)
-        e = hipMemcpy(h->wide_ids_dev, wide.data(), sizeof(int) * h->nwide, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        set_error("batched: %s", hipGetErrorString(e));
-        return SIL_ERR_HIP;
-    }
-    return SIL_OK;
+    char* at = static_cast<char*>(h->wide_host);
+    for (int k = 0; k < 2; ++k, at += map_bytes) h->map_host[k] = reinterpret_cast<WideBlock*>(at);
+    for (int k = 0; k < 2; ++k, at += done_bytes) h->done_host[k] = reinterpret_cast<int*>(at);
+    for (int k = 0; k < 2; ++k, at += sizeof(int)) h->nactive_host[k] = reinterpret_cast<int*>(at);
+    if (h->nsmall)
+        SIL_CHECK_HIP(hipMemcpy(h->order_dev, order.data(), sizeof(int) * h->nsmall, hipMemcpyHostToDevice));
+    return map_wide(h);
 }
 
 // a fixed number of iterations of every problem (tolerance 0): equal work
@@ -301,8 +412,7 @@ int probe(sil_batched_poisson h, int iterations, double* seconds)
     for (int rep = 0; rep < 2; ++rep) { // a warm-up, then the timed run
         SIL_CHECK_HIP(hipDeviceSynchronize());
         const auto t0 = std::chrono::steady_clock::now();
-        if (h->nwide && (rc = solve_wide(h, 0.0, iterations, replace, 0))) return rc;
-        if (h->nsmall) SIL_CHECK_HIP(hipGraphLaunch(h->graph, 0));
+        if ((rc = solve_both(h, 0.0, iterations, replace, 0))) return rc;
         SIL_CHECK_HIP(hipDeviceSynchronize());
         *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     }
@@ -333,7 +443,13 @@ int sil_batched_poisson2d_create(sil_batched_poisson* out, int32_t nproblems, co
         h->max_side = std::max(h->max_side, (int)sides[i]);
     }
     h->total = off;
-    int wide_side = 192;
+    // Problems of at least this side take the wide path.  Both paths run at
+    // once, so the line lies where the persistent kernel's largest problem (one
+    // workgroup) ends before the wide path does.  128 problems of sides 32–512:
+    // 145–146 ms for lines from 48 to 128, 150 at 192; 30 of sides 20–180: 9.3 ms
+    // up to 96, 10.8 at 128, 21 at 160, 30 at 192 (none wide); 100 of sides 17–90:
+    // 4.8 ms at 96 (none wide), 4.9 at 48.
+    int wide_side = 96;
     if (const char* e = std::getenv("SIL_BATCH_WIDE_SIDE")) wide_side = std::max(3, std::atoi(e));
     int rc;
     if ((rc = dalloc(&h->problems_dev, nproblems)) || (rc = dalloc(&h->queue, 1)) || (rc = dalloc(&h->wx32, off)) ||
@@ -346,6 +462,15 @@ int sil_batched_poisson2d_create(sil_batched_poisson* out, int32_t nproblems, co
     }
     // small problems: one workgroup each in the persistent kernel, largest
     // first; large ones: the wide path
+    if (hipStreamCreateWithFlags(&h->side_stream, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&h->fork, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&h->join, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&h->wide_event[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&h->wide_event[1], hipEventDisableTiming) != hipSuccess) {
+        release(h);
+        set_error("batched_poisson2d_create: stream or event creation failed");
+        return SIL_ERR_HIP;
+    }
     if ((rc = partition(h, wide_side))) {
         release(h);
         return rc;
@@ -360,6 +485,10 @@ int sil_batched_poisson2d_create(sil_batched_poisson* out, int32_t nproblems, co
         set_error("batched_poisson2d_create: %s", hipGetErrorString(e));
         return SIL_ERR_HIP;
     }
+    // while a compute unit has at most two problems, 16 wavefronts each beat
+    // eight (30 of sides 20–180: 9.2 against 10.0 ms) and four, the default of
+    // before (100 of sides 17–90: 4.8 against 6.9 ms)
+    h->block = h->nsmall <= 2 * h->cus ? 1024 : 512;
     rc = batched_weights(h->problems_dev, nproblems, h->max_side, kappa, h->wx32, h->wy32, h->wx64, h->wy64,
                          h->dinv32, 0);
     if (rc == SIL_OK && hipDeviceSynchronize() != hipSuccess) rc = SIL_ERR_HIP;
@@ -402,8 +531,7 @@ int sil_batched_poisson2d_solve(sil_batched_poisson h, const double* rhs, double
     SIL_CHECK_HIP(hipMemcpyAsync(h->b, rhs, sizeof(double) * h->total, hipMemcpyDeviceToDevice, s));
     SIL_CHECK_HIP(hipStreamSynchronize(s));
     const auto t0 = std::chrono::steady_clock::now();
-    if (h->nwide && (rc = solve_wide(h, st->relative_tolerance, st->max_iterations, replace, s))) return rc;
-    if (h->nsmall) SIL_CHECK_HIP(hipGraphLaunch(h->graph, s));
+    if ((rc = solve_both(h, st->relative_tolerance, st->max_iterations, replace, s))) return rc;
     SIL_CHECK_HIP(hipStreamSynchronize(s));
     const double dt = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     if (seconds) *seconds = dt;
@@ -483,8 +611,7 @@ int sil_batched_poisson2d_autotune_shape(sil_batched_poisson h, const double* rh
         for (int a = 0; a < (h->nwide ? 3 : 1); ++a) {
             if (a > 0 && nbx_c[a] == nbx_c[a - 1]) continue;
             h->nbx = nbx_c[a];
-            if (h->wide_graph) (void)hipGraphExecDestroy(h->wide_graph);
-            h->wide_graph = nullptr;
+            if ((rc = map_wide(h))) return rc;
             for (int c = 0; c < (h->nsmall ? 3 : 1); ++c) {
                 h->block = blocks[c];
                 double dt = 0.0;
@@ -502,6 +629,7 @@ int sil_batched_poisson2d_autotune_shape(sil_batched_poisson h, const double* rh
     int rc = partition(h, best.wide_side);
     if (rc) return rc;
     h->nbx = std::min(best.wide_workgroups, h->nbx_max);
+    if ((rc = map_wide(h))) return rc;
     h->block = best.block;
     *chosen = best;
     return SIL_OK;

@@ -111,3 +111,37 @@ def test_shape_autotune_keeps_every_problem_solved():
         assert np.linalg.norm(r) <= 1.0001e-10 * np.linalg.norm(rhs[p])
     x2, results2, _ = solver.solve(b)
     assert torch.equal(x, x2) and [r["iterations"] for r in results2] == [r["iterations"] for r in results]
+
+
+@pytest.mark.parametrize("limit", [1, 7, 8, 9, 17])
+@pytest.mark.parametrize("replace", [0, 3])
+def test_wide_and_persistent_paths_take_the_same_iterations(limit, replace, monkeypatch):
+    """A limit on the iterations inside, at the end of and just after a chunk
+    of steps, with and without replacement steps of their own in between:
+    the wide path counts and iterates as the persistent kernel does (FP32
+    recurrences of at most 17 iterations, sums in another order: 1e-4)."""
+    from similie_amd.batched import BatchedPoisson2D
+    from similie_amd.solvers import StrongFormulationSolverSettings
+
+    sides, kap, rhs = problems(7, 9, 3, 70)
+    sides[0], sides[1] = 3, 33  # one unknown; 1089 nodes: a second workgroup of 65
+    rng = np.random.default_rng(3)
+    kap = [np.exp(rng.standard_normal((n, n))) for n in sides]
+    rhs = [np.pad(rng.standard_normal((n - 2, n - 2)), 1) for n in sides]
+    rhs[4][:] = 0.0  # solved before the first step
+    kappa = torch.from_numpy(np.concatenate([k.ravel() for k in kap])).cuda()
+    b = torch.from_numpy(np.concatenate([r.ravel() for r in rhs])).cuda()
+    st = StrongFormulationSolverSettings(relative_tolerance=1e-10, precision="mixed", preconditioner="jacobi",
+                                         max_iterations=limit, replace_interval=replace)
+    got = []
+    for side in ("3", "100000"):
+        monkeypatch.setenv("SIL_BATCH_WIDE_SIDE", side)
+        x, results, _ = BatchedPoisson2D(sides, kappa).solve(b, settings=st)
+        got.append((x.cpu().numpy(), results))
+    (xw, rw), (xp, rp) = got
+    for p, n in enumerate(sides):
+        assert rw[p]["iterations"] == rp[p]["iterations"] <= limit, p
+        assert rw[p]["converged"] == rp[p]["converged"], p
+        assert abs(rw[p]["true_relative_residual"] - rp[p]["true_relative_residual"]) <= \
+            1e-4 * rp[p]["true_relative_residual"] + 1e-10
+    assert np.linalg.norm(xw - xp) <= 1e-4 * np.linalg.norm(xp)
