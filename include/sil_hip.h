@@ -193,8 +193,8 @@ int sil_magnetostatics3d_create(sil_operator* out, int64_t nx, int64_t ny, int64
  * follow NonlinearMagnetostaticsHamiltonian with the InterpolatedNonlinear-
  * BHCurve of (bh_b, bh_h) (host arrays, 2..64 samples, bh_b increasing;
  * src/similie/physics/magnetostatics/nonlinear_magnetostatics.py:14-227), the
- * others are linear with mu_nodal.  sil_operator_apply gives F(x) and keeps
- * x's material state; sil_minimize_strong_formulation_residual runs the
+ * others are linear with mu_nodal.  sil_operator_apply gives F(x);
+ * sil_minimize_strong_formulation_residual runs the
  * reference's Newton branch (minimize_strong_formulation_residual.hpp
  * :1383-1569; identity or Jacobi; with SIL_PRECISION_MIXED the inner CG
  * applies the Jacobian in FP32 and converges on its FP64 residual, F(x)

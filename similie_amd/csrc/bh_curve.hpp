@@ -27,29 +27,67 @@ __device__ inline double h_from_b(const BhCurve& c, double b)
     return c.h[i] + c.dh_db[i] * (b - c.b[i]);
 }
 
-__device__ inline double dh_db_from_b(const BhCurve& c, double b)
+// The curve in LDS with its brackets laid out for a branch-free search:
+// edge[m] = q[m + 1] for the inner samples, +∞ from there on, so the bracket
+// of q is the number of edges below it.  (A search that stops at the bracket
+// is a chain of dependent reads, twice per node, and cost the curl-curl march
+// more than its memory: 83 µs for F on 113 × 97 × 129 nodes, 34 with the count.)
+struct BhTable {
+    alignas(16) double edge[kBhMax];
+    double b[kBhMax], h[kBhMax], dh[kBhMax];
+    int n;
+};
+
+// by every thread of the workgroup; the caller's barrier follows
+__device__ __forceinline__ void load_bh_table(BhTable& t, const BhCurve* __restrict__ c)
 {
-    if (b <= c.b[0]) return c.dh_db[0];
-    if (b >= c.b[c.n - 1]) return c.dh_db[c.n - 2];
-    return c.dh_db[bracket_q(c, b * b)];
+    const int n = c->n;
+    for (int i = threadIdx.x; i < kBhMax; i += blockDim.x) {
+        t.edge[i] = i + 2 < n ? c->q[i + 1] : __builtin_inf();
+        const int k = i < n ? i : 0;
+        t.b[i] = c->b[k];
+        t.h[i] = c->h[k];
+        t.dh[i] = c->dh_db[k];
+    }
+    if (threadIdx.x == 0) t.n = n;
 }
 
-// f, f′, f″ of f(q) = h(√q)/√q (h_over_b_from_q and its q-derivatives)
-__device__ inline void h_over_b_q(const BhCurve& c, double q, double& f, double& f1, double& f2)
+// the bracket of q = b²: the number of inner samples below it
+__device__ __forceinline__ int bh_bracket(const BhTable& t, double q)
 {
-    if (q == 0.0) {
-        f = dh_db_from_b(c, 0.0);
-        f1 = 0.0;
-        f2 = 0.0;
-        return;
+    typedef double D2 __attribute__((ext_vector_type(2)));
+    int i = 0;
+    for (int m = 0; m < t.n - 2; m += 8) {
+        const D2* e = reinterpret_cast<const D2*>(&t.edge[m]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const D2 v = e[u];
+            i += (q > v[0] ? 1 : 0) + (q > v[1] ? 1 : 0);
+        }
     }
-    const double b = sqrt(q);
-    const double h = h_from_b(c, b), dh = dh_db_from_b(c, b);
-    f = h / b;
-    const double d1 = (dh * b - h) / (b * b);             // d(h/b)/db
-    const double d2 = 2.0 * (h - dh * b) / (b * b * b);   // d²(h/b)/db²
-    f1 = d1 / (2.0 * b);
-    f2 = d2 / (4.0 * q) - d1 / (4.0 * q * b);
+    return i;
+}
+
+// h(b) on bracket i: constant below the first sample, along the last segment
+// past the end
+__device__ __forceinline__ double bh_h(const BhTable& t, int i, double b)
+{
+    return b <= t.b[0] ? t.h[0] : t.h[i] + t.dh[i] * (b - t.b[i]);
+}
+
+// The response of a node whose induction squares to q.  With the energy
+// ½ q f(q), f = h(b)/b, q = b²:
+//   ∂H/∂B = a B,  ∂²H/∂B∂B = a I + c B Bᵀ,
+//   a = f + q f′ = (h/b + h′)/2,   c = 2 (2 f′ + q f″) = (h′ − h/b)/(2 q)
+// (f′ = (h′ b − h)/(2 b³), f″ by one more derivative: h″ = 0 on a segment).
+__device__ __forceinline__ void bh_response(const BhTable& t, double q, double& a, double& c)
+{
+    const int i = bh_bracket(t, q);
+    const double b = sqrt(q), dh = t.dh[i], h = bh_h(t, i, b);
+    const bool zero = q == 0.0;
+    const double f = zero ? dh : h / b;
+    a = 0.5 * (f + dh);
+    c = zero ? 0.0 : (dh - f) / (2.0 * q);
 }
 
 }  // namespace sil

@@ -303,6 +303,7 @@ int sil_magnetostatics3d_apply_jacobian(sil_operator op, const double* state, co
     SIL_REQUIRE(op && state && in && out, SIL_ERR_INVALID, "magnetostatics3d_apply_jacobian: null argument");
     SIL_REQUIRE(op->kind == OP_MS3D_NONLINEAR, SIL_ERR_INVALID, "apply_jacobian: not a nonlinear operator");
     hipStream_t s = as_stream(stream);
+    if (ms3d_material_march_ok(op->ms)) return ms3d_material_jacobian64(op->ms, op->nl, state, in, out, s);
     int rc = ms3d_state(op->ms, op->nl, state, s);
     if (rc) return rc;
     return ms3d_jacobian_apply64(op->ms, op->nl, in, out, DotEpilogue{nullptr}, nullptr, nullptr, s);
@@ -312,10 +313,7 @@ int sil_magnetostatics3d_jacobian_diagonal(sil_operator op, const double* state,
 {
     SIL_REQUIRE(op && state && diag, SIL_ERR_INVALID, "magnetostatics3d_jacobian_diagonal: null argument");
     SIL_REQUIRE(op->kind == OP_MS3D_NONLINEAR, SIL_ERR_INVALID, "jacobian_diagonal: not a nonlinear operator");
-    hipStream_t s = as_stream(stream);
-    int rc = ms3d_state(op->ms, op->nl, state, s);
-    if (rc) return rc;
-    return ms3d_jacobian_diagonal(op->ms, op->nl, diag, s);
+    return ms3d_material_diagonal(op->ms, op->nl, state, diag, as_stream(stream));
 }
 
 int sil_magnetostatics3d_post_process(sil_operator op, const double* potential, const double* cell_mu,
@@ -647,8 +645,8 @@ int sil_operator_apply(sil_operator op, const double* in, double* out, void* str
 {
     SIL_REQUIRE(op && in && out, SIL_ERR_INVALID, "operator_apply: null argument");
     if (op->kind == OP_MS3D_NONLINEAR) {
-        // F(in); the operator keeps in's state (a later Jacobian is taken there)
         hipStream_t s = as_stream(stream);
+        if (ms3d_material_march_ok(op->ms)) return ms3d_material_apply64(op->ms, op->nl, in, out, s);
         int rc = ms3d_state(op->ms, op->nl, in, s);
         if (rc) return rc;
         return ms3d_state_apply64(op->ms, op->nl, in, out, s);

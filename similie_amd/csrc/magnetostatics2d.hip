@@ -161,6 +161,9 @@ __global__ void k_ms2d_state(int64_t nx, int64_t ny, const double* __restrict__ 
                              const BhCurve* __restrict__ curve, const double* __restrict__ x,
                              State2<double>* __restrict__ st, State2<float>* __restrict__ st32)
 {
+    __shared__ BhTable table;
+    load_bh_table(table, curve);
+    __syncthreads();
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (t >= nx * ny) return;
     const int64_t i = t % nx, j = t / nx;
@@ -170,10 +173,7 @@ __global__ void k_ms2d_state(int64_t nx, int64_t ny, const double* __restrict__ 
         by = x[t] - x[t + 1];
         if (ferro[t]) {
             const double q = bx * bx + by * by;
-            double f, f1, f2;
-            h_over_b_q(*curve, q, f, f1, f2);
-            a = f + q * f1;
-            c = 2.0 * (2.0 * f1 + q * f2);
+            bh_response(table, q, a, c);
         } else {
             a = nu[t];
         }

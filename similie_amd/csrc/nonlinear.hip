@@ -26,6 +26,7 @@
 #include <chrono>
 #include <cmath>
 #include <new>
+#include <type_traits>
 
 #include "bh_curve.hpp"
 #include "operators.hpp"
@@ -48,8 +49,6 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kNormBlocks = 1024;
 
-// ------------------------------------------------------------ B-H curve ---
-
 // ---------------------------------------------------------------- state ---
 
 struct StateArgs {
@@ -70,6 +69,9 @@ struct StateArgs {
 // the moment stencils), then (a, c) of its material
 __global__ __launch_bounds__(kBlock) void k_nl_state(StateArgs s, const double* __restrict__ x)
 {
+    __shared__ BhTable curve;
+    load_bh_table(curve, s.curve);
+    __syncthreads();
     const int64_t nn = s.nx * s.ny * s.nz;
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < nn; t += (int64_t)gridDim.x * blockDim.x) {
         const int64_t i = t % s.nx, j = (t / s.nx) % s.ny, k = t / (s.nx * s.ny);
@@ -87,10 +89,7 @@ __global__ __launch_bounds__(kBlock) void k_nl_state(StateArgs s, const double* 
             bz = A(i + 1, j, k, 1) - a0y - A(i, j + 1, k, 0) + a0x;
             if (s.ferro[t]) {
                 const double q = bx * bx + by * by + bz * bz;
-                double f, f1, f2;
-                h_over_b_q(*s.curve, q, f, f1, f2);
-                sa = f + q * f1;
-                sc = 2.0 * (2.0 * f1 + q * f2);
+                bh_response(curve, q, sa, sc);
             }
         }
         s.a[t] = sa;
@@ -167,6 +166,102 @@ __global__ __launch_bounds__(kBlock) void k_nl_jdiag(DiagArgs d, double* __restr
                     v += kReach[C][p].coeff * kReach[C][q].coeff * wk(kReach[C][p].m, kReach[C][q].m, i, j, k);
             diag[3 * t + C] = v + d.penalty * wa[C];
         }
+    }
+}
+
+// The same diagonal from the potential itself: the state of the four sampled
+// nodes n, n − e_x, n − e_y, n − e_z is formed here (three of them again by
+// their neighbours) instead of being written and read back, 129 bytes a node
+// for 24 of output: 113 × 97 × 129 nodes, state and diagonal 38 + 38 µs, this
+// 40–52.
+__global__ __launch_bounds__(kBlock) void k_nl_jdiag_at(StateArgs s, DiagArgs d, const double* __restrict__ x,
+                                                        double* __restrict__ diag)
+{
+    __shared__ BhTable curve;
+    load_bh_table(curve, s.curve);
+    __syncthreads();
+    const uint32_t nx = (uint32_t)s.nx, ny = (uint32_t)s.ny, nz = (uint32_t)s.nz;
+    const int64_t plane = s.nx * s.ny, nn = plane * s.nz;
+    for (int64_t t = blockIdx.x * (int64_t)kBlock + threadIdx.x; t < nn; t += (int64_t)gridDim.x * kBlock) {
+        uint32_t i, j, k;
+        if (nn <= UINT32_MAX) { // uniform: 32-bit divisions
+            i = (uint32_t)t % nx;
+            j = (uint32_t)t / nx % ny;
+            k = (uint32_t)t / nx / ny;
+        } else {
+            i = (uint32_t)(t % s.nx);
+            j = (uint32_t)(t / s.nx % s.ny);
+            k = (uint32_t)(t / plane);
+        }
+        auto interior = [&](uint32_t ii, uint32_t jj, uint32_t kk) {
+            return ii > 0 && jj > 0 && kk > 0 && ii + 1 < nx && jj + 1 < ny && kk + 1 < nz;
+        };
+        if (!interior(i, j, k)) {
+            diag[3 * t] = diag[3 * t + 1] = diag[3 * t + 2] = 1.0;
+            continue;
+        }
+        struct Node {
+            double K[3][3]; // w_m (a δ + c B_m B_m′)
+        };
+        // w_m K_mm′ at the node `back` steps behind along axis AX (interior or all zero)
+        auto node = [&](auto AX) {
+            constexpr int ax = decltype(AX)::value; // −1: n itself
+            const uint32_t ii = i - (ax == 0), jj = j - (ax == 1), kk = k - (ax == 2);
+            Node o{};
+            if (!interior(ii, jj, kk)) return o;
+            const int64_t at = ii + s.nx * (jj + s.ny * (int64_t)kk);
+            auto A = [&](uint32_t p, uint32_t q, uint32_t r, int64_t idx, int comp) {
+                return interior(p, q, r) ? x[3 * idx + comp] : 0.0;
+            };
+            const int64_t ex = at + 1, ey = at + s.nx, ez = at + plane;
+            const double a0x = x[3 * at], a0y = x[3 * at + 1], a0z = x[3 * at + 2];
+            const double B[3] = {A(ii, jj + 1, kk, ey, 2) - a0z - A(ii, jj, kk + 1, ez, 1) + a0y,
+                                 -A(ii + 1, jj, kk, ex, 2) + a0z + A(ii, jj, kk + 1, ez, 0) - a0x,
+                                 A(ii + 1, jj, kk, ex, 1) - a0y - A(ii, jj + 1, kk, ey, 0) + a0x};
+            double sa = s.nu[at], sc = 0.0;
+            if (s.ferro[at]) {
+                const double q = B[0] * B[0] + B[1] * B[1] + B[2] * B[2];
+                bh_response(curve, q, sa, sc);
+            }
+            const double lx = d.ls[0][ii], ly = d.ls[1][jj], lz = d.ls[2][kk];
+            const double ilx = d.inv_ls[0][ii], ily = d.inv_ls[1][jj], ilz = d.inv_ls[2][kk];
+            const double w[3] = {lx * ily * ilz, ly * ilx * ilz, lz * ilx * ily};
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+#pragma unroll
+                for (int mp = 0; mp < 3; ++mp) {
+                    const double K = (m == mp ? sa : 0.0) + sc * B[m] * B[mp];
+                    o.K[m][mp] = m == 1 ? w[m] * K * d.ysign : w[m] * K;
+                }
+            return o;
+        };
+        const Node n0 = node(std::integral_constant<int, -1>{});
+        const double lx = d.ls[0][i], ly = d.ls[1][j], lz = d.ls[2][k];
+        const double ilx = d.inv_ls[0][i], ily = d.inv_ls[1][j], ilz = d.inv_ls[2][k];
+        const double wa[3] = {ly * lz * ilx, lx * lz * ily, lx * ly * ilz};
+        const Node bx = node(std::integral_constant<int, 0>{});
+        const Node by = node(std::integral_constant<int, 1>{});
+        const Node bz = node(std::integral_constant<int, 2>{});
+        // the two single-moment neighbours, then the four products of the two
+        // moments at n (kReach), in the order of k_nl_jdiag
+        double v0 = bz.K[1][1] + by.K[2][2];
+        v0 += n0.K[1][1];
+        v0 -= n0.K[1][2];
+        v0 -= n0.K[2][1];
+        v0 += n0.K[2][2];
+        double v1 = bz.K[0][0] + bx.K[2][2];
+        v1 += n0.K[0][0];
+        v1 -= n0.K[0][2];
+        v1 -= n0.K[2][0];
+        v1 += n0.K[2][2];
+        double v2 = by.K[0][0] + bx.K[1][1];
+        v2 += n0.K[0][0];
+        v2 -= n0.K[0][1];
+        v2 -= n0.K[1][0];
+        v2 += n0.K[1][1];
+        diag[3 * t] = v0 + d.penalty * wa[0];
+        diag[3 * t + 1] = v1 + d.penalty * wa[1];
+        diag[3 * t + 2] = v2 + d.penalty * wa[2];
     }
 }
 
@@ -259,9 +354,10 @@ int ms3d_state(const Ms3dData& d, const NlData& nl, const double* x, hipStream_t
     return SIL_OK;
 }
 
-int ms3d_jacobian_diagonal(const Ms3dData& d, const NlData& nl, double* diag, hipStream_t s)
+namespace {
+DiagArgs diag_args(const Ms3dData& d, const NlData& nl)
 {
-    DiagArgs a{d.nx,
+    return DiagArgs{d.nx,
                d.ny,
                d.nz,
                d.divg ? 0.0 : d.penalty,
@@ -271,9 +367,30 @@ int ms3d_jacobian_diagonal(const Ms3dData& d, const NlData& nl, double* diag, hi
                nl.st_a,
                nl.st_c,
                {nl.st_b[0], nl.st_b[1], nl.st_b[2]}};
+}
+}  // namespace
+
+int ms3d_material_diagonal(const Ms3dData& d, const NlData& nl, const double* state, double* diag, hipStream_t s)
+{
+    StateArgs a{};
+    a.nx = d.nx;
+    a.ny = d.ny;
+    a.nz = d.nz;
+    a.nu = d.nu;
+    a.ferro = nl.ferro;
+    a.curve = nl.curve;
     const int64_t nn = d.nx * d.ny * d.nz;
     const unsigned g = static_cast<unsigned>(std::min<int64_t>((nn + kBlock - 1) / kBlock, 16384));
-    hipLaunchKernelGGL(k_nl_jdiag, dim3(g), dim3(kBlock), 0, s, a, diag);
+    hipLaunchKernelGGL(k_nl_jdiag_at, dim3(g), dim3(kBlock), 0, s, a, diag_args(d, nl), state, diag);
+    SIL_LAUNCH_CHECK();
+    return ms3d_gauge_diagonal_add(d, diag, s);
+}
+
+int ms3d_jacobian_diagonal(const Ms3dData& d, const NlData& nl, double* diag, hipStream_t s)
+{
+    const int64_t nn = d.nx * d.ny * d.nz;
+    const unsigned g = static_cast<unsigned>(std::min<int64_t>((nn + kBlock - 1) / kBlock, 16384));
+    hipLaunchKernelGGL(k_nl_jdiag, dim3(g), dim3(kBlock), 0, s, diag_args(d, nl), diag);
     SIL_LAUNCH_CHECK();
     return ms3d_gauge_diagonal_add(d, diag, s);
 }

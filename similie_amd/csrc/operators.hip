@@ -20,6 +20,7 @@
 #include <type_traits>
 
 #include "apply_epilogue.hpp"
+#include "bh_curve.hpp"
 #include "buffer_io.hpp"
 #include "operators.hpp"
 
@@ -45,12 +46,23 @@ struct MsArgs {
     const T* st_c;
     const T* st_b[3];
     const NodeState<T>* st4; // (a, c, B0_x, B0_y) per node
+    // the material itself (RESP_MATERIAL, RESP_JACOBIAN_AT): ferromagnetic
+    // flag per node, the B-H curve, and the potential the Jacobian is taken at
+    const uint8_t* ferro;
+    const BhCurve* curve;
+    const T* xs;
 };
 
 // material response of the curl-curl march: ν·B (linear), a·B (the
 // nonlinear operator at the state's own x) or a·δB + c·B0·(B0·δB) (its
-// Jacobian at the state)
-enum MsResponse { RESP_LINEAR = 0, RESP_SCALED = 1, RESP_JACOBIAN = 2 };
+// Jacobian at the state), with a, c and B0 from the stored state; or the same
+// two with the material evaluated in the march, from the B it forms anyway
+// (RESP_MATERIAL) or from a second potential marched beside the input
+// (RESP_JACOBIAN_AT): an application at a new state then writes and reads no
+// state (129 bytes a node written and 8 to 40 read back).  113 × 97 × 129
+// nodes: F 38 + 22 → 34 µs, J(x) v 38 + 45 → 42 µs.  FP64, pipelined march only;
+// CG, which applies J at one state many times, keeps the stored state.
+enum MsResponse { RESP_LINEAR = 0, RESP_SCALED = 1, RESP_JACOBIAN = 2, RESP_MATERIAL = 3, RESP_JACOBIAN_AT = 4 };
 
 // p_new = z + β p_old with z = D⁻¹ r (Jacobi) or r: the CG direction, in
 // the arithmetic of p_value.  The arrays are the solver's own (16-byte
@@ -340,8 +352,13 @@ struct MsPipeLds {
     double dot[TY];
 };
 
-// material record per node: ν (linear), a (the operator at its state) or
-// (a, c, B0x, B0y, B0z) (its Jacobian)
+template <typename T, int TY>
+struct MsPlanes {
+    T a[2][3][TY][64];
+};
+
+// material record per node: ν (linear, or the material evaluated here), a (the
+// operator at its state) or (a, c, B0x, B0y, B0z) (its Jacobian)
 template <int RESP>
 constexpr int ms_state_width()
 {
@@ -363,8 +380,13 @@ __global__ __launch_bounds__(64 * TY) void k_ms3d_pipe(MsArgs<T> a, const T* __r
                                                        int nty, int chunk, int64_t pstride)
 {
     constexpr bool PU = MODE == PIPE_PU, QD = MODE == PIPE_QDOTS;
+    constexpr bool MAT = RESP == RESP_MATERIAL || RESP == RESP_JACOBIAN_AT, XS = RESP == RESP_JACOBIAN_AT;
+    static_assert(!MAT || (MODE == PIPE_X && sizeof(T) == 8), "material responses: FP64 applications only");
     __shared__ MsPipeLds<T, TY> s;
+    __shared__ std::conditional_t<XS, MsPlanes<T, TY>, char> sx; // the state potential's planes
+    __shared__ std::conditional_t<MAT, BhTable, char> curve;
     if (pu.done && *pu.done) return; // uniform
+    if constexpr (MAT) load_bh_table(curve, a.curve);
     const int lane = threadIdx.x & 63, row = threadIdx.x >> 6;
 
     // XCD-contiguous tile order: hardware places workgroup b on XCD b % 8
@@ -407,12 +429,17 @@ __global__ __launch_bounds__(64 * TY) void k_ms3d_pipe(MsArgs<T> a, const T* __r
     const __amdgpu_buffer_rsrc_t rrr = buffer_of(QD ? pu.r + 3 * plane * k0 : x, QD ? in_bytes : 0);
     const __amdgpu_buffer_rsrc_t rpn = buffer_of(PU ? pu.p_new + 3 * plane * ka : out, PU ? out_bytes : 0);
     const double beta = PU ? *pu.beta : 0.0;
-    const T* st0 = RESP == RESP_LINEAR ? a.nu : (RESP == RESP_SCALED ? a.st_a : reinterpret_cast<const T*>(a.st4));
+    const T* st0 = (RESP == RESP_LINEAR || MAT)
+                       ? a.nu
+                       : (RESP == RESP_SCALED ? a.st_a : reinterpret_cast<const T*>(a.st4));
     const int64_t st0_width = RESP == RESP_JACOBIAN ? 4 : 1;
     const __amdgpu_buffer_rsrc_t rs0 =
         buffer_of(st0 + st0_width * plane * k0, (kb - k0) * plane * st0_width * (int64_t)sizeof(T));
     const __amdgpu_buffer_rsrc_t rs1 = buffer_of(RESP == RESP_JACOBIAN ? a.st_b[2] + plane * k0 : st0,
                                                  RESP == RESP_JACOBIAN ? (kb - k0) * plane * (int64_t)sizeof(T) : 0);
+    const __amdgpu_buffer_rsrc_t rfe =
+        buffer_of(MAT ? (const void*)(a.ferro + plane * k0) : st0, MAT ? (kb - k0) * plane : 0);
+    const __amdgpu_buffer_rsrc_t rxs = buffer_of(XS ? a.xs + 3 * plane * k0 : x, XS ? in_bytes : 0);
 
     // raw input of this lane's node in plane q (zero outside the planes
     // read): x, or (r, D⁻¹, p_old) under PU
@@ -446,9 +473,20 @@ __global__ __launch_bounds__(64 * TY) void k_ms3d_pipe(MsArgs<T> a, const T* __r
             }
         }
     };
+    auto load_xs = [&](int64_t q, T v[3]) {
+        if constexpr (XS)
+            buffer_load3<T>(rxs,
+                            (inij && q < qe)
+                                ? static_cast<uint32_t>(((q - k0) * plane + node) * 3 * (int64_t)sizeof(T))
+                                : kOutside,
+                            v);
+    };
     // material record of plane q (only planes k0 … kb−1 have an H)
-    auto load_state = [&](int64_t q, T m[SW]) {
+    auto load_state = [&](int64_t q, T m[SW], unsigned& ferro) {
         const bool ok = inij && q < kb;
+        if constexpr (MAT)
+            ferro = __builtin_amdgcn_raw_buffer_load_b8(
+                rfe, ok ? static_cast<uint32_t>((q - k0) * plane + node) : kOutside, 0, 0);
         const int64_t n = (q - k0) * plane + node;
         if constexpr (RESP == RESP_JACOBIAN) {
             buffer_load4<T>(rs0, ok ? static_cast<uint32_t>(n * 4 * (int64_t)sizeof(T)) : kOutside, m);
@@ -465,15 +503,21 @@ __global__ __launch_bounds__(64 * TY) void k_ms3d_pipe(MsArgs<T> a, const T* __r
     // requested into MB[u+1].  No register holding a load in flight is
     // copied, so the wavefront never waits for a load before its consumer.
     // RB: raw records in flight; PC: inputs formed from them (PC[u] = A(k))
-    T RB[3][RW], PC[3][3], MB[3][SW];
+    T RB[3][RW], PC[3][3], MB[3][SW], XB[3][3];
+    unsigned FB[3] = {0u, 0u, 0u};
     load(k0, RB[0]);
     load(k0 + 1, RB[1]);
-    load_state(k0, MB[0]);
+    load_xs(k0, XB[0]);
+    load_xs(k0 + 1, XB[1]);
+    load_state(k0, MB[0], FB[0]);
     input(RB[0], PC[0]);
     {
         const bool ik = interior(k0);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) s.a[0][c][row][lane] = ik ? PC[0][c] : T(0);
+        for (int c = 0; c < 3; ++c) {
+            s.a[0][c][row][lane] = ik ? PC[0][c] : T(0);
+            if constexpr (XS) sx.a[0][c][row][lane] = ik ? XB[0][c] : T(0);
+        }
     }
     __syncthreads();
 
@@ -486,7 +530,8 @@ __global__ __launch_bounds__(64 * TY) void k_ms3d_pipe(MsArgs<T> a, const T* __r
         const T* M0 = MB[u];
         const int buf = static_cast<int>(k - k0) & 1;
         load(k + 2, RB[u2]);
-        load_state(k + 1, MB[u1]);
+        load_xs(k + 2, XB[u2]);
+        load_state(k + 1, MB[u1], FB[u1]);
         input(RB[u1], PC[u1]);
         const T* P0 = PC[u];
         const T* P1 = PC[u1];
@@ -511,11 +556,39 @@ __global__ __launch_bounds__(64 * TY) void k_ms3d_pipe(MsArgs<T> a, const T* __r
             H[0] = cx * nu * bx;
             H[1] = cy * nu * by;
             H[2] = cz * nu * bz;
-        } else if constexpr (RESP == RESP_SCALED) {
-            const T sa = M0[0];
+        } else if constexpr (RESP == RESP_SCALED || RESP == RESP_MATERIAL) {
+            T sa = M0[0];
+            if constexpr (RESP == RESP_MATERIAL) {
+                if (ik && FB[u]) {
+                    double ra, rc;
+                    bh_response(curve, bx * bx + by * by + bz * bz, ra, rc);
+                    sa = ra;
+                }
+            }
             H[0] = cx * (bx * sa);
             H[1] = cy * (by * sa);
             H[2] = cz * (bz * sa);
+        } else if constexpr (RESP == RESP_JACOBIAN_AT) {
+            // the induction of the state potential, as of the input
+            T X0[3], X1[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                X0[c] = ik ? XB[u][c] : T(0);
+                X1[c] = ik1 ? XB[u1][c] : T(0);
+            }
+            const T sx1 = sx.a[buf][1][row][lp], sx2 = sx.a[buf][2][row][lp];
+            const T sy0 = sx.a[buf][0][rp][lane], sy2 = sx.a[buf][2][rp][lane];
+            const T b0x = sy2 - X0[2] - X1[1] + X0[1];
+            const T b0y = -sx2 + X0[2] + X1[0] - X0[0];
+            const T b0z = sx1 - X0[1] - sy0 + X0[0];
+            double sa = M0[0], sc = 0.0;
+            if (ik && FB[u]) bh_response(curve, b0x * b0x + b0y * b0y + b0z * b0z, sa, sc);
+            const T cd = sc * (b0x * bx + b0y * by + b0z * bz);
+            H[0] = cx * (sa * bx + cd * b0x);
+            H[1] = cy * (sa * by + cd * b0y);
+            H[2] = cz * (sa * bz + cd * b0z);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) sx.a[buf ^ 1][c][row][lane] = X1[c];
         } else {
             const T sa = M0[0], sc = M0[1], b0x = M0[2], b0y = M0[3], b0z = M0[4];
             const T cd = sc * (b0x * bx + b0y * by + b0z * bz);
@@ -964,7 +1037,8 @@ struct MsPipeShape {
 constexpr int64_t kComputeUnits = 256;
 constexpr int kMsPipeChunkDefault = 24;
 
-MsPipeShape ms_pipe_shape(const Ms3dData& d)
+// `rows`: 0, or the tile rows the kernel is built for
+MsPipeShape ms_pipe_shape(const Ms3dData& d, int rows = 0)
 {
     static const MsPipeShape fixed = [] {
         MsPipeShape p{-1, 0};
@@ -977,10 +1051,11 @@ MsPipeShape ms_pipe_shape(const Ms3dData& d)
         }
         return p;
     }();
-    if (fixed.ty >= 0) return fixed;
+    if (fixed.ty >= 0 && (rows == 0 || fixed.ty == 0)) return fixed;
     MsPipeShape best{16, kMsPipeChunkDefault};
     double least = 0.0;
     for (const int ty : {16, 8}) {
+        if (rows != 0 && ty != rows) continue;
         const int64_t tiles = ((d.nx + 61) / 62) * ((d.ny + ty - 3) / (ty - 2));
         for (int c = kMsPipeChunkDefault; c >= 2; --c) {
             const int64_t nb = tiles * ((d.nz + c - 1) / c);
@@ -1160,6 +1235,51 @@ int64_t max_dot_blocks() { return kMaxDotBlocks; }
 int ms3d_state_apply64(const Ms3dData& d, const NlData& nl, const double* x, double* out, hipStream_t s)
 {
     return ms_apply<double, RESP_SCALED>(d, x, out, DotEpilogue{nullptr}, nullptr, nullptr, s, &nl);
+}
+
+namespace {
+// an application with the material evaluated in the march (tiles of eight rows:
+// the record of the second potential needs the registers)
+template <int RESP>
+int ms_apply_material(const Ms3dData& d, const NlData& nl, const double* xs, const double* in, double* out,
+                      hipStream_t s)
+{
+    const MsPipeShape ps = ms_pipe_shape(d, 8);
+    MsArgs<double> a = ms_args<double>(d);
+    a.ferro = nl.ferro;
+    a.curve = nl.curve;
+    a.xs = xs;
+    const int ptx = (int)((d.nx + 61) / 62), pny = (int)((d.ny + 5) / 6);
+    const int64_t nb = (int64_t)ptx * pny * ((d.nz + ps.chunk - 1) / ps.chunk);
+    SIL_REQUIRE(nb <= INT32_MAX, SIL_ERR_UNSUPPORTED, "nonlinear operator: grid too large for one launch");
+    hipLaunchKernelGGL((k_ms3d_pipe<double, RESP, 8, PIPE_X>), dim3((unsigned)nb), dim3(64 * 8), 0, s, a, in, out,
+                       (double*)nullptr, PUpdate<double>{}, ptx, pny, ps.chunk, (int64_t)0);
+    SIL_LAUNCH_CHECK();
+    if (d.divg) {
+        hipLaunchKernelGGL((k_ms3d_gauge<double>), dim3(nblk(d.nx * d.ny * d.nz)), dim3(kBlock), 0, s, gauge_args(d),
+                           in, out, (double*)nullptr, (const int*)nullptr);
+        SIL_LAUNCH_CHECK();
+    }
+    return SIL_OK;
+}
+}  // namespace
+
+bool ms3d_material_march_ok(const Ms3dData& d)
+{
+    const MsPipeShape ps = ms_pipe_shape(d, 8);
+    const int64_t chunk_bytes = (int64_t)(ps.chunk + 2) * d.nx * d.ny * 3 * (int64_t)sizeof(double);
+    return ps.ty > 0 && d.nx >= 3 && d.ny >= 3 && d.nz >= 3 && chunk_bytes <= kMaxBufferBytes;
+}
+
+int ms3d_material_apply64(const Ms3dData& d, const NlData& nl, const double* x, double* out, hipStream_t s)
+{
+    return ms_apply_material<RESP_MATERIAL>(d, nl, nullptr, x, out, s);
+}
+
+int ms3d_material_jacobian64(const Ms3dData& d, const NlData& nl, const double* state, const double* in, double* out,
+                             hipStream_t s)
+{
+    return ms_apply_material<RESP_JACOBIAN_AT>(d, nl, state, in, out, s);
 }
 
 int ms3d_jacobian_apply64(const Ms3dData& d, const NlData& nl, const double* in, double* out, DotEpilogue dot,

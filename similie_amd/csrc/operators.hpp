@@ -168,6 +168,13 @@ int ms3d_jacobian_apply64(const Ms3dData& d, const NlData& nl, const double* in,
 int ms3d_jacobian_apply32(const Ms3dData& d, const NlData& nl, const float* in, float* out, DotEpilogue dot,
                           const PUpdate<float>* pu, int* nblocks_out, hipStream_t s);
 int ms3d_jacobian_diagonal(const Ms3dData& d, const NlData& nl, double* diag, hipStream_t s);
+// F(x), J(state)·in and the diagonal of J(state) in one kernel each, the stored
+// state untouched (the first two where ms3d_material_march_ok)
+bool ms3d_material_march_ok(const Ms3dData& d);
+int ms3d_material_apply64(const Ms3dData& d, const NlData& nl, const double* x, double* out, hipStream_t s);
+int ms3d_material_jacobian64(const Ms3dData& d, const NlData& nl, const double* state, const double* in, double* out,
+                             hipStream_t s);
+int ms3d_material_diagonal(const Ms3dData& d, const NlData& nl, const double* state, double* diag, hipStream_t s);
 
 // cell B, H, Maxwell stress and force density of a potential (postprocess.hip);
 // curve may be null when cell_nonlinear is

@@ -213,3 +213,28 @@ def test_nonlinear_solve_rejects_unsupported_settings(S):
     with pytest.raises(L.SilError, match="SpdIsai preconditioner runs in FP64"):
         S.minimize_strong_formulation_residual(op, b, settings=S.StrongFormulationSolverSettings(
             preconditioner="spd_isai", precision="mixed"))
+
+
+@pytest.mark.parametrize("samples", [2, 3, 10, 11, 63, 64])
+@pytest.mark.parametrize("shape", [(3, 3, 3), (63, 7, 4), (64, 8, 5), (65, 13, 9), (5, 4, 31)])
+def test_terms_at_one_state_match_the_oracle(S, shape, samples):
+    """F(x), J(x) v and the diagonal of J(x), each in one kernel with the
+    material evaluated inside: tiles one node short, full and one over, short
+    and long walks along z; curves that fill the bracket search's steps of
+    eight samples exactly, by one more and by one less; nodes with no field,
+    below the first sample (which is not at zero), on samples and far past the
+    last one.  Response and sums are a few dozen FP64 operations on values the
+    curl may cancel by a factor of 10: 1e-12 of the largest value."""
+    rng = np.random.default_rng(samples)
+    b = 0.02 + np.cumsum(rng.uniform(0.02, 0.1, samples))
+    h = np.cumsum(rng.uniform(20.0, 500.0, samples))
+    op, ref, rng = make(S, shape, sum(shape), bh=(b, h), penalty=50.0, ferro_share=0.7)
+    n = op.size()
+    x = rng.standard_normal((n // 3, 3)) * np.repeat(rng.choice([0.0, 0.005, 0.3, 5.0], n // 3), 3).reshape(-1, 3)
+    x[: n // 9] = 0.0
+    x = x.reshape(-1)
+    v = rng.standard_normal(n)
+    xt, vt = cuda(x), cuda(v)
+    assert rel(op.apply(xt).cpu().numpy(), ref.apply(x)) <= 1e-12
+    assert rel(op.apply_jacobian(xt, vt).cpu().numpy(), ref.jacobian_apply(x, v)) <= 1e-12
+    assert rel(op.jacobian_diagonal(xt).cpu().numpy(), ref.jacobian_diagonal(x)) <= 1e-12
