@@ -8,52 +8,44 @@
 
 namespace sil {
 
-__device__ inline int bracket_q(const BhCurve& c, double q)
-{
-    if (q <= c.q[0]) return 0;
-    for (int i = 0; i + 1 < c.n; ++i)
-        if (q <= c.q[i + 1]) return i;
-    return c.n - 2;
-}
-
-__device__ inline double h_from_b(const BhCurve& c, double b)
-{
-    if (b <= c.b[0]) return c.h[0];
-    if (b >= c.b[c.n - 1]) {
-        const int i = c.n - 2;
-        return c.h[i] + c.dh_db[i] * (b - c.b[i]);
-    }
-    const int i = bracket_q(c, b * b);
-    return c.h[i] + c.dh_db[i] * (b - c.b[i]);
-}
-
 // The curve in LDS with its brackets laid out for a branch-free search:
 // edge[m] = q[m + 1] for the inner samples, +∞ from there on, so the bracket
 // of q is the number of edges below it.  (A search that stops at the bracket
 // is a chain of dependent reads, twice per node, and cost the curl-curl march
 // more than its memory: 83 µs for F on 113 × 97 × 129 nodes, 34 with the count.)
-struct BhTable {
+struct BhEdges {
     alignas(16) double edge[kBhMax];
-    double b[kBhMax], h[kBhMax], dh[kBhMax];
     int n;
 };
 
+struct BhTable : BhEdges {
+    double b[kBhMax], h[kBhMax], dh_db[kBhMax];
+};
+
 // by every thread of the workgroup; the caller's barrier follows
+__device__ __forceinline__ void load_bh_edges(BhEdges& t, const BhCurve* __restrict__ c)
+{
+    const int n = c->n;
+    for (int i = threadIdx.x; i < kBhMax; i += blockDim.x) t.edge[i] = i + 2 < n ? c->q[i + 1] : __builtin_inf();
+    if (threadIdx.x == 0) t.n = n;
+}
+
 __device__ __forceinline__ void load_bh_table(BhTable& t, const BhCurve* __restrict__ c)
 {
     const int n = c->n;
     for (int i = threadIdx.x; i < kBhMax; i += blockDim.x) {
-        t.edge[i] = i + 2 < n ? c->q[i + 1] : __builtin_inf();
-        const int k = i < n ? i : 0;
-        t.b[i] = c->b[k];
-        t.h[i] = c->h[k];
-        t.dh[i] = c->dh_db[k];
+        // (entries past the last sample are never read)
+        const double q = c->q[i + 1 < kBhMax ? i + 1 : i], b = c->b[i], h = c->h[i], dh = c->dh_db[i];
+        t.edge[i] = i + 2 < n ? q : __builtin_inf();
+        t.b[i] = b;
+        t.h[i] = h;
+        t.dh_db[i] = dh;
     }
     if (threadIdx.x == 0) t.n = n;
 }
 
 // the bracket of q = b²: the number of inner samples below it
-__device__ __forceinline__ int bh_bracket(const BhTable& t, double q)
+__device__ __forceinline__ int bh_bracket(const BhEdges& t, double q)
 {
     typedef double D2 __attribute__((ext_vector_type(2)));
     int i = 0;
@@ -68,11 +60,12 @@ __device__ __forceinline__ int bh_bracket(const BhTable& t, double q)
     return i;
 }
 
-// h(b) on bracket i: constant below the first sample, along the last segment
-// past the end
-__device__ __forceinline__ double bh_h(const BhTable& t, int i, double b)
+// h(b) on bracket i of a table or the curve itself: constant below the first
+// sample, along the last segment past the end
+template <class Curve>
+__device__ __forceinline__ double bh_h(const Curve& t, int i, double b)
 {
-    return b <= t.b[0] ? t.h[0] : t.h[i] + t.dh[i] * (b - t.b[i]);
+    return b <= t.b[0] ? t.h[0] : t.h[i] + t.dh_db[i] * (b - t.b[i]);
 }
 
 // The response of a node whose induction squares to q.  With the energy
@@ -83,7 +76,7 @@ __device__ __forceinline__ double bh_h(const BhTable& t, int i, double b)
 __device__ __forceinline__ void bh_response(const BhTable& t, double q, double& a, double& c)
 {
     const int i = bh_bracket(t, q);
-    const double b = sqrt(q), dh = t.dh[i], h = bh_h(t, i, b);
+    const double b = sqrt(q), dh = t.dh_db[i], h = bh_h(t, i, b);
     const bool zero = q == 0.0;
     const double f = zero ? dh : h / b;
     a = 0.5 * (f + dh);

@@ -41,7 +41,7 @@ constexpr int kTx = 64;
 constexpr int kTy = 8;
 constexpr int kHx = kTx + 1;
 constexpr int kHy = kTy + 1;
-constexpr int kPostBlock = 256;
+constexpr int kPostBlock = 640;
 constexpr int kXcdCount = 8;
 
 struct PostArgs {
@@ -57,6 +57,17 @@ struct PostArgs {
     double* force;          // [cell][3] or null
     int64_t tiles_x, tiles_y, tiles, per_xcd;
 };
+
+// two consecutive values (the second only if `both`), streamed past the caches;
+// rows start at any 8-byte address
+__device__ __forceinline__ void store_pair(double* at, double v0, double v1, bool both)
+{
+    typedef double Pair __attribute__((ext_vector_type(2), aligned(8)));
+    if (both)
+        __builtin_nontemporal_store(Pair{v0, v1}, reinterpret_cast<Pair*>(at));
+    else
+        __builtin_nontemporal_store(v0, at);
+}
 
 // spacing of the cell-centre grid at centre i of m centres
 __device__ inline double centre_spacing(const double* c, int64_t m, int64_t i)
@@ -74,11 +85,14 @@ __device__ inline double centre_spacing(const double* c, int64_t m, int64_t i)
 // wavefront store covers 512 contiguous bytes) instead of one 24- or 48-byte
 // record per lane
 template <bool TWO_D, bool STAGED>
-__global__ void __launch_bounds__(kPostBlock) k_ms3d_post(PostArgs p)
+__global__ void __launch_bounds__(kPostBlock, 8) k_ms3d_post(PostArgs p)
 {
-    static_assert(kTx * kTy == 2 * kPostBlock, "two tile cells per thread");
+    static_assert(kHx * kHy <= kPostBlock, "one cell per thread, the halo's included");
     __shared__ double s_t[6][kHy * kHx];
     __shared__ double s_o[6][STAGED ? kTx * kTy : 1];
+    // (the brackets only: with the whole curve a compute unit holds two
+    // workgroups instead of three)
+    __shared__ BhEdges edges;
 
     // XCD-contiguous tiles: workgroup b runs on XCD b % 8, which takes a
     // contiguous range of tiles so vertical neighbours share its L2
@@ -95,18 +109,47 @@ __global__ void __launch_bounds__(kPostBlock) k_ms3d_post(PostArgs p)
     const int64_t sx = TWO_D ? 1 : 3, sy = sx * p.nx, sz = sy * p.ny;
     const double wz = TWO_D ? 1.0 : p.coord[2][k + 1] - p.coord[2][k];
 
-    for (int t = threadIdx.x; t < kHx * kHy; t += kPostBlock) {
-        const int lx = t % kHx, ly = t / kHx;
-        const int64_t i = i0 - 1 + lx, j = j0 - 1 + ly;
+    const int ht = threadIdx.x, hx_ = ht % kHx, hy_ = ht / kHx;
+    const int64_t hi = i0 - 1 + hx_, hj = j0 - 1 + hy_;
+    const bool here = ht < kHx * kHy && hi >= 0 && hi < mx && hj >= 0 && hj < my;
+    const int64_t cell = hi + mx * (hj + my * k);
+    // the cell's values are requested before the barrier that the curve's
+    // brackets need: potential at the cell's node and its three neighbours
+    // (2D: A_z at the node, e_x, e_y), μ, the material flag
+    double at[12], mu = 1.0, wx = 1.0, wy = 1.0;
+    bool iron = false;
+    if (here) {
+        const double* a0 = p.a + (hi * sx + hj * sy + k * sz);
+        if constexpr (TWO_D) {
+            at[0] = a0[0];
+            at[3] = a0[sx];
+            at[6] = a0[sy];
+        } else {
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                at[m] = a0[m];
+                at[3 + m] = m == 0 ? 0.0 : a0[sx + m];
+                at[6 + m] = m == 1 ? 0.0 : a0[sy + m];
+                at[9 + m] = m == 2 ? 0.0 : a0[sz + m];
+            }
+        }
+        wx = xc[hi + 1] - xc[hi];
+        wy = yc[hj + 1] - yc[hj];
+        iron = p.nonlinear && p.nonlinear[cell] != 0.0;
+        mu = p.mu[cell];
+    }
+    if (p.nonlinear) {
+        load_bh_edges(edges, p.curve);
+        __syncthreads();
+    }
+    if (ht < kHx * kHy) {
+        const int lx = hx_, ly = hy_, t = ht;
         double T[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        if (i >= 0 && i < mx && j >= 0 && j < my) {
-            const int64_t cell = i + mx * (j + my * k);
-            const double* a0 = p.a + (i * sx + j * sy + k * sz);
-            const double wx = xc[i + 1] - xc[i], wy = yc[j + 1] - yc[j];
+        if (here) {
             double B[3];
             if constexpr (TWO_D) {
-                const double mx_ = -a0[0] + a0[sy];  // moment of B_x, the stencil's order
-                const double my_ = a0[0] - a0[sx];   // moment of B_y
+                const double mx_ = -at[0] + at[6];  // moment of B_x, the stencil's order
+                const double my_ = at[0] - at[3];   // moment of B_y
                 const double rx = fabs(wx) < 1e-14 ? 0.0 : 1.0 / wx;
                 const double ry = fabs(wy) < 1e-14 ? 0.0 : 1.0 / wy;
                 B[0] = ry * mx_;
@@ -114,32 +157,31 @@ __global__ void __launch_bounds__(kPostBlock) k_ms3d_post(PostArgs p)
                 B[2] = 0.0;
             } else {
                 // forward_value moments, the taps in the stencil's order
-                double m0 = a0[sy + 2];
-                m0 = m0 - a0[2];
-                m0 = m0 - a0[sz + 1];
-                m0 = m0 + a0[1];
-                double m1 = -a0[sx + 2];
-                m1 = m1 + a0[2];
-                m1 = m1 + a0[sz + 0];
-                m1 = m1 - a0[0];
-                double m2 = a0[sx + 1];
-                m2 = m2 - a0[1];
-                m2 = m2 - a0[sy + 0];
-                m2 = m2 + a0[0];
+                double m0 = at[8];
+                m0 = m0 - at[2];
+                m0 = m0 - at[10];
+                m0 = m0 + at[1];
+                double m1 = -at[5];
+                m1 = m1 + at[2];
+                m1 = m1 + at[9];
+                m1 = m1 - at[0];
+                double m2 = at[4];
+                m2 = m2 - at[1];
+                m2 = m2 - at[6];
+                m2 = m2 + at[0];
                 B[0] = m0 / (wy * wz);
                 B[1] = m1 / (wx * wz);
                 B[2] = m2 / (wx * wy);
             }
             double H[3] = {0.0, 0.0, 0.0};
-            if (p.nonlinear && p.nonlinear[cell] != 0.0) {
+            if (iron) {
                 const double q = B[0] * B[0] + B[1] * B[1] + B[2] * B[2];
                 const double bn = sqrt(q);
                 if (bn != 0.0) {
-                    const double scale = h_from_b(*p.curve, bn) / bn;
+                    const double scale = bh_h(*p.curve, bh_bracket(edges, bn * bn), bn) / bn;
                     for (int m = 0; m < 3; ++m) H[m] = scale * B[m];
                 }
             } else {
-                const double mu = p.mu[cell];
                 for (int m = 0; m < 3; ++m) H[m] = B[m] / mu;
             }
             const double half = 0.5 * (B[0] * H[0] + B[1] * H[1] + B[2] * H[2]);
@@ -171,21 +213,24 @@ __global__ void __launch_bounds__(kPostBlock) k_ms3d_post(PostArgs p)
     const int64_t nv = mx - i0 < kTx ? mx - i0 : kTx;  // valid cells of each tile row
     if constexpr (STAGED) {
         __syncthreads();
+        // rows of W values a cell leave as pairs (an odd row's last one alone)
         if (p.induction || p.field)
-            for (int e = threadIdx.x; e < kTy * 3 * kTx; e += kPostBlock) {
-                const int r = e / (3 * kTx), q = e % (3 * kTx), cl = q / 3, m = q % 3;
+            for (int e = threadIdx.x; e < kTy * 3 * kTx / 2; e += kPostBlock) {
+                const int r = e / (3 * kTx / 2), q = 2 * (e % (3 * kTx / 2));
                 const int64_t j = j0 + r;
-                if (j >= my || cl >= nv) continue;
-                const int64_t base = 3 * (i0 + mx * (j + my * k));
-                if (p.induction) __builtin_nontemporal_store(s_o[m][r * kTx + cl], p.induction + base + q);
-                if (p.field) __builtin_nontemporal_store(s_o[3 + m][r * kTx + cl], p.field + base + q);
+                if (j >= my || q >= 3 * nv) continue;
+                const int64_t at = 3 * (i0 + mx * (j + my * k)) + q;
+                const int c0 = r * kTx + q / 3, m0 = q % 3, c1 = r * kTx + (q + 1) / 3, m1 = (q + 1) % 3;
+                if (p.induction) store_pair(p.induction + at, s_o[m0][c0], s_o[m1][c1], q + 1 < 3 * nv);
+                if (p.field) store_pair(p.field + at, s_o[3 + m0][c0], s_o[3 + m1][c1], q + 1 < 3 * nv);
             }
         if (p.stress)
-            for (int e = threadIdx.x; e < kTy * 6 * kTx; e += kPostBlock) {
-                const int r = e / (6 * kTx), q = e % (6 * kTx), cl = q / 6, m = q % 6;
+            for (int e = threadIdx.x; e < kTy * 6 * kTx / 2; e += kPostBlock) {
+                const int r = e / (6 * kTx / 2), q = 2 * (e % (6 * kTx / 2)), cl = q / 6, m = q % 6;
                 const int64_t j = j0 + r;
                 if (j >= my || cl >= nv) continue;
-                __builtin_nontemporal_store(s_t[m][(r + 1) * kHx + cl + 1], p.stress + 6 * (i0 + mx * (j + my * k)) + q);
+                const int c = (r + 1) * kHx + cl + 1;
+                store_pair(p.stress + 6 * (i0 + mx * (j + my * k)) + q, s_t[m][c], s_t[m + 1][c], true);
             }
         if (!p.force) return;
     } else {
@@ -193,13 +238,11 @@ __global__ void __launch_bounds__(kPostBlock) k_ms3d_post(PostArgs p)
         __syncthreads();
     }
 
-    double fo[2][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
-    int slot = 0;
-
-    for (int t = threadIdx.x; t < kTx * kTy; t += kPostBlock, ++slot) {
-        const int lx = 1 + t % kTx, ly = 1 + t / kTx;
-        const int64_t i = i0 - 1 + lx, j = j0 - 1 + ly;
-        if (i >= mx || j >= my) continue;
+    double fo[3] = {0.0, 0.0, 0.0};
+    const int t = threadIdx.x;
+    const int lx = 1 + t % kTx, ly = 1 + t / kTx;
+    const int64_t i = i0 - 1 + lx, j = j0 - 1 + ly;
+    if (t < kTx * kTy && i < mx && j < my) {
         const int c = ly * kHx + lx;
         const int cw = c - 1, cs = c - kHx;  // (i−1, j) and (i, j−1)
         const double hx = centre_spacing(xc, mx, i), hy = centre_spacing(yc, my, j);
@@ -214,7 +257,6 @@ __global__ void __launch_bounds__(kPostBlock) k_ms3d_post(PostArgs p)
         const double c2 = fabs(hx * hy) >= 1e-14 ? 1.0 / (fabs(hx) * fabs(hy)) : 0.0;
         // one-forms (ω_x, ω_y): (T_xx, T_xy), (T_xy, T_yy), (T_xz, T_yz)
         constexpr int kPick[3][2] = {{0, 3}, {3, 1}, {4, 5}};
-        const int64_t cell = i + mx * (j + my * k);
 #pragma unroll
         for (int f = 0; f < 3; ++f) {
             const double eta_y = cxy * s_t[kPick[f][0]][c];
@@ -226,22 +268,22 @@ __global__ void __launch_bounds__(kPostBlock) k_ms3d_post(PostArgs p)
             acc = acc + eta_y_w;
             acc = acc - eta_x_s;
             if constexpr (STAGED)
-                fo[slot][f] = c2 * -acc;
+                fo[f] = c2 * -acc;
             else
                 p.force[3 * cell + f] = c2 * -acc;
         }
     }
     if constexpr (STAGED) {
         __syncthreads();  // every read of s_o and s_t is done
-        slot = 0;
-        for (int t = threadIdx.x; t < kTx * kTy; t += kPostBlock, ++slot)
-            for (int f = 0; f < 3; ++f) s_o[f][t] = fo[slot][f];
+        if (t < kTx * kTy)
+            for (int f = 0; f < 3; ++f) s_o[f][t] = fo[f];
         __syncthreads();
-        for (int e = threadIdx.x; e < kTy * 3 * kTx; e += kPostBlock) {
-            const int r = e / (3 * kTx), q = e % (3 * kTx), cl = q / 3, m = q % 3;
-            const int64_t j = j0 + r;
-            if (j >= my || cl >= nv) continue;
-            __builtin_nontemporal_store(s_o[m][r * kTx + cl], p.force + 3 * (i0 + mx * (j + my * k)) + q);
+        for (int e = threadIdx.x; e < kTy * 3 * kTx / 2; e += kPostBlock) {
+            const int r = e / (3 * kTx / 2), q = 2 * (e % (3 * kTx / 2));
+            const int64_t jr = j0 + r;
+            if (jr >= my || q >= 3 * nv) continue;
+            store_pair(p.force + 3 * (i0 + mx * (jr + my * k)) + q, s_o[q % 3][r * kTx + q / 3],
+                       s_o[(q + 1) % 3][r * kTx + (q + 1) / 3], q + 1 < 3 * nv);
         }
     }
 }
