@@ -353,13 +353,23 @@ struct sil_staged_laplacian_s {
 };
 
 namespace sil {
-// Tile configuration of the fused 3D Laplacian; the environment overrides
-// it (SIL_LAP3D_TILE="variant,ty,xchunk[,zw or planes in flight]").
-FusedTile default_lap3d_tile()
+// Tile configuration of the fused 3D Laplacian by the output's extents; the
+// environment overrides it (SIL_LAP3D_TILE="variant,ty,xchunk[,zw or planes in
+// flight]").  The staged march with two planes of loads in flight and
+// non-temporal stores throughout.  From 12 million nodes on 16 rows and 32
+// planes a workgroup, which reads the least twice (256³, diagonal metric: 272
+// against 278–285 µs for 8 rows).  Below, that shape leaves the chip a last
+// wave of few workgroups, or idle (65³: 49 µs), and 8 rows with as many planes
+// as fill it are faster: 65³ 11.4, 107 × 75 × 93 16.4 (from 56),
+// 200 × 180 × 190 111 (from 146), 300 × 61 × 500 140 (from 160) µs.
+FusedTile default_lap3d_tile(const int64_t* ext)
 {
-    // staged march, 16-row tiles, two planes of loads in flight, 32 planes
-    // per workgroup, non-temporal output stores: the fastest measured shape
     FusedTile t{FUSED_STAGE, 2, 16, 32, 1};
+    if (ext != nullptr && ext[0] * ext[1] * ext[2] > 0 && ext[0] * ext[1] * ext[2] < 12000000) {
+        int64_t blocks = 0;
+        t.ty = 8;
+        t.xchunk = march_chunk(((ext[2] + 61) / 62) * ((ext[1] + 5) / 6), ext[0], 2, &blocks);
+    }
     if (const char* e = std::getenv("SIL_LAP3D_TILE")) {
         int v = 1, ty = 8, xc = 32, zw = 64;
         const int n = std::sscanf(e, "%d,%d,%d,%d", &v, &ty, &xc, &zw);
@@ -401,7 +411,7 @@ int sil_make_staged_laplacian(sil_staged_laplacian* out, sil_grid grid, int32_t 
         if (n == 2 && k == 0) op->path = 1;
         if (n == 3 && k == 1) op->path = 2;
     }
-    op->tile = default_lap3d_tile();
+    op->tile = default_lap3d_tile(op->path == 2 ? out_view->extent : nullptr);
     *out = op;
     return SIL_OK;
 }
@@ -453,7 +463,7 @@ int sil_staged_laplacian_autotune(sil_staged_laplacian op, double* out, const do
     // staged x-march (z neighbours by DPP): rows, planes in flight, planes per
     // workgroup; pipelined x-march: rows of 64 lanes
     const FusedTile candidates[] = {
-        {FUSED_STAGE, 2, 16, 32, 1}, {FUSED_STAGE, 1, 16, 32, 1}, {FUSED_STAGE, 2, 12, 32, 1},
+        op->tile, {FUSED_STAGE, 2, 16, 32, 1}, {FUSED_STAGE, 1, 16, 32, 1}, {FUSED_STAGE, 2, 12, 32, 1},
         {FUSED_STAGE, 2, 8, 32, 1},  {FUSED_STAGE, 2, 16, 24, 1}, {FUSED_STAGE, 2, 16, 40, 1},
         {FUSED_STAGE, 2, 16, 32, 0}, {FUSED_PIPE, 64, 12, 32, 1}, {FUSED_PIPE, 64, 16, 32, 0},
         {FUSED_PIPE, 64, 8, 32, 0},

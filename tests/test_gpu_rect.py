@@ -133,3 +133,37 @@ def test_degenerate_spacings_take_the_general_kernels():
         o = torch.empty(w.shape, dtype=torch.float64, device="cuda")
         E.laplacian(gg, k, o, cuda(w))
         assert close(o, orc.laplacian(og, k, w, extents)), k
+
+
+MARCH = [
+    ([2, 6, 62], (1, 2)),       # one full tile, one chunk
+    ([9, 7, 63], (1, 2)),       # one node past the tile along y and z
+    ([23, 13, 125], (1, 2)),    # chunks with a remainder
+    ([131, 63, 64], (0, 3)),    # 0- and 3-forms march from 500 000 nodes on
+]
+
+
+@pytest.mark.parametrize("kind", ["identity", "diagonal", "singular"])
+@pytest.mark.parametrize("extents,degrees", MARCH)
+def test_marching_laplacian_matches_oracle(extents, degrees, kind):
+    """Δ on 3D grids wide enough for the march (k_rect_lap3_march, and for
+    index-last 1-forms the fused march at the chunk its size selects)."""
+    import similie_amd.exterior as E
+
+    rng = np.random.default_rng(sum(extents))
+    axes = [np.cumsum(np.concatenate([[0.0], rng.uniform(0.5, 1.5, e - 1)])) for e in extents]
+    m = metric_of(rng, extents, 3, kind)
+    mk = orc.METRIC_IDENTITY if m is None else orc.METRIC_DIAGONAL
+    og = orc.Geometry(extents, axes=axes, metric_kind=mk, metric=None if m is None else m.reshape(-1, 3))
+    gg = E.Grid(extents, axis_coords=axes, metric=None if m is None else cuda(m), metric_kind=mk)
+    for k in degrees:
+        w = rng.standard_normal(tuple(extents) + (comb(3, k),))
+        for oext in (extents, [e - 1 for e in extents]):
+            ref = orc.laplacian(og, k, w, oext)
+            for order in orders(3):
+                t = stored(w.shape, order)
+                t.copy_(cuda(w))
+                o = stored(tuple(oext) + (comb(3, k),), order)
+                o.fill_(float("nan"))
+                E.laplacian(gg, k, o, t, comp_dim=3)
+                assert close(o, ref), (k, oext, order)
