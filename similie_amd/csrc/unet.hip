@@ -26,6 +26,7 @@
 // the flipped, channel-transposed weights with the ReLU mask applied while
 // the tile is staged; the weight gradient is a second MFMA GEMM over pixels
 // with per-workgroup partial sums reduced in a fixed order.
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <new>
@@ -61,14 +62,6 @@ constexpr long kComputeUnits = 256;
 struct alignas(16) Chunk8 {
     bf16 v[8];
 };
-
-__device__ __forceinline__ Chunk8 zero_chunk()
-{
-    Chunk8 c;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) c.v[i] = to_bf16(0.f);
-    return c;
-}
 
 // a D fragment of the transposed products (lane: one pixel, the channels
 // d_row(l, r)) after bias, as BF16 with optional ReLU (on the rounded
@@ -120,45 +113,12 @@ __device__ __forceinline__ TileWalk xcd_walk(int ntiles)
 // their combination (done when the chunk is written to LDS, so that the
 // loads of the next tile stay in flight while the current one is computed).
 template <int MODE>
-struct RawChunk {
-    static constexpr int n = MODE == ST_POOL ? 4 : (MODE == ST_PLAIN ? 1 : 2);
-    Chunk8 c[n];
-};
-
-template <int MODE>
-__device__ __forceinline__ void load_raw(RawChunk<MODE>& r, const bf16* __restrict__ X, const bf16* __restrict__ X2,
-                                         int b, int gy, int gx, int part, int H, int W)
-{
-    if (MODE == ST_POOL) {
-        const int W2 = 2 * W;
-        const size_t base = (((size_t)b * 2 * H + 2 * gy) * W2 + 2 * gx) * C + part * 8;
-        r.c[0] = *reinterpret_cast<const Chunk8*>(&X[base]);
-        r.c[1] = *reinterpret_cast<const Chunk8*>(&X[base + C]);
-        r.c[2] = *reinterpret_cast<const Chunk8*>(&X[base + (size_t)W2 * C]);
-        r.c[3] = *reinterpret_cast<const Chunk8*>(&X[base + (size_t)W2 * C + C]);
-        return;
-    }
-    const size_t off = (((size_t)b * H + gy) * W + gx) * C + part * 8;
-    r.c[0] = *reinterpret_cast<const Chunk8*>(&X[off]);
-    if (MODE == ST_UPADD) {
-        const size_t q = (((size_t)b * (H / 2) + gy / 2) * (W / 2) + gx / 2) * C + part * 8;
-        r.c[1] = *reinterpret_cast<const Chunk8*>(&X2[q]);
-    } else if (MODE == ST_MASK) {
-        r.c[1] = *reinterpret_cast<const Chunk8*>(&X2[off]);
-    }
-}
-
-template <int MODE>
-__device__ __forceinline__ void zero_raw(RawChunk<MODE>& r)
-{
-#pragma unroll
-    for (int i = 0; i < RawChunk<MODE>::n; ++i) r.c[i] = zero_chunk();
-}
+constexpr int kRaw = MODE == ST_POOL ? 4 : (MODE == ST_PLAIN ? 1 : 2);
 
 // the combination on packed words (two BF16 channels per word, the lower
 // channel in the low half), each sum formed in FP32 and rounded once
 template <int MODE>
-__device__ __forceinline__ U32x4 combine_words(const U32x4 (&w)[RawChunk<MODE>::n])
+__device__ __forceinline__ U32x4 combine_words(const U32x4 (&w)[kRaw<MODE>])
 {
     if constexpr (MODE == ST_PLAIN) {
         return w[0];
@@ -196,46 +156,13 @@ __device__ __forceinline__ Chunk8 chunk_of(U32x4 v)
     return c;
 }
 
-template <int MODE>
-__device__ __forceinline__ Chunk8 combine(const RawChunk<MODE>& r)
-{
-    U32x4 w[RawChunk<MODE>::n];
-#pragma unroll
-    for (int i = 0; i < RawChunk<MODE>::n; ++i) w[i] = words_of(r.c[i]);
-    return chunk_of(combine_words<MODE>(w));
-}
-
-template <int MODE>
-__device__ __forceinline__ Chunk8 stage_chunk(const bf16* __restrict__ X, const bf16* __restrict__ X2, int b, int gy,
-                                              int gx, int part, int H, int W)
-{
-    RawChunk<MODE> r;
-    load_raw<MODE>(r, X, X2, b, gy, gx, part, H, W);
-    return combine<MODE>(r);
-}
-
-// the (TH+2)×(TW+2) input tile with origin (oy0−1, ox0−1), zero outside
-template <int MODE>
-__device__ __forceinline__ void stage_tile(bf16* __restrict__ sX, const bf16* __restrict__ X,
-                                           const bf16* __restrict__ X2, int b, int oy0, int ox0, int H, int W)
-{
-    for (int c = threadIdx.x; c < (TH + 2) * (TW + 2) * 4; c += NT) {
-        const int pix = c >> 2, part = c & 3;
-        const int ty = pix / (TW + 2), tx = pix % (TW + 2);
-        const int gy = oy0 - 1 + ty, gx = ox0 - 1 + tx;
-        Chunk8 v = zero_chunk();
-        if (gy >= 0 && gy < H && gx >= 0 && gx < W) v = stage_chunk<MODE>(X, X2, b, gy, gx, part, H, W);
-        *reinterpret_cast<Chunk8*>(&sX[pix * CP + part * 8]) = v;
-    }
-}
-
 // The raw chunks of one staged chunk through buffer resources over one image
 // of X and X2: a chunk outside the image (in == false) reads zeros and needs
 // no branch, so the compiler's wait before the chunks are combined counts
 // only the loads issued before them.
 template <int MODE>
 struct RawBuf {
-    U32x4 c[RawChunk<MODE>::n];
+    U32x4 c[kRaw<MODE>];
 };
 
 template <int MODE>
@@ -430,87 +357,192 @@ __global__ __launch_bounds__(conv_threads(MODE), conv_wgs_per_cu(MODE)) void k_c
 
 // weight gradient: dW[tap][co][ci] += Σ_q dZ[q][co] · X[q + off(tap)][ci],
 // dZ = dY ⊙ [Yfwd > 0]; db[co] += Σ_q dZ[q][co].  One partial per workgroup
-// (grid-stride over tiles), reduced later in a fixed order.
-template <int MODE>
-__global__ __launch_bounds__(NT) void k_conv33_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ X2,
-                                                     const bf16* __restrict__ dY, const bf16* __restrict__ Yf,
-                                                     float* __restrict__ part_w, float* __restrict__ part_b, int B,
-                                                     int H, int W)
+// (a walk over tiles), reduced later in a fixed order.
+//
+// The products sum over pixels, so both operands are wanted with consecutive
+// pixels in a lane while the tensors hold consecutive channels: they are
+// transposed as they are staged, X by 4 and dZ by 2 pixels × 8 channels a
+// thread, into [channel][pixel] planes whose pitches (an odd multiple of 16
+// bytes) keep the 16-byte fragment reads of 32 channels off each other's
+// banks.  One 20-byte read of a lane then holds the pixels of all three kx,
+// shifted into place in registers, and each of 8 wavefronts runs the 9 taps of
+// one output row (18 MFMAs a tile on 10 LDS reads of 16 bytes).  As in
+// k_conv33 the loads of the tile after next are in flight while one is
+// computed, through buffer resources, with the planes double-buffered (84 KB:
+// one workgroup a compute unit).  16 images of 256²: 54 µs for the full-size
+// layers, near the 42 their three tensors take to stream; the 32² to 128² ones
+// 9–20 µs, half of it launch and the closing sums.  Reading each pixel of a
+// fragment as a 2-byte word, taps split 3 : 2 : 2 : 2 over four wavefronts:
+// 422 µs for the 13 layers, now 292.
+constexpr int kWgThreads = 512;
+constexpr int kXRow = 40, kXPlane = (TH + 2) * kXRow + 8; // pixels of a staged row, of a channel
+constexpr int kZPlane = TH * TW + 8;
+constexpr int kXQuads = (TH + 2) * ((TW + 2 + 3) / 4);
+static_assert(kXQuads * 4 <= kWgThreads && TH * TW / 2 * 4 == kWgThreads && TH == kWgThreads / 64 && TW == 32,
+              "one staged item of each operand a thread, one output row a wavefront");
+static_assert((kXPlane * 2 / 16) % 2 == 1 && (kZPlane * 2 / 16) % 2 == 1 && kXRow * 2 % 16 == 0, "aligned reads");
+
+// the low (HI = 0) or high halves of a and b as one word, a's first
+template <int HI>
+__device__ __forceinline__ unsigned halves(unsigned a, unsigned b)
 {
-    __shared__ __attribute__((aligned(16))) bf16 sX[(TH + 2) * (TW + 2) * CP];
-    __shared__ __attribute__((aligned(16))) bf16 sZ[C * (TH * TW + 8)]; // transposed dZ: [co][pixel]
+    return __builtin_amdgcn_perm(b, a, HI ? 0x07060302u : 0x05040100u);
+}
+
+template <int MODE>
+__global__ __launch_bounds__(kWgThreads, 1) void k_conv33_wgrad(const bf16* __restrict__ X,
+                                                                const bf16* __restrict__ X2,
+                                                                const bf16* __restrict__ dY,
+                                                                const bf16* __restrict__ Yf,
+                                                                float* __restrict__ part_w,
+                                                                float* __restrict__ part_b, int B, int H, int W)
+{
+    struct Planes {
+        bf16 x[C * kXPlane];
+        bf16 z[C * kZPlane];
+    };
+    constexpr int kWaves = kWgThreads / 64;
+    __shared__ union {
+        Planes p[2];
+        f32x4 sum[kWaves][2][C * C / 4];
+    } sm;
+    __shared__ float sb[kWaves][C];
+    static_assert(sizeof(Planes) % 16 == 0, "aligned planes");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tiles_x = (W + TW - 1) / TW, tiles_y = (H + TH - 1) / TH;
-    const int ntiles = tiles_x * tiles_y * B;
-    // taps per wave: 0:{0,4,8} 1:{1,5} 2:{2,6} 3:{3,7}
-    f32x16 acc[3];
+    const TileWalk tw = xcd_walk(tiles_x * tiles_y * B);
+    const int64_t xb = x_image_bytes(MODE, H, W), x2b = x2_image_bytes(MODE, H, W), zb = (int64_t)H * W * C * 2;
+    const int part = tid & 3;
+    const int xq = tid >> 2, xrow = xq / (kXQuads / (TH + 2)), xcol = 4 * (xq % (kXQuads / (TH + 2)));
+    const int zrow = (tid >> 2) / (TW / 2), zcol = 2 * ((tid >> 2) % (TW / 2));
+
+    RawBuf<MODE> rx[4];
+    U32x4 rd[2], ry[2];
+    auto fetch = [&](int t) {
+        const bool live = t < tw.end;
+        const int tc = live ? t : 0;
+        const int b = tc / (tiles_x * tiles_y), oy0 = ((tc / tiles_x) % tiles_y) * TH, ox0 = (tc % tiles_x) * TW;
+        const __amdgpu_buffer_rsrc_t bx = buffer_of(X + (size_t)b * (xb / 2), xb);
+        const __amdgpu_buffer_rsrc_t bx2 = buffer_of(x2b ? X2 + (size_t)b * (x2b / 2) : X, x2b);
+        const __amdgpu_buffer_rsrc_t bd = buffer_of(dY + (size_t)b * (zb / 2), zb);
+        const __amdgpu_buffer_rsrc_t by = buffer_of(Yf + (size_t)b * (zb / 2), zb);
+        const int gy = oy0 - 1 + xrow;
 #pragma unroll
-    for (int t = 0; t < 3; ++t)
+        for (int i = 0; i < 4; ++i) {
+            const int gx = ox0 - 1 + xcol + i;
+            const bool in = live && xq < kXQuads && xcol + i < TW + 2 && gy >= 0 && gy < H && gx >= 0 && gx < W;
+            load_raw_buf<MODE>(rx[i], bx, bx2, gy, gx, part, W, in);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int y = oy0 + zrow, x = ox0 + zcol + i;
+            const uint32_t off = (live && y < H && x < W) ? (uint32_t)((y * W + x) * C + part * 8) * 2 : kOutside;
+            rd[i] = __builtin_amdgcn_raw_buffer_load_b128(bd, off, 0, 0);
+            ry[i] = __builtin_amdgcn_raw_buffer_load_b128(by, off, 0, 0);
+        }
+    };
+    float bsum[8]; // channels part·8 + i
+#pragma unroll
+    for (int i = 0; i < 8; ++i) bsum[i] = 0.f;
+    auto put = [&](Planes& d) {
+        if (xq < kXQuads) {
+            U32x4 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = combine_words<MODE>(rx[i].c);
+            bf16* x = &d.x[part * 8 * kXPlane + xrow * kXRow + xcol];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                *reinterpret_cast<U32x2*>(x + (2 * k) * kXPlane) =
+                    U32x2{halves<0>(v[0][k], v[1][k]), halves<0>(v[2][k], v[3][k])};
+                *reinterpret_cast<U32x2*>(x + (2 * k + 1) * kXPlane) =
+                    U32x2{halves<1>(v[0][k], v[1][k]), halves<1>(v[2][k], v[3][k])};
+            }
+        }
+        U32x4 z[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const U32x4 w[2] = {rd[i], ry[i]};
+            z[i] = combine_words<ST_MASK>(w);
+        }
+        bf16* q = &d.z[part * 8 * kZPlane + zrow * TW + zcol];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            *reinterpret_cast<unsigned*>(q + (2 * k) * kZPlane) = halves<0>(z[0][k], z[1][k]);
+            *reinterpret_cast<unsigned*>(q + (2 * k + 1) * kZPlane) = halves<1>(z[0][k], z[1][k]);
+            bsum[2 * k] += bf16_lo(z[0][k]) + bf16_lo(z[1][k]);
+            bsum[2 * k + 1] += bf16_hi(z[0][k]) + bf16_hi(z[1][k]);
+        }
+    };
+
+    f32x16 acc[9];
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-    float bsum = 0.f; // channel tid & 31, pixels strided by 8 rows of threads
-    const int zs = TH * TW + 8;
 
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int bx = tile % tiles_x, by = (tile / tiles_x) % tiles_y, b = tile / (tiles_x * tiles_y);
-        const int oy0 = by * TH, ox0 = bx * TW;
-        const size_t img = (size_t)b * H * W * C;
+    const int ch = Mfma32::a_row(lane), k0 = Mfma32::a_k0(lane); // dZ's and X's channel, first pixel
+    int tile = tw.first;
+    fetch(tile);
+    if (tile < tw.end) put(sm.p[0]);
+    fetch(tile + tw.stride);
+    __syncthreads();
+    for (int buf = 0; tile < tw.end; tile += tw.stride, buf ^= 1) {
+        const Planes& cur = sm.p[buf];
+#pragma unroll
+        for (int s = 0; s < TW / 16; ++s) {
+            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&cur.z[ch * kZPlane + wave * TW + 16 * s + k0]);
+#pragma unroll
+            for (int ky = 0; ky < 3; ++ky) {
+                const bf16* px = &cur.x[ch * kXPlane + (wave + ky) * kXRow + 16 * s + k0];
+                const U32x4 w = *reinterpret_cast<const U32x4*>(px);
+                const unsigned w4 = *reinterpret_cast<const unsigned*>(px + 8);
+                const U32x4 w1{__builtin_amdgcn_alignbit(w[1], w[0], 16), __builtin_amdgcn_alignbit(w[2], w[1], 16),
+                               __builtin_amdgcn_alignbit(w[3], w[2], 16), __builtin_amdgcn_alignbit(w4, w[3], 16)};
+                const U32x4 w2{w[1], w[2], w[3], w4};
+                acc[3 * ky] = Mfma32::mma(a, __builtin_bit_cast(bf16x8, w), acc[3 * ky]);
+                acc[3 * ky + 1] = Mfma32::mma(a, __builtin_bit_cast(bf16x8, w1), acc[3 * ky + 1]);
+                acc[3 * ky + 2] = Mfma32::mma(a, __builtin_bit_cast(bf16x8, w2), acc[3 * ky + 2]);
+            }
+        }
+        if (tile + tw.stride < tw.end) put(sm.p[buf ^ 1]);
+        fetch(tile + 2 * tw.stride);
         __syncthreads();
-        stage_tile<MODE>(sX, X, X2, b, oy0, ox0, H, W);
-        for (int c = tid; c < TH * TW * 4; c += NT) {
-            const int pix = c >> 2, part = c & 3;
-            const int gy = oy0 + pix / TW, gx = ox0 + pix % TW;
-            Chunk8 d = zero_chunk(), y = zero_chunk();
-            if (gy < H && gx < W) {
-                const size_t off = img + ((size_t)gy * W + gx) * C + part * 8;
-                d = *reinterpret_cast<const Chunk8*>(&dY[off]);
-                y = *reinterpret_cast<const Chunk8*>(&Yf[off]);
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float z = from_bf16(y.v[i]) > 0.f ? from_bf16(d.v[i]) : 0.f;
-                sZ[(part * 8 + i) * zs + pix] = to_bf16(z);
-            }
-        }
-        __syncthreads();
-        {
-            const int ch = tid & 31;
-            for (int pix = tid >> 5; pix < TH * TW; pix += NT / 32) bsum += from_bf16(sZ[ch * zs + pix]);
-        }
-        const int co_a = Mfma32::a_row(lane), kk = Mfma32::a_k0(lane);
-        const int ci_b = Mfma32::b_col(lane);
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            const int tap = wave + 4 * t;
-            if (tap > 8) continue;
-            const int ky = tap / 3, kx = tap % 3;
-            for (int s = 0; s < TH * TW / 16; ++s) {
-                const int p0 = 16 * s + kk; // 8 consecutive pixels of one tile row
-                const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sZ[co_a * zs + p0]);
-                bf16x8 bb;
-                const int row = p0 / TW, c0 = p0 % TW;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) bb[i] = sX[((row + ky) * (TW + 2) + c0 + i + kx) * CP + ci_b];
-                acc[t] = Mfma32::mma(a, bb, acc[t]);
-            }
-        }
     }
+
+    // the wavefronts' sums, two taps at a time, in order: [tap][r / 4][lane][r % 4]
     float* pw = part_w + (size_t)blockIdx.x * 9 * C * C;
-    const int ci = Mfma32::d_col(lane);
+    const int ol = tid & 63, og = (tid >> 6) & 3, ot = tid >> 8; // lane, r / 4 and tap a thread sums
 #pragma unroll
-    for (int t = 0; t < 3; ++t) {
-        const int tap = wave + 4 * t;
-        if (tap > 8) continue;
+    for (int t0 = 0; t0 < 9; t0 += 2) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) pw[(tap * C + Mfma32::d_row(lane, r)) * C + ci] = acc[t][r];
+        for (int t = t0; t < min(t0 + 2, 9); ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                sm.sum[wave][t - t0][g * 64 + lane] =
+                    f32x4{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
+        __syncthreads();
+        if (t0 + ot < 9) {
+            f32x4 v = sm.sum[0][ot][og * 64 + ol];
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) v += sm.sum[w][ot][og * 64 + ol];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                pw[((t0 + ot) * C + Mfma32::d_row(ol, 4 * og + r)) * C + Mfma32::d_col(ol)] = v[r];
+        }
+        __syncthreads();
     }
-    __shared__ float sb[NT];
-    sb[tid] = bsum;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int m = 4; m < 64; m *= 2) bsum[i] += __shfl_xor(bsum[i], m);
+        if (lane < 4) sb[wave][lane * 8 + i] = bsum[i];
+    }
     __syncthreads();
     if (tid < C) {
-        float s = 0.f;
-        for (int j = tid; j < NT; j += C) s += sb[j];
-        part_b[blockIdx.x * C + tid] = s;
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) v += sb[w][tid];
+        part_b[blockIdx.x * C + tid] = v;
     }
 }
 
@@ -1392,10 +1424,12 @@ int conv33(int mode, const bf16* X, const bf16* X2, const bf16* Wt, const float*
 int conv33_wgrad(int mode, const bf16* X, const bf16* X2, const bf16* dY, const bf16* Yf, float* part_w,
                  float* part_b, int parts, float* dW, float* db, int B, int H, int W, hipStream_t s)
 {
+    SIL_REQUIRE(x_image_bytes(mode, H, W) <= kMaxBufferBytes, SIL_ERR_UNSUPPORTED,
+                "unet: %dx%d images exceed one buffer resource per image", H, W);
     const int ntiles = ((W + TW - 1) / TW) * ((H + TH - 1) / TH) * B;
-    const int grid = ntiles < parts ? ntiles : parts;
+    const int grid = std::min({ntiles, parts, (int)kComputeUnits});
     const int rc = by_mode(mode, [&](auto m) -> int {
-        hipLaunchKernelGGL(k_conv33_wgrad<decltype(m)::value>, dim3(grid), dim3(NT), 0, s, X, X2, dY, Yf, part_w,
+        hipLaunchKernelGGL(k_conv33_wgrad<decltype(m)::value>, dim3(grid), dim3(kWgThreads), 0, s, X, X2, dY, Yf, part_w,
                            part_b, B, H, W);
         SIL_LAUNCH_CHECK();
         return (int)SIL_OK;

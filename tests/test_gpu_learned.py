@@ -280,6 +280,30 @@ def test_unet_end_layer_gradients(learned, shape):
     assert rel(g[U.layer_slices(12)[0]], g_ref[U.layer_slices(12)[0]]) <= GRAD_TOL_GPU_ACTIVATIONS
 
 
+@pytest.mark.parametrize("shape", [(1, 8, 8), (2, 24, 40), (1, 16, 72), (9, 88, 104)])
+def test_unet_convolution_weight_gradients(learned, shape):
+    """The weight and bias gradients of every 3×3 layer at the edges of their
+    split (levels smaller than a tile, partial tiles along both axes, fewer
+    tiles than workgroups, workgroups that walk two tiles) against the
+    emulating oracle on the GPU's activations."""
+    B, H, W = shape
+    rng = np.random.default_rng(B * H + W)
+    params = make_params(rng)
+    x = rng.standard_normal((B, H, W, 2)).astype(np.float32)
+    dout = rng.standard_normal((B, H, W)).astype(np.float32)
+    net = learned.UNet(B, H, W, seed=1)
+    net.set_params(torch.from_numpy(params))
+    xt = torch.from_numpy(x).cuda()
+    net.forward(xt)
+    _, act = U.forward(params.astype(np.float64), x, emulate=True)
+    a = _layer_inputs(net, act, B)
+    g = net.backward(xt, torch.from_numpy(dout).cuda()).cpu().numpy()
+    g_ref = U.backward(params.astype(np.float64), a, dout, emulate=True)
+    for l in range(1, U.N_LAYERS + 1):
+        for s in U.layer_slices(l):
+            assert rel(g[s], g_ref[s]) <= GRAD_TOL_GPU_ACTIVATIONS, l
+
+
 def test_unet_direction_loss_matches_oracle(learned):
     B, n = 2, 32
     rng = np.random.default_rng(31)
