@@ -51,7 +51,6 @@ struct Workspace {
     int64_t part_stride = 0;    // slots per partial-sum array
     CgScalars* sc = nullptr;
     CgScalars* host_sc = nullptr; // pinned
-    int apply_blocks = 0;
     bool jacobi_ready = false;
     // SpdIsai: factor G, its transpose, t = G r and z = Gᵀ t
     CsrData isai_g, isai_gt;
@@ -102,24 +101,6 @@ __device__ double reduce_partials(const double* p, int count)
     double v = 0.0;
     for (int i = threadIdx.x; i < count; i += blockDim.x) v += p[i];
     return block_sum(v);
-}
-
-template <typename T>
-__global__ __launch_bounds__(kUpdBlock) void k_dot2(const T* __restrict__ a, const T* __restrict__ b, int64_t n,
-                                                    double* __restrict__ partials)
-{
-    double v = 0.0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        v += (double)a[i] * (double)b[i];
-    __shared__ double sh[kUpdBlock / 64];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int i = 0; i < kUpdBlock / 64; ++i) s += sh[i];
-        partials[blockIdx.x] = s;
-    }
 }
 
 // r = b, x = 0, p_old = 0; partials for <b,b>, <r,z>
@@ -668,15 +649,6 @@ int ensure_workspace(sil_operator op, bool mixed, hipStream_t s)
             return rc;
         w.part_stride = max_dot_blocks();
         SIL_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&w.host_sc), sizeof(CgScalars)));
-        // number of blocks of one operator application
-        int nb = 0;
-        if (op->kind == OP_MAGNETOSTATICS3D || op->kind == OP_MS3D_JACOBIAN)
-            nb = static_cast<int>((op->ms.nx * op->ms.ny * op->ms.nz + 255) / 256);
-        else if (op->kind == OP_POISSON2D)
-            nb = static_cast<int>((op->p2.nx * op->p2.ny + 255) / 256);
-        else if (op->kind == OP_MAGNETOSTATICS2D || op->kind == OP_MS2D_JACOBIAN)
-            nb = static_cast<int>((op->m2.nx * op->m2.ny + 255) / 256);
-        w.apply_blocks = nb;
         (void)s;
     }
     if (!mixed && !w.r) {
