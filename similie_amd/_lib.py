@@ -313,11 +313,19 @@ def check(status):
 
 
 def stream_handle(stream=None):
-    """HIP stream handle of a torch stream (torch's current stream by default)."""
+    """HIP stream handle of a torch stream (torch's current stream by default).
+
+    The default is asked for as a raw handle (0.33 µs): building the Stream
+    object that torch.cuda.current_stream() returns took 2.7 of the 7.5 µs of a
+    staged Laplacian's call on 256² nodes."""
     import torch
 
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return ctypes.c_void_p(stream.cuda_stream)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(raw(torch.cuda.current_device()))
 
 
 def ptr(t):

@@ -167,3 +167,23 @@ def test_marching_laplacian_matches_oracle(extents, degrees, kind):
                 o.fill_(float("nan"))
                 E.laplacian(gg, k, o, t, comp_dim=3)
                 assert close(o, ref), (k, oext, order)
+
+
+def test_default_stream_is_the_current_one():
+    """calls without a stream go to torch's current stream, inside and outside
+    a stream context and under capture"""
+    import similie_amd._lib as L
+
+    def same():
+        return (L.stream_handle().value or 0) == torch.cuda.current_stream().cuda_stream
+
+    assert same()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert same() and L.stream_handle().value == side.cuda_stream
+    graph = torch.cuda.CUDAGraph()
+    t = torch.zeros(4, device="cuda")
+    with torch.cuda.graph(graph):
+        t.add_(1.0)
+        assert same()
+    assert L.stream_handle(side).value == side.cuda_stream
