@@ -119,7 +119,7 @@ __global__ void __launch_bounds__(kPostBlock, 8) k_ms3d_post(PostArgs p)
     const int ht = threadIdx.x, hx_ = ht % kHx, hy_ = ht / kHx;
     const int64_t hi = i0 - 1 + hx_, hj = j0 - 1 + hy_;
     const bool here = ht < kHx * kHy && hi >= 0 && hi < mx && hj >= 0 && hj < my;
-    const int64_t cell = hi + mx * (hj + my * k);
+    const int64_t hcell = hi + mx * (hj + my * k);
     // the cell's values are requested before the barrier that the curve's
     // brackets need: potential at the cell's node and its three neighbours
     // (2D: A_z at the node, e_x, e_y), μ, the material flag
@@ -142,8 +142,8 @@ __global__ void __launch_bounds__(kPostBlock, 8) k_ms3d_post(PostArgs p)
         }
         wx = xc[hi + 1] - xc[hi];
         wy = yc[hj + 1] - yc[hj];
-        iron = p.nonlinear && p.nonlinear[cell] != 0.0;
-        mu = p.mu[cell];
+        iron = p.nonlinear && p.nonlinear[hcell] != 0.0;
+        mu = p.mu[hcell];
     }
     if (p.nonlinear) {
         load_bh_edges(edges, p.curve);
@@ -207,11 +207,11 @@ __global__ void __launch_bounds__(kPostBlock, 8) k_ms3d_post(PostArgs p)
                     }
                 } else {
                     if (p.induction)
-                        for (int m = 0; m < 3; ++m) p.induction[3 * cell + m] = B[m];
+                        for (int m = 0; m < 3; ++m) p.induction[3 * hcell + m] = B[m];
                     if (p.field)
-                        for (int m = 0; m < 3; ++m) p.field[3 * cell + m] = H[m];
+                        for (int m = 0; m < 3; ++m) p.field[3 * hcell + m] = H[m];
                     if (p.stress)
-                        for (int m = 0; m < 6; ++m) p.stress[6 * cell + m] = T[m];
+                        for (int m = 0; m < 6; ++m) p.stress[6 * hcell + m] = T[m];
                 }
             }
         }
@@ -277,7 +277,7 @@ __global__ void __launch_bounds__(kPostBlock, 8) k_ms3d_post(PostArgs p)
             if constexpr (STAGED)
                 fo[f] = c2 * -acc;
             else
-                p.force[3 * cell + f] = c2 * -acc;
+                p.force[3 * (i + mx * (j + my * k)) + f] = c2 * -acc;
         }
     }
     if constexpr (STAGED) {

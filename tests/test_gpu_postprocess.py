@@ -1,6 +1,9 @@
 """Cell post-processing on the GPU (B, H, Maxwell stress, xy-slice force
 density) against the oracle, through the C ABI."""
 import json
+import os
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -140,3 +143,48 @@ def test_solve_then_post_process():
     # the core carries the flux: |B| there well above the air's
     B = out.magnetic_induction.cpu().numpy()
     assert np.median(np.linalg.norm(B[tags == 2], axis=1)) > 10 * np.median(np.linalg.norm(B[tags == 1], axis=1))
+
+
+def check_every_cell_between_guards():
+    """3D and 2D operators on ragged tiles: every cell of the four outputs
+    against the oracle, nothing stored before or after them"""
+    import similie_amd._lib as L
+    import similie_amd.solvers as S
+
+    pad = 4096
+    for shape, nonlinear in (((70, 21, 5), True), ((65, 9, 3), False), ((64, 8), True), ((131, 18), False), ((2, 2), True)):
+        print(f"guarded post_process shape={shape} nonlinear={nonlinear}", flush=True)
+        rng = np.random.default_rng(sum(shape))
+        coords = axes(shape, rng)
+        n, nodes = int(np.prod([s - 1 for s in shape])), int(np.prod(shape))
+        pot = rng.standard_normal(nodes * (3 if len(shape) == 3 else 1)) * 0.7
+        mu = rng.uniform(1.0, 4.0, n) * MU0
+        nl = (rng.random(n) < 0.5).astype(float) if nonlinear else None
+        curve = (CURVE["b"], CURVE["h"]) if nonlinear else (None, None)
+        if len(shape) == 3:
+            op = operator(coords, nonlinear)
+            call, ref = L.lib().sil_magnetostatics3d_post_process, orc.ms_post_process(coords, pot, mu, nl, *curve)
+        else:
+            mu_n = torch.full((nodes,), MU0, dtype=torch.float64, device="cuda")
+            op = (S.NonlinearMagnetostaticsOperator2D(*coords, mu_n, torch.ones_like(mu_n), *curve) if nonlinear
+                  else S.MagnetostaticsOperator2D(*coords, mu_n))
+            call, ref = L.lib().sil_magnetostatics2d_post_process, orc.ms2d_post_process(coords, pot, mu, nl, *curve)
+        held = [dev(pot), dev(mu)] + ([dev(nl)] if nonlinear else [])
+        buf = [torch.full((w * n + 2 * pad,), -7.5, dtype=torch.float64, device="cuda") for w in (3, 3, 6, 3)]
+        L.check(call(op.handle, L.ptr(held[0]), L.ptr(held[1]), L.ptr(held[2]) if nonlinear else None,
+                     *[L.ptr(b[pad:]) for b in buf], None))
+        torch.cuda.synchronize()
+        for name, b, r in zip(NAMES, buf, ref):
+            assert torch.all(b[:pad] == -7.5) and torch.all(b[-pad:] == -7.5), name
+            check(b[pad:-pad].reshape(r.shape), r, name)
+
+
+@pytest.mark.parametrize("staged", ["1", "0"])
+def test_both_store_variants_write_their_own_cells_only(staged):
+    """SIL_POST_STAGED is read once per process: each variant in a process of
+    its own"""
+    child = subprocess.run([sys.executable, "-c", "import conftest, test_gpu_postprocess as t; "
+                            "t.check_every_cell_between_guards(); print('checked')"],
+                           cwd=Path(__file__).parent, env={**os.environ, "SIL_POST_STAGED": staged},
+                           capture_output=True, text=True, timeout=100)
+    assert child.returncode == 0 and "checked" in child.stdout, child.stdout + child.stderr
