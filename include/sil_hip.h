@@ -270,12 +270,14 @@ int sil_magnetostatics2d_air_gap_diagnostics(sil_operator op, const double* cell
                                              void* stream);
 
 /* apply_jacobian (magnetostatics_onelab.hpp:2918-3113): out = J(state)·in,
- * the derivative of the nonlinear operator at the potential `state`. */
+ * the derivative of the nonlinear operator at the potential `state`; out may
+ * overlap state, not in. */
 int sil_magnetostatics3d_apply_jacobian(sil_operator op, const double* state, const double* in, double* out,
                                         void* stream);
 
 /* the diagonal of J(state) (the Jacobi preconditioner of each Newton step,
- * which the reference takes from the assembled Jacobian, :1434-1438) */
+ * which the reference takes from the assembled Jacobian, :1434-1438); diag may
+ * overlap state */
 int sil_magnetostatics3d_jacobian_diagonal(sil_operator op, const double* state, double* diag, void* stream);
 
 /* Nodal permeability = mean over adjacent cells (magnetostatics_onelab.hpp

@@ -1,5 +1,6 @@
 // extern "C" entry points of the linear operators and the CG solve.
 #include <cmath>
+#include <cstdint>
 #include <cstdlib>
 #include <new>
 #include <vector>
@@ -42,6 +43,13 @@ double local_spacing(const double* c, int64_t n, int64_t i)
     if (i == 0) return c[1] - c[0];
     if (i + 1 == n) return c[n - 1] - c[n - 2];
     return 0.5 * (c[i + 1] - c[i - 1]);
+}
+
+// whether two vectors of n values share memory
+bool overlap(const double* a, const double* b, int64_t n)
+{
+    const auto pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return (pa < pb ? pb - pa : pa - pb) < sizeof(double) * static_cast<uint64_t>(n);
 }
 
 void free_operator(sil_operator op)
@@ -303,7 +311,10 @@ int sil_magnetostatics3d_apply_jacobian(sil_operator op, const double* state, co
     SIL_REQUIRE(op && state && in && out, SIL_ERR_INVALID, "magnetostatics3d_apply_jacobian: null argument");
     SIL_REQUIRE(op->kind == OP_MS3D_NONLINEAR, SIL_ERR_INVALID, "apply_jacobian: not a nonlinear operator");
     hipStream_t s = as_stream(stream);
-    if (ms3d_material_march_ok(op->ms)) return ms3d_material_jacobian64(op->ms, op->nl, state, in, out, s);
+    // the march reads the state at neighbouring nodes while it writes: a result
+    // that takes the state's place needs the material stored first
+    if (ms3d_material_march_ok(op->ms) && !overlap(state, out, op->n))
+        return ms3d_material_jacobian64(op->ms, op->nl, state, in, out, s);
     int rc = ms3d_state(op->ms, op->nl, state, s);
     if (rc) return rc;
     return ms3d_jacobian_apply64(op->ms, op->nl, in, out, DotEpilogue{nullptr}, nullptr, nullptr, s);
@@ -313,7 +324,12 @@ int sil_magnetostatics3d_jacobian_diagonal(sil_operator op, const double* state,
 {
     SIL_REQUIRE(op && state && diag, SIL_ERR_INVALID, "magnetostatics3d_jacobian_diagonal: null argument");
     SIL_REQUIRE(op->kind == OP_MS3D_NONLINEAR, SIL_ERR_INVALID, "jacobian_diagonal: not a nonlinear operator");
-    return ms3d_material_diagonal(op->ms, op->nl, state, diag, as_stream(stream));
+    hipStream_t s = as_stream(stream);
+    if (!overlap(state, diag, op->n)) return ms3d_material_diagonal(op->ms, op->nl, state, diag, s);
+    // in the state's place: the material stored first, as above
+    int rc = ms3d_state(op->ms, op->nl, state, s);
+    if (rc) return rc;
+    return ms3d_jacobian_diagonal(op->ms, op->nl, diag, s);
 }
 
 int sil_magnetostatics3d_post_process(sil_operator op, const double* potential, const double* cell_mu,

@@ -238,3 +238,27 @@ def test_terms_at_one_state_match_the_oracle(S, shape, samples):
     assert rel(op.apply(xt).cpu().numpy(), ref.apply(x)) <= 1e-12
     assert rel(op.apply_jacobian(xt, vt).cpu().numpy(), ref.jacobian_apply(x, v)) <= 1e-12
     assert rel(op.jacobian_diagonal(xt).cpu().numpy(), ref.jacobian_diagonal(x)) <= 1e-12
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3), (65, 13, 9), (40, 33, 21)])
+def test_results_may_take_the_states_place(S, shape):
+    """J(state)·v and diag J(state) written over the state itself, or over a
+    part of it"""
+    import similie_amd._lib as L
+
+    op, ref, rng = make(S, shape, sum(shape))
+    n = op.size()
+    x, v = 0.5 * rng.standard_normal(n), rng.standard_normal(n)
+    jv, diag = ref.jacobian_apply(x, v), ref.jacobian_diagonal(x)
+    vt = cuda(v)
+    for shift in (0, 3, -3):  # the result starts where the state does, 3 values behind or before it
+        for name, want in (("apply_jacobian", jv), ("jacobian_diagonal", diag)):
+            buf = torch.zeros(n + 6, dtype=torch.float64, device="cuda")
+            state, out = buf[3:3 + n], buf[3 + shift:3 + shift + n]
+            state.copy_(cuda(x))
+            if name == "apply_jacobian":
+                op.apply_jacobian(state, vt, out=out)
+            else:
+                L.check(L.lib().sil_magnetostatics3d_jacobian_diagonal(op.handle, L.ptr(state), L.ptr(out), None))
+                torch.cuda.synchronize()
+            assert rel(out.cpu().numpy(), want) <= 1e-12, (name, shift)
