@@ -8,11 +8,11 @@
 
 namespace sil {
 
-// The curve in LDS with its brackets laid out for a branch-free search:
-// edge[m] = q[m + 1] for the inner samples, +∞ from there on, so the bracket
-// of q is the number of edges below it.  (A search that stops at the bracket
-// is a chain of dependent reads, twice per node, and cost the curl-curl march
-// more than its memory: 83 µs for F on 113 × 97 × 129 nodes, 34 with the count.)
+// The curve in LDS with its brackets laid out for a branch-free search: the
+// bracket of q is the number of edges below it.  (A search that stops at the
+// bracket is a chain of dependent reads, twice per node, and cost the curl-curl
+// march more than its memory: 83 µs for F on 113 × 97 × 129 nodes, 34 with the
+// count.)
 struct BhEdges {
     alignas(16) double edge[kBhMax];
     int n;
@@ -25,26 +25,24 @@ struct BhTable : BhEdges {
 // by every thread of the workgroup; the caller's barrier follows
 __device__ __forceinline__ void load_bh_edges(BhEdges& t, const BhCurve* __restrict__ c)
 {
-    const int n = c->n;
-    for (int i = threadIdx.x; i < kBhMax; i += blockDim.x) t.edge[i] = i + 2 < n ? c->q[i + 1] : __builtin_inf();
-    if (threadIdx.x == 0) t.n = n;
+    for (int i = threadIdx.x; i < kBhMax; i += blockDim.x) t.edge[i] = c->edge[i];
+    if (threadIdx.x == 0) t.n = c->n;
 }
 
 __device__ __forceinline__ void load_bh_table(BhTable& t, const BhCurve* __restrict__ c)
 {
-    const int n = c->n;
     for (int i = threadIdx.x; i < kBhMax; i += blockDim.x) {
-        // (entries past the last sample are never read)
-        const double q = c->q[i + 1 < kBhMax ? i + 1 : i], b = c->b[i], h = c->h[i], dh = c->dh_db[i];
-        t.edge[i] = i + 2 < n ? q : __builtin_inf();
+        // (b, h and dh_db past the last sample are never read)
+        const double e = c->edge[i], b = c->b[i], h = c->h[i], dh = c->dh_db[i];
+        t.edge[i] = e;
         t.b[i] = b;
         t.h[i] = h;
         t.dh_db[i] = dh;
     }
-    if (threadIdx.x == 0) t.n = n;
+    if (threadIdx.x == 0) t.n = c->n;
 }
 
-// the bracket of q = b²: the number of inner samples below it
+// the bracket of q = b²
 __device__ __forceinline__ int bh_bracket(const BhEdges& t, double q)
 {
     typedef double D2 __attribute__((ext_vector_type(2)));
@@ -75,8 +73,9 @@ __device__ __forceinline__ double bh_h(const Curve& t, int i, double b)
 // (f′ = (h′ b − h)/(2 b³), f″ by one more derivative: h″ = 0 on a segment).
 __device__ __forceinline__ void bh_response(const BhTable& t, double q, double& a, double& c)
 {
-    const int i = bh_bracket(t, q);
-    const double b = sqrt(q), dh = t.dh_db[i], h = bh_h(t, i, b);
+    const double b = sqrt(q);
+    const int i = bh_bracket(t, b * b);
+    const double dh = t.dh_db[i], h = bh_h(t, i, b);
     const bool zero = q == 0.0;
     const double f = zero ? dh : h / b;
     a = 0.5 * (f + dh);

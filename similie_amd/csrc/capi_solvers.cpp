@@ -133,7 +133,18 @@ int attach_material(sil_operator op, int64_t nn, const double* ferromagnetic_nod
     for (int i = 0; i < nsamples; ++i) {
         c.b[i] = bh_b[i];
         c.h[i] = bh_h[i];
-        c.q[i] = bh_b[i] * bh_b[i];
+    }
+    // The bracket of b ≥ 0 is the last segment where b reaches the last sample,
+    // else the first segment i with b² ≤ q[0] or b² ≤ q[i + 1], q[i] = b[i]²
+    // (nonlinear_magnetostatics.py:14-181): the number of edges below b², an
+    // edge being the greatest q up to its sample (q falls where samples are
+    // negative), kept below the last sample's where b can reach that.
+    const double last = bh_b[nsamples - 1];
+    const double cap = last > 0.0 ? std::nextafter(last * last, 0.0) : -INFINITY;
+    double greatest = bh_b[0] * bh_b[0];
+    for (int i = 0; i < kBhMax; ++i) {
+        if (i + 2 < nsamples) greatest = std::fmax(greatest, bh_b[i + 1] * bh_b[i + 1]);
+        c.edge[i] = i + 2 < nsamples ? std::fmin(greatest, cap) : INFINITY;
     }
     for (int i = 0; i + 1 < nsamples; ++i) c.dh_db[i] = (c.h[i + 1] - c.h[i]) / (c.b[i + 1] - c.b[i]);
     BhCurve* dc = nullptr;

@@ -44,7 +44,8 @@ struct Ms3dData {
 constexpr int kBhMax = 64;
 struct BhCurve {
     int n;
-    double b[kBhMax], h[kBhMax], q[kBhMax], dh_db[kBhMax];
+    double b[kBhMax], h[kBhMax], dh_db[kBhMax];
+    double edge[kBhMax]; // of the brackets (bh_curve.hpp)
 };
 
 // a node's material state as one aligned record: a, c and the first two

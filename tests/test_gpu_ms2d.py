@@ -325,3 +325,27 @@ def test_newton_with_spd_isai_matches_the_oracle():
     assert rel(x, xr) <= 1e-7
     r = b.cpu().numpy() - ref.apply(x.cpu().numpy())
     assert np.linalg.norm(r) <= 1.0001e-10 * np.linalg.norm(b.cpu().numpy())
+
+
+@pytest.mark.parametrize("curve", [([-2.0, -1.0, 0.0, 1.0, 2.0], [-1000.0, -100.0, 0.0, 100.0, 1000.0]),
+                                   ([-3.0, -0.5, 0.25, 1.5], [-700.0, -90.0, 40.0, 900.0]),
+                                   ([-4.0, -2.0, -0.5], [-4000.0, -1500.0, -150.0])])
+def test_curve_with_negative_samples(curve):
+    """the bracket where b² does not increase over the samples"""
+    import similie_amd.solvers as S
+
+    rng = np.random.default_rng(11)
+    shape = (33, 21)
+    coords, ferro, mu, x = nonlinear_case(shape, rng, 0.8)
+    v = rng.standard_normal(x.size)
+    op = S.NonlinearMagnetostaticsOperator2D(*coords, dev(mu), dev(ferro), *curve)
+    ref = orc.Magnetostatics2D(shape, mu, ferro, *[np.array(c) for c in curve])
+    x_d, v_d = dev(x), dev(v)
+    assert rel(op.apply(x_d), ref.apply(x)) <= 1e-12
+    assert rel(op.apply_jacobian(x_d, v_d), ref.apply(v, x)) <= 1e-12
+    assert rel(op.jacobian_diagonal(x_d), ref.diagonal(x)) <= 1e-12
+    cells = 32 * 20
+    out = op.post_process(x_d, dev(np.full(cells, MU0)), dev(np.ones(cells)))
+    torch.cuda.synchronize()
+    for got, r in zip(out, orc.ms2d_post_process(coords, x, np.full(cells, MU0), np.ones(cells), *curve)):
+        assert rel(got, r) <= 1e-12

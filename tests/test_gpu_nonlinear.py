@@ -262,3 +262,38 @@ def test_results_may_take_the_states_place(S, shape):
                 L.check(L.lib().sil_magnetostatics3d_jacobian_diagonal(op.handle, L.ptr(state), L.ptr(out), None))
                 torch.cuda.synchronize()
             assert rel(out.cpu().numpy(), want) <= 1e-12, (name, shift)
+
+
+# curves whose b² does not increase: the bracket is the first segment that b²
+# does not pass, the last one from the last sample on
+NEGATIVE_CURVES = {
+    "odd": ([-2.0, -1.0, 0.0, 1.0, 2.0], [-1000.0, -100.0, 0.0, 100.0, 1000.0]),
+    "below_the_first_sample": ([-3.0, -0.5, 0.25, 0.75, 1.5], [-700.0, -90.0, 40.0, 200.0, 900.0]),
+    "ends_at_zero": ([-2.0, -1.5, -0.25, 0.0], [-900.0, -400.0, -30.0, 0.0]),
+    "negative_only": ([-4.0, -2.0, -1.0, -0.5], [-4000.0, -1500.0, -400.0, -150.0]),
+    "long": (np.linspace(-1.0, 2.5, 64), np.linspace(-1.0, 2.5, 64) ** 3 * 500.0 + np.linspace(-1.0, 2.5, 64) * 80.0),
+}
+
+
+@pytest.mark.parametrize("name", list(NEGATIVE_CURVES))
+def test_curves_with_negative_samples(S, name):
+    """F, J·v, diag J, the assembled Jacobian (from the stored state) and the
+    cells' field"""
+    bh = [np.array(a) for a in NEGATIVE_CURVES[name]]
+    op, ref, rng = make(S, (17, 9, 12), 5, bh=bh, penalty=50.0, ferro_share=0.7)
+    n = op.size()
+    x = rng.standard_normal((n // 3, 3)) * np.repeat(rng.choice([0.02, 0.3, 2.0], n // 3), 3).reshape(-1, 3)
+    x, v = x.reshape(-1), rng.standard_normal(n)
+    xt, vt = cuda(x), cuda(v)
+    assert rel(op.apply(xt).cpu().numpy(), ref.apply(x)) <= 1e-12
+    jv = ref.jacobian_apply(x, v)
+    assert rel(op.apply_jacobian(xt, vt).cpu().numpy(), jv) <= 1e-12
+    assert rel(op.jacobian_diagonal(xt).cpu().numpy(), ref.jacobian_diagonal(x)) <= 1e-12
+    assert rel(op.assemble_jacobian(xt).apply(vt).cpu().numpy(), jv) <= 1e-12
+    coords = [np.cumsum(rng.uniform(0.5, 1.5, s)) for s in (17, 9, 12)]
+    op = S.NonlinearMagnetostaticsOperator3D(*coords, cuda(np.full(n // 3, MU0)), cuda(np.ones(n // 3)), *bh)
+    cells = 16 * 8 * 11
+    out = op.post_process(xt, cuda(np.full(cells, MU0)), cuda(np.ones(cells)))
+    want = orc.ms_post_process(coords, x, np.full(cells, MU0), np.ones(cells), *bh)
+    for got, r in zip(out, want):
+        assert rel(got.cpu().numpy(), r) <= 1e-12
