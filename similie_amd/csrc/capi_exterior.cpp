@@ -150,7 +150,7 @@ int sil_grid_create(sil_grid* out, int32_t ndim, const int64_t* extent, const do
     g->geom.nodal = nodal_positions;
     for (int a = 0; a < ndim; ++a) g->geom.ext[a] = extent[a];
     if (axis_coords) {
-        double least[SIL_MAX_DIM];
+        double least[SIL_MAX_DIM], greatest = 1.0;
         g->geom.regular = true;
         for (int a = 0; a < ndim; ++a) {
             const int64_t n = extent[a];
@@ -160,42 +160,42 @@ int sil_grid_create(sil_grid* out, int32_t ndim, const int64_t* extent, const do
                 set_error("grid_create: null coordinate array for axis %d", a);
                 return SIL_ERR_INVALID;
             }
-            // per-node edge length: forward, backward at the last node, 0 on
-            // one node; its reciprocal behind it
-            double* h = static_cast<double*>(std::malloc(sizeof(double) * 2 * n));
+            // per-node edge length: forward, backward at the last node, 0 on one node
+            double* h = static_cast<double*>(std::malloc(sizeof(double) * n));
             if (h == nullptr) {
                 sil_grid_destroy(g);
                 set_error("grid_create: out of host memory");
                 return SIL_ERR_INVALID;
             }
             least[a] = INFINITY;
+            double most = 1.0;
             for (int64_t i = 0; i < n; ++i) {
                 h[i] = (i + 1 < n) ? c[i + 1] - c[i] : (i > 0 ? c[i] - c[i - 1] : 0.0);
-                h[n + i] = 1.0 / h[i];
                 least[a] = std::fmin(least[a], std::fabs(h[i]));
-                // a NaN or infinite edge, or one whose reciprocal is, is not regular
-                if (!std::isfinite(h[i]) || !std::isfinite(h[n + i])) g->geom.regular = false;
+                most = std::fmax(most, std::fabs(h[i]));
+                if (!std::isfinite(h[i])) g->geom.regular = false;
             }
+            greatest *= most;
             hipError_t e1 = hipMalloc(&g->axis_storage[a], sizeof(double) * n);
-            hipError_t e2 = hipMalloc(&g->spacing[a], sizeof(double) * 2 * n);
+            hipError_t e2 = hipMalloc(&g->spacing[a], sizeof(double) * n);
             hipError_t e3 = e1 == hipSuccess ? hipMemcpy(g->axis_storage[a], c, sizeof(double) * n, hipMemcpyHostToDevice)
                                              : e1;
-            hipError_t e4 =
-                e2 == hipSuccess ? hipMemcpy(g->spacing[a], h, sizeof(double) * 2 * n, hipMemcpyHostToDevice) : e2;
+            hipError_t e4 = e2 == hipSuccess ? hipMemcpy(g->spacing[a], h, sizeof(double) * n, hipMemcpyHostToDevice)
+                                             : e2;
             std::free(h);
             if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess || e4 != hipSuccess) {
                 sil_grid_destroy(g);
                 set_error("grid_create: device allocation or copy failed");
                 return SIL_ERR_HIP;
             }
-            g->inv_spacing[a] = g->spacing[a] + n;
             g->geom.axis[a] = g->axis_storage[a];
             g->geom.spacing[a] = g->spacing[a];
-            g->geom.inv_spacing[a] = g->inv_spacing[a];
         }
         // a node is degenerate for degree k where the edge product of some
         // k axes is below 1e-14 (geometry.hpp): the least product of every
-        // axis set decides for the whole grid
+        // axis set decides for the whole grid.  Products up to 1e100 leave the
+        // kernels' reciprocals of volumes far from the ends of the range.
+        if (!(greatest <= 1e100)) g->geom.regular = false;
         for (unsigned m = 1; m < (1u << ndim); ++m) {
             double p = 1.0;
             for (int a = 0; a < ndim; ++a)

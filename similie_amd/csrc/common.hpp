@@ -162,11 +162,10 @@ struct DevGeom {
     int64_t ext[SIL_MAX_DIM];
     const double* axis[SIL_MAX_DIM]; // device coordinates (rectilinear)
     const double* nodal;             // device [node][ndim] (general)
-    // rectilinear: edge length per node (forward, backward at the last node)
-    // and its reciprocal, device; regular: finite and far enough from zero
-    // that no node is degenerate for any degree
+    // rectilinear: edge length per node (forward, backward at the last node),
+    // device; regular: far enough from zero that no node is degenerate for any
+    // degree, and from infinity for products of them
     const double* spacing[SIL_MAX_DIM];
-    const double* inv_spacing[SIL_MAX_DIM];
     bool regular;
     int metric_kind;
     const double* metric;
@@ -178,5 +177,4 @@ struct sil_grid_s {
     sil::DevGeom geom;
     double* axis_storage[SIL_MAX_DIM]; // device copies of the axis coordinates
     double* spacing[SIL_MAX_DIM];      // device per-node edge lengths (rectilinear)
-    double* inv_spacing[SIL_MAX_DIM];  // device reciprocals of spacing (one allocation with it)
 };

@@ -8,16 +8,15 @@
 // is derived again, with its square roots and divisions, for each
 // coefficient read from it: 2.76 ms for Δ of a 2-form on 107 × 75 × 93 nodes,
 // where the inputs and outputs take 11 µs to stream.  Here one thread per
-// node reads the star of each node it touches once, as s_a and 1/s_a per
-// axis (s_a = √|g_aa|·|h_a|, 1/h_a from the grid), every coefficient is a
-// product of N of them, and all axis sets are template constants.  The
-// neighbours' values come through the caches: consecutive threads hold
-// consecutive nodes of the last axis.  Diagonal metric, general kernel → here:
-//   Δ of a 2-form, 107 × 75 × 93 nodes     2753 → 21 µs
-//   Δ of a 2-form, 256³ nodes              353 µs (1.8 TB/s)
-//   δ of a 2-form, 129 × 120 × 135 nodes   1633 → 54 µs (2.8 TB/s)
-//   Δ of a 1-form, 2048 × 1999 nodes       3742 → 83 µs
-//   ⋆ of a 1-form, 256³ nodes              1931 → 251 µs (4.8 TB/s, a copy's rate)
+// node forms the star of each node it touches once (star_of_edges), and
+// all axis sets are template constants.  The neighbours' values come through the
+// caches: consecutive threads hold consecutive nodes of the last axis.  Diagonal
+// metric, general kernel → here:
+//   Δ of a 2-form, 107 × 75 × 93 nodes     2753 → 19 µs
+//   Δ of a 2-form, 256³ nodes              327 µs (3.7 TB/s)
+//   δ of a 2-form, 129 × 120 × 135 nodes   1633 → 41 µs (3.7 TB/s)
+//   Δ of a 1-form, 2048 × 1999 nodes       3742 → 79 µs
+//   ⋆ of a 1-form, 256³ nodes              1931 → 235 µs (5.1 TB/s, a copy's rate)
 //   d of a 1-form, 256³ nodes              1141 → 248 µs
 // δ, ⋆ and d are bound by memory, Δ on 3D grids by the steps of its march
 // (k_rect_lap3_march), elsewhere by the FP64 work of a node's stars.
@@ -65,80 +64,156 @@ struct RectView {
 template <int N>
 struct RectGeom {
     const double* __restrict__ h[N]; // spacing per node
-    const double* __restrict__ r[N]; // 1 / spacing
     const double* __restrict__ g;    // [node][N], null for the identity
     uint32_t ext[N];
     int64_t node[N]; // node strides of g
 };
 
+// The ⋆ coefficient of each source axis set, sign left out: Π_tgt s / Π_src s,
+// s_a = √|g_aa|·|h_a|
 template <int N>
 struct Star {
-    double s[N], r[N]; // s_a and 1/s_a
+    double c[1 << N];
 };
 
-// s = √v |h| and r = 1/s = |1/h|/√v, v = |g|: the hardware estimate of 1/√v
-// refined by two Newton–Raphson steps, then √v corrected by its residual
-// v − q² and 1/s by 1 − s r, each to about half an ulp (without the
-// corrections the operators are twice as far from FP64's exact results).
-// v = 0, the reference's singular metric, leaves both at 0; v = ∞ gives ∞
-// and 0.
-__device__ __forceinline__ void axis_star(double g, double h, double rh, double& s, double& r)
+// n / d, y ≈ 1/d: one rounding where a product with a rounded 1/d has two
+__device__ __forceinline__ double quotient(double n, double d, double y)
 {
-    const double v = fabs(g);
-    double y = __builtin_amdgcn_rsq(v);
-    const double hv = 0.5 * v;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) y = fma(y, fma(-(hv * y), y, 0.5), y);
-    double q = v * y;
-    q = fma(fma(-q, q, v), 0.5 * y, q);
-    const bool end = v == 0.0 || v == __builtin_inf();
-    y = end ? 0.0 : y;
-    q = end ? v : q;
-    s = q * fabs(h);
-    r = y * fabs(rh);
-    const double e = fma(-s, r, 1.0);
-    r = end ? r : fma(e, r, r);
+    const double q = n * y;
+    return fma(fma(-d, q, n), y, q);
 }
 
-template <int N, bool DIAG>
-__device__ __forceinline__ Star<N> load_star(const RectGeom<N>& g, const uint32_t (&idx)[N])
+// the hardware's estimate of 1/d (2⁻²⁴) after a Newton–Raphson step: a first
+// guess for quotient
+__device__ __forceinline__ double guess_reciprocal(double d)
+{
+    const double y = __builtin_amdgcn_rcp(d);
+    return fma(y, fma(-d, y, 1.0), y);
+}
+
+// √v to half an ulp: the hardware's estimate of 1/√v (2⁻²⁴), one of Goldschmidt's
+// steps and a correction by the residual v − g²
+__device__ __forceinline__ double root(double v)
+{
+    const double y = __builtin_amdgcn_rsq(v);
+    double g = v * y, h = 0.5 * y;
+    const double r = fma(-g, h, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    return fma(fma(-g, g, v), h, g);
+}
+
+// the star of the edge measures s (in the plain range, see diag_star): the
+// quotients of products that the general kernels form, with 1/V, V = Π s, as the
+// first guess of every quotient's reciprocal (1/d = n/V).  Products of s and of
+// rounded 1/s, which stood here before, round once more per source axis: rms of
+// a coefficient, N = 3, k = 1 to 3, identity metric 8.2, 9.4, 10.5 · 1e-17, now
+// 6.7, 6.7, 8.2 as in the general kernels.
+template <int N>
+__device__ __forceinline__ Star<N> star_of_edges(const double (&s)[N])
 {
     Star<N> o;
+    double V = 1.0;
+#pragma unroll
+    for (int a = 0; a < N; ++a) V *= s[a];
+    const double y = guess_reciprocal(V);
+    static_for<1 << N>([&](auto SRC) {
+        constexpr unsigned src = decltype(SRC)::value;
+        double num = 1.0, den = 1.0;
+#pragma unroll
+        for (int a = 0; a < N; ++a) ((src >> a) & 1u ? den : num) *= s[a];
+        o.c[src] = src == 0 ? V : quotient(num, den, num * y);
+    });
+    return o;
+}
+
+// diagonal metric.  Where some √|g_aa|·|h_a| leaves 1e±45 (zero, infinite and NaN
+// metrics among them; plain turns false) the node is worked out again with EXACT,
+// with divisions: behind the node's other work, so that no branch keeps its loads
+// from being in flight together.
+template <int N, bool EXACT>
+__device__ __forceinline__ Star<N> diag_star(const double (&m)[N], const double (&h)[N], bool& plain)
+{
+    double s[N];
+    if constexpr (EXACT) {
+        Star<N> o;
+        bool ok = true; // a zero entry makes the whole metric singular
+#pragma unroll
+        for (int a = 0; a < N; ++a) {
+            s[a] = sqrt(fabs(m[a])) * fabs(h[a]);
+            ok = ok && m[a] != 0.0;
+        }
+        static_for<1 << N>([&](auto SRC) {
+            constexpr unsigned src = decltype(SRC)::value;
+            double num = 1.0, den = 1.0;
+#pragma unroll
+            for (int a = 0; a < N; ++a) ((src >> a) & 1u ? den : num) *= s[a];
+            o.c[src] = ok && den != 0.0 ? num / den : 0.0;
+        });
+        return o;
+    } else {
+#pragma unroll
+        for (int a = 0; a < N; ++a) {
+            s[a] = root(fabs(m[a])) * fabs(h[a]);
+            plain = plain && s[a] > 1e-45 && s[a] < 1e45;
+        }
+        return star_of_edges<N>(s);
+    }
+}
+
+template <int N, bool DIAG, bool EXACT>
+__device__ __forceinline__ Star<N> load_star(const RectGeom<N>& g, const uint32_t (&idx)[N], bool& plain)
+{
+    double h[N];
+#pragma unroll
+    for (int a = 0; a < N; ++a) h[a] = g.h[a][idx[a]];
     if constexpr (DIAG) {
         int64_t lin = 0;
 #pragma unroll
         for (int a = 0; a < N; ++a) lin += (int64_t)idx[a] * g.node[a];
         double m[N];
-        bool ok = true;
 #pragma unroll
-        for (int a = 0; a < N; ++a) {
-            m[a] = g.g[lin * N + a];
-            ok = ok && m[a] != 0.0;
-        }
-#pragma unroll
-        for (int a = 0; a < N; ++a) {
-            // a zero entry makes the whole metric singular
-            axis_star(ok ? m[a] : 0.0, g.h[a][idx[a]], g.r[a][idx[a]], o.s[a], o.r[a]);
-        }
+        for (int a = 0; a < N; ++a) m[a] = g.g[lin * N + a];
+        return diag_star<N, EXACT>(m, h, plain);
     } else {
 #pragma unroll
-        for (int a = 0; a < N; ++a) {
-            o.s[a] = fabs(g.h[a][idx[a]]);
-            o.r[a] = fabs(g.r[a][idx[a]]);
-        }
+        for (int a = 0; a < N; ++a) h[a] = fabs(h[a]);
+        return star_of_edges<N>(h);
     }
-    return o;
 }
+
+// identity metric on the nodes of one column along x: what y and z give is
+// formed once, a plane costs 10 to 17 operations (star_of_edges 20 to 40: Δ of a
+// 3-form, 256³ nodes, 73 against 80 µs)
+struct IdentColumn {
+    double P, iP, zy, yz; // h_y h_z, its reciprocal, h_z / h_y, h_y / h_z
+
+    __device__ __forceinline__ IdentColumn(double hy, double hz)
+    {
+        hy = fabs(hy);
+        hz = fabs(hz);
+        P = hy * hz;
+        const double y = guess_reciprocal(P);
+        iP = quotient(1.0, P, y);
+        zy = quotient(hz, hy, hz * y);
+        yz = quotient(hy, hz, hy * y);
+    }
+
+    __device__ __forceinline__ Star<3> at(double hx) const
+    {
+        hx = fabs(hx);
+        const double rx = guess_reciprocal(hx);
+        return {{hx * P, quotient(P, hx, rx), hx * zy, quotient(zy, hx, rx), hx * yz, quotient(yz, hx, rx),
+                 quotient(hx, P, iP), quotient(iP, hx, rx)}};
+    }
+};
 
 // ⋆ from the axes SRC onto their complement: sign · Π_tgt s / Π_src s
 template <int N, unsigned SRC>
 __device__ __forceinline__ double star_coef(const Star<N>& o)
 {
     constexpr int sign = concat_sign(SRC, ((1u << N) - 1u) & ~SRC, N);
-    double v = (SRC & 1u) ? o.r[0] : o.s[0];
-    if constexpr (N > 1) v *= (SRC & 2u) ? o.r[1] : o.s[1];
-    if constexpr (N > 2) v *= (SRC & 4u) ? o.r[2] : o.s[2];
-    return sign < 0 ? -v : v;
+    return sign < 0 ? -o.c[SRC] : o.c[SRC];
 }
 
 template <int N>
@@ -259,123 +334,140 @@ __global__ __launch_bounds__(kRectBlock) void k_rect_coboundary(const double* __
     }
 }
 
-template <int N, int K, bool DIAG>
-__global__ __launch_bounds__(kRectBlock) void k_rect_hodge(RectGeom<N> g, const double* __restrict__ in,
-                                                           RectView<N> vin, double* __restrict__ out,
-                                                           RectView<N> vout, uint32_t total)
+// One node of ⋆, δ and Δ: the components at n into v; false where a metric
+// asks for EXACT
+template <int N, int K, bool DIAG, bool EXACT>
+__device__ __forceinline__ bool hodge_node(const RectGeom<N>& g, const Form<N>& w, const Node<N>& n,
+                                           double (&v)[combos<N, N - K>()])
 {
-    const Form<N> w{in, vin};
-    for (uint32_t t = blockIdx.x * kRectBlock + threadIdx.x; t < total; t += gridDim.x * kRectBlock) {
-        Node<N> n;
-        rect_decode<N>(t, vout.ext, n.i);
-        const int64_t o = rect_offset<N>(vout, n.i);
-        const Star<N> s = load_star<N, DIAG>(g, n.i);
-        static_for<combos<N, N - K>()>([&](auto C) {
-            constexpr int c = decltype(C)::value;
-            constexpr unsigned src = ((1u << N) - 1u) & ~kCombos.mask[N][N - K][c];
-            out[o + c * vout.cstr] = star_coef<N, src>(s) * w.template at<src>(n);
-        });
-    }
+    bool plain = true;
+    const Star<N> s = load_star<N, DIAG, EXACT>(g, n.i, plain);
+    static_for<combos<N, N - K>()>([&](auto C) {
+        constexpr int c = decltype(C)::value;
+        constexpr unsigned src = ((1u << N) - 1u) & ~kCombos.mask[N][N - K][c];
+        v[c] = star_coef<N, src>(s) * w.template at<src>(n);
+    });
+    return plain;
 }
 
-template <int N, int K, bool DIAG>
-__global__ __launch_bounds__(kRectBlock) void k_rect_codifferential(RectGeom<N> g, const double* __restrict__ in,
-                                                                    RectView<N> vin, double* __restrict__ out,
-                                                                    RectView<N> vout, uint32_t total)
+template <int N, int K, bool DIAG, bool EXACT>
+__device__ __forceinline__ bool codifferential_node(const RectGeom<N>& g, const Form<N>& w, const Node<N>& n,
+                                                    double (&v)[combos<N, K - 1>()])
 {
-    const Form<N> w{in, vin};
-    for (uint32_t t = blockIdx.x * kRectBlock + threadIdx.x; t < total; t += gridDim.x * kRectBlock) {
-        Node<N> n;
-        rect_decode<N>(t, vout.ext, n.i);
-        const int64_t o = rect_offset<N>(vout, n.i);
-        const Star<N> s = load_star<N, DIAG>(g, n.i);
-        Star<N> sb[N];
-        static_for<N>([&](auto A) {
-            constexpr int a = decltype(A)::value;
-            sb[a] = load_star<N, DIAG>(g, back<N, a>(n).i);
-        });
-        static_for<combos<N, K - 1>()>([&](auto C) {
-            constexpr int c = decltype(C)::value;
-            constexpr unsigned I = kCombos.mask[N][K - 1][c];
-            out[o + c * vout.cstr] = codiff<N, K, I, false>(
-                w, n, s, [&](auto A, const Node<N>&) -> const Star<N>& { return sb[decltype(A)::value]; });
-        });
-    }
+    bool plain = true;
+    const Star<N> s = load_star<N, DIAG, EXACT>(g, n.i, plain);
+    Star<N> sb[N];
+    static_for<N>([&](auto A) {
+        constexpr int a = decltype(A)::value;
+        sb[a] = load_star<N, DIAG, EXACT>(g, back<N, a>(n).i, plain);
+    });
+    static_for<combos<N, K - 1>()>([&](auto C) {
+        constexpr int c = decltype(C)::value;
+        constexpr unsigned I = kCombos.mask[N][K - 1][c];
+        v[c] = codiff<N, K, I, false>(w, n, s,
+                                      [&](auto A, const Node<N>&) -> const Star<N>& { return sb[decltype(A)::value]; });
+    });
+    return plain;
 }
 
 // Δ = δd + dδ.  Stars of n, n ± e_a and (for dδ, where a component moves along
 // one axis and δ steps back along another) n + e_a − e_b.
-template <int N, int K, bool DIAG>
-__global__ __launch_bounds__(kRectBlock) void k_rect_laplacian(RectGeom<N> g, const double* __restrict__ in,
-                                                               RectView<N> vin, double* __restrict__ out,
-                                                               RectView<N> vout, uint32_t total)
+template <int N, int K, bool DIAG, bool EXACT>
+__device__ __forceinline__ bool laplacian_node(const RectGeom<N>& g, const Form<N>& w, const Node<N>& n,
+                                               double (&v)[combos<N, K>()])
 {
+    bool plain = true;
+    const Star<N> s = load_star<N, DIAG, EXACT>(g, n.i, plain);
+    Star<N> sb[N];
+    static_for<N>([&](auto A) {
+        constexpr int a = decltype(A)::value;
+        sb[a] = load_star<N, DIAG, EXACT>(g, back<N, a>(n).i, plain);
+    });
+    auto sb_of = [&](auto A, const Node<N>&) -> const Star<N>& { return sb[decltype(A)::value]; };
+    static_for<combos<N, K>()>([&](auto C) {
+        constexpr int c = decltype(C)::value;
+        constexpr unsigned I = kCombos.mask[N][K][c];
+        v[c] = 0.0;
+        if constexpr (K < N) v[c] += codiff<N, K + 1, I, true>(w, n, s, sb_of);
+    });
+    if constexpr (K > 0) {
+        // (dδω)_I = Σ_a ± [(δω)_{I∖a}(n + e_a) − (δω)_{I∖a}(n)], the
+        // difference 0 at the last node of the axis
+        static_for<N>([&](auto A) {
+            constexpr int a = decltype(A)::value;
+            const Node<N> f = next<N, a>(n, g.ext);
+            const bool inner = n.i[a] + 1 < g.ext[a];
+            const Star<N> sf = load_star<N, DIAG, EXACT>(g, f.i, plain);
+            auto sf_back = [&](auto B, const Node<N>& m) {
+                constexpr int b = decltype(B)::value;
+                if constexpr (b == a)
+                    return s; // f − e_a = n (at the last node f's value is dropped)
+                else
+                    return load_star<N, DIAG, EXACT>(g, m.i, plain);
+            };
+            static_for<combos<N, K>()>([&](auto C) {
+                constexpr int c = decltype(C)::value;
+                constexpr unsigned I = kCombos.mask[N][K][c];
+                if constexpr ((I >> a) & 1u) {
+                    constexpr unsigned J = I & ~(1u << a);
+                    const double here = codiff<N, K, J, false>(w, n, s, sb_of);
+                    const double ahead = codiff<N, K, J, false>(w, f, sf, sf_back);
+                    v[c] += axis_sign<I, a>() * ((inner ? ahead : here) - here);
+                }
+            });
+        });
+    }
+    return plain;
+}
+
+template <RectOp OP, int N, int K, bool DIAG>
+__global__ __launch_bounds__(kRectBlock) void k_rect_node(RectGeom<N> g, const double* __restrict__ in,
+                                                          RectView<N> vin, double* __restrict__ out, RectView<N> vout,
+                                                          uint32_t total)
+{
+    constexpr int KO = OP == RectOp::Hodge ? N - K : (OP == RectOp::Codifferential ? K - 1 : K);
     const Form<N> w{in, vin};
     for (uint32_t t = blockIdx.x * kRectBlock + threadIdx.x; t < total; t += gridDim.x * kRectBlock) {
         Node<N> n;
         rect_decode<N>(t, vout.ext, n.i);
         const int64_t o = rect_offset<N>(vout, n.i);
-        const Star<N> s = load_star<N, DIAG>(g, n.i);
-        Star<N> sb[N];
-        static_for<N>([&](auto A) {
-            constexpr int a = decltype(A)::value;
-            sb[a] = load_star<N, DIAG>(g, back<N, a>(n).i);
-        });
-        auto sb_of = [&](auto A, const Node<N>&) -> const Star<N>& { return sb[decltype(A)::value]; };
-        double acc[combos<N, K>()];
-        static_for<combos<N, K>()>([&](auto C) {
-            constexpr int c = decltype(C)::value;
-            constexpr unsigned I = kCombos.mask[N][K][c];
-            acc[c] = 0.0;
-            if constexpr (K < N) acc[c] += codiff<N, K + 1, I, true>(w, n, s, sb_of);
-        });
-        if constexpr (K > 0) {
-            // (dδω)_I = Σ_a ± [(δω)_{I∖a}(n + e_a) − (δω)_{I∖a}(n)], the
-            // difference 0 at the last node of the axis
-            static_for<N>([&](auto A) {
-                constexpr int a = decltype(A)::value;
-                const Node<N> f = next<N, a>(n, g.ext);
-                const bool inner = n.i[a] + 1 < g.ext[a];
-                const Star<N> sf = load_star<N, DIAG>(g, f.i);
-                auto sf_back = [&](auto B, const Node<N>& m) {
-                    constexpr int b = decltype(B)::value;
-                    if constexpr (b == a)
-                        return s; // f − e_a = n (at the last node f's value is dropped)
-                    else
-                        return load_star<N, DIAG>(g, m.i);
-                };
-                static_for<combos<N, K>()>([&](auto C) {
-                    constexpr int c = decltype(C)::value;
-                    constexpr unsigned I = kCombos.mask[N][K][c];
-                    if constexpr ((I >> a) & 1u) {
-                        constexpr unsigned J = I & ~(1u << a);
-                        const double here = codiff<N, K, J, false>(w, n, s, sb_of);
-                        const double ahead = codiff<N, K, J, false>(w, f, sf, sf_back);
-                        acc[c] += axis_sign<I, a>() * ((inner ? ahead : here) - here);
-                    }
-                });
-            });
+        double v[combos<N, KO>()];
+        auto node = [&](auto EXACT) {
+            constexpr bool exact = decltype(EXACT)::value;
+            if constexpr (OP == RectOp::Hodge)
+                return hodge_node<N, K, DIAG, exact>(g, w, n, v);
+            else if constexpr (OP == RectOp::Codifferential)
+                return codifferential_node<N, K, DIAG, exact>(g, w, n, v);
+            else
+                return laplacian_node<N, K, DIAG, exact>(g, w, n, v);
+        };
+        if (__builtin_expect(!node(std::false_type{}), 0)) {
+            // read again: the registers of the plain form hold nothing for this
+#pragma unroll
+            for (int a = 0; a < N; ++a) asm volatile("" : "+v"(n.i[a]));
+            node(std::true_type{});
         }
-        static_for<combos<N, K>()>([&](auto C) {
+        static_for<combos<N, KO>()>([&](auto C) {
             constexpr int c = decltype(C)::value;
-            out[o + c * vout.cstr] = acc[c];
+            out[o + c * vout.cstr] = v[c];
         });
     }
 }
 
 // Δ on 3D grids by a march along x: a workgroup owns 62 (z) × (TY − 2) (y)
 // nodes with a one-node halo and walks a chunk of x planes, so a node's star is
-// formed once per tile where k_rect_laplacian forms the stars of its 13 nodes.
+// formed once per tile where k_rect_node forms the stars of its 13 nodes.
 // Registers hold ω, the stars, ⋆ω and δω of planes p and p + 1 and ⋆dω of
 // p − 1; the y and z neighbours of ω, ⋆ω, ⋆dω and δω go through LDS, two
 // barriers a plane; plane p + 2 is requested a step before it is used.  Sums
-// and their order are those of k_rect_laplacian.  8 rows: two workgroups of a
-// 1- or 2-form a compute unit (91–106 registers, 45–53 KB of LDS), four of a 0-
-// or 3-form, which hide each other's barriers.  Diagonal metric, gather → march:
-//   2-form  65³ 22 → 14, 107 × 75 × 93 67 → 21, 129 × 120 × 135 177 → 43,
-//           256³ 1524 → 353 µs
-//   0-form  256³ 395 → 198 µs;  3-form  256³ 607 → 190 µs
-//   1-form  component-first, 256³ 1517 → 316 µs (index-last: dec_fused.hip)
+// and their order are those of k_rect_node.  8 rows: two workgroups of a
+// 1- or 2-form a compute unit (82–100 registers, 45–53 KB of LDS), three or four
+// of a 0- or 3-form, which hide each other's barriers (the bound holds the
+// 3-form's at 64 registers, four workgroups).  Diagonal metric, gather → march:
+//   2-form  65³ 18 → 12, 107 × 75 × 93 42 → 19, 129 × 120 × 135 107 → 43,
+//           256³ 981 → 330 µs
+//   0-form  256³ 279 → 168 µs;  3-form  256³ 390 → 165 µs
+//   1-form  component-first, 256³ 903 → 303 µs (index-last: dec_fused.hip)
 template <int K, int TY>
 struct MarchLds {
     double w[combos<3, K>()][TY][64];                       // ω(p): +y, +z neighbours of dω
@@ -385,9 +477,9 @@ struct MarchLds {
 };
 
 template <int K, bool DIAG, int TY>
-__global__ __launch_bounds__(64 * TY) void k_rect_lap3_march(RectGeom<3> g, const double* __restrict__ in,
-                                                             RectView<3> vin, double* __restrict__ out,
-                                                             RectView<3> vout, int ntz, int nty, int chunk)
+__global__ __launch_bounds__(64 * TY, K == 3 ? 8 : 1) void
+k_rect_lap3_march(RectGeom<3> g, const double* __restrict__ in, RectView<3> vin, double* __restrict__ out,
+                  RectView<3> vout, int ntz, int nty, int chunk)
 {
     constexpr int C = combos<3, K>(), CA = combos<3, K + 1>(), CD = combos<3, K - 1>();
     constexpr unsigned all = 7u;
@@ -414,11 +506,12 @@ __global__ __launch_bounds__(64 * TY) void k_rect_lap3_march(RectGeom<3> g, cons
     const int lp = lane < 63 ? lane + 1 : lane, lm = lane > 0 ? lane - 1 : lane;
     const double* col = in + jc * vin.str[1] + kc * vin.str[2];
     const double* gcol = DIAG ? g.g + 3 * (jc * g.node[1] + kc) : nullptr;
-    const double hy = g.h[1][jc], ry = g.r[1][jc], hz = g.h[2][kc], rz = g.r[2][kc];
+    const double hy = g.h[1][jc], hz = g.h[2][kc];
+    const IdentColumn ident(hy, hz);
 
     // the raw values of plane x (clamped into the grid)
     struct Raw {
-        double w[C], m[3], h, r;
+        double w[C], m[3], h;
     };
     auto request = [&](int64_t x, Raw& o) {
         const int64_t xc = min(max(x, (int64_t)0), Nx - 1);
@@ -431,21 +524,16 @@ __global__ __launch_bounds__(64 * TY) void k_rect_lap3_march(RectGeom<3> g, cons
             for (int a = 0; a < 3; ++a) o.m[a] = q[a];
         }
         o.h = g.h[0][xc];
-        o.r = g.r[0][xc];
     };
     auto star_of = [&](const Raw& o) {
-        Star<3> s;
         if constexpr (DIAG) {
-            const bool ok = o.m[0] != 0.0 && o.m[1] != 0.0 && o.m[2] != 0.0;
-            axis_star(ok ? o.m[0] : 0.0, o.h, o.r, s.s[0], s.r[0]);
-            axis_star(ok ? o.m[1] : 0.0, hy, ry, s.s[1], s.r[1]);
-            axis_star(ok ? o.m[2] : 0.0, hz, rz, s.s[2], s.r[2]);
+            const double h[3] = {o.h, hy, hz};
+            bool plain = true;
+            const Star<3> s = diag_star<3, false>(o.m, h, plain);
+            return __builtin_expect(plain, 1) ? s : diag_star<3, true>(o.m, h, plain);
         } else {
-            s.s[0] = fabs(o.h), s.r[0] = fabs(o.r);
-            s.s[1] = fabs(hy), s.r[1] = fabs(ry);
-            s.s[2] = fabs(hz), s.r[2] = fabs(rz);
+            return ident.at(o.h);
         }
-        return s;
     };
 
     double W[C], B[K > 0 ? C : 1], D[K > 0 ? CD : 1], Aback[K < 3 ? CA : 1];
@@ -599,7 +687,6 @@ RectGeom<N> rect_geom(const DevGeom& g)
     int64_t lin = 1;
     for (int a = N - 1; a >= 0; --a) {
         r.h[a] = g.spacing[a];
-        r.r[a] = g.inv_spacing[a];
         r.ext[a] = static_cast<uint32_t>(g.ext[a]);
         r.node[a] = lin;
         lin *= g.ext[a];
@@ -617,18 +704,22 @@ constexpr int kMarchRows = 8;
 
 struct March {
     int ntz, nty, chunk;
-    int64_t blocks; // 0: k_rect_laplacian
+    int64_t blocks; // 0: k_rect_node
 };
 
 // The march takes a grid where enough of its lanes hold nodes to write, and a
 // 0- or 3-form also needs 500 000 nodes: below, the gather of 7 stars is the
-// shorter chain (65³, 0-form, diagonal metric: 8.7 against 10.7 µs; 107 × 75 ×
-// 93: 19 against 16).  A gather costs a node 2 (0-form) to 5 times (2-form,
-// diagonal metric) a lane's step here.  On 256 × 256 × z nodes, gather / march:
-//   0-form, diagonal   z = 25: 32/40    z = 33: 42/40
-//   2-form, identity   z = 17: 34/43    z = 25: 49/43
-//   2-form, diagonal   z = 9:  41/56    z = 17: 76/56
-//   3-form, diagonal   z = 17: 35/38    z = 25: 49/38
+// shorter chain (79³, diagonal metric: 0-form 10 against 12 µs, 3-form 14 against
+// 12; 107 × 75 × 93: 14 against 14, 20 against 13).  On 256 × 256 × z nodes, of 62
+// along z, gather / march in µs (1-form component-first):
+//   identity  0-form  z = 29: 17/20   z = 33: 19/20   z = 41: 23/20
+//             1-form  z = 17: 33/41   z = 21: 40/41   z = 25: 47/42
+//             2-form  z = 17: 34/41   z = 21: 40/41   z = 25: 47/41
+//             3-form  z = 25: 18/20   z = 29: 21/20
+//   diagonal  0-form  z = 29: 28/34   z = 33: 31/34   z = 41: 38/34
+//             1-form  z = 13: 42/53   z = 17: 54/53   z = 21: 66/53
+//             2-form  z = 13: 43/52   z = 17: 54/53   z = 21: 68/53
+//             3-form  z = 17: 25/31   z = 21: 30/31   z = 25: 35/31
 template <int K, bool DIAG>
 March march_shape(const RectView<3>& o)
 {
@@ -637,7 +728,7 @@ March march_shape(const RectView<3>& o)
     m.nty = (int)((o.ext[1] + kMarchRows - 3) / (kMarchRows - 2));
     const int64_t tiles = (int64_t)m.ntz * m.nty, column = (int64_t)o.ext[1] * o.ext[2];
     constexpr bool ends = K == 0 || K == 3;
-    constexpr double used = K == 0 ? 0.375 : (!ends && DIAG ? 0.125 : 0.25);
+    constexpr double used = K == 0 ? 0.4 : (K == 3 ? (DIAG ? 0.26 : 0.31) : (DIAG ? 0.2 : 0.25));
     if ((ends && column * o.ext[0] < 500000) || (double)column < used * 64 * kMarchRows * (double)tiles) return m;
     m.chunk = march_chunk(tiles, o.ext[0], ends ? 4 : 2, &m.blocks);
     if (m.blocks > INT32_MAX) m.blocks = 0;
@@ -658,9 +749,15 @@ void rect_launch(RectOp op, const DevGeom* g, const double* in, const sil_view& 
     const RectGeom<N> rg = rect_geom<N>(*g);
     auto go = [&](auto D) {
         constexpr bool diag = decltype(D)::value;
-        if (op == RectOp::Hodge)
-            hipLaunchKernelGGL((k_rect_hodge<N, K, diag>), grid, block, 0, stream, rg, in, vi, out, vo, total);
-        else if (op == RectOp::Laplacian) {
+        auto gather = [&](auto OP) {
+            hipLaunchKernelGGL((k_rect_node<decltype(OP)::value, N, K, diag>), grid, block, 0, stream, rg, in, vi, out,
+                               vo, total);
+        };
+        if (op == RectOp::Hodge) {
+            gather(std::integral_constant<RectOp, RectOp::Hodge>{});
+        } else if (op == RectOp::Codifferential) {
+            if constexpr (K > 0) gather(std::integral_constant<RectOp, RectOp::Codifferential>{});
+        } else {
             if constexpr (N == 3) {
                 const March m = march_shape<K, diag>(vo);
                 if (m.blocks > 0) {
@@ -669,11 +766,8 @@ void rect_launch(RectOp op, const DevGeom* g, const double* in, const sil_view& 
                     return;
                 }
             }
-            hipLaunchKernelGGL((k_rect_laplacian<N, K, diag>), grid, block, 0, stream, rg, in, vi, out, vo, total);
+            gather(std::integral_constant<RectOp, RectOp::Laplacian>{});
         }
-        else if constexpr (K > 0)
-            hipLaunchKernelGGL((k_rect_codifferential<N, K, diag>), grid, block, 0, stream, rg, in, vi, out, vo,
-                               total);
     };
     if (rg.g)
         go(std::true_type{});

@@ -3,6 +3,7 @@
 their rule can go wrong: one- and two-node axes (the general kernels), grids
 that leave a partial workgroup, component-first and permuted storage, output
 domains shorter than the grid, singular and extreme metric entries."""
+from itertools import combinations
 from math import comb
 
 import numpy as np
@@ -187,3 +188,77 @@ def test_default_stream_is_the_current_one():
         t.add_(1.0)
         assert same()
     assert L.stream_handle(side).value == side.cuda_stream
+
+
+def edge_lengths(axes):
+    h = [np.append(np.diff(a), a[-1] - a[-2]) for a in axes]
+    return np.stack(np.meshgrid(*[np.abs(x) for x in h], indexing="ij"), axis=-1)
+
+
+def star_quotients(h, m, src, real):
+    """Π_tgt s / Π_src s at every node, s_a = √|m_a| h_a, in the arithmetic `real`"""
+    s = h.astype(real) if m is None else np.sqrt(np.abs(m).astype(real)) * h.astype(real)
+    num, den = np.ones(h.shape[:-1], dtype=real), np.ones(h.shape[:-1], dtype=real)
+    for a in range(h.shape[-1]):
+        if a in src:
+            den = den * s[..., a]
+        else:
+            num = num * s[..., a]
+    return num / den
+
+
+def device_star(axes, m, k):
+    """|⋆| of a k-form of ones: {source axes: coefficient per node}"""
+    import similie_amd.exterior as E
+
+    n, extents = len(axes), tuple(len(a) for a in axes)
+    gg = E.Grid(extents, axis_coords=axes, metric=None if m is None else cuda(m),
+                metric_kind=orc.METRIC_IDENTITY if m is None else orc.METRIC_DIAGONAL)
+    w = torch.ones(extents + (comb(n, k),), dtype=torch.float64, device="cuda")
+    o = torch.empty(extents + (comb(n, n - k),), dtype=torch.float64, device="cuda")
+    E.hodge_star(gg, k, o, w)
+    o = np.abs(o.cpu().numpy())
+    return {tuple(a for a in range(n) if a not in tgt): o[..., q] for q, tgt in enumerate(combinations(range(n), n - k))}
+
+
+@pytest.mark.parametrize("kind", ["identity", "diagonal"])
+@pytest.mark.parametrize("extents", [[60000], [300, 200], [40, 40, 40]])
+def test_star_rounds_no_more_than_quotients_of_products(extents, kind):
+    """The rms rounding of every coefficient against 64-bit mantissas, and that
+    of quotients of FP64 products, as the general kernels form them.  Over
+    64 000 nodes the two rms figures are known to about 0.5 %: 2 % apart is a
+    difference in the arithmetic."""
+    n = len(extents)
+    rng = np.random.default_rng(n)
+    axes = [np.cumsum(np.concatenate([[0.0], np.exp(rng.uniform(-4.0, 2.0, e - 1))])) for e in extents]
+    m = None if kind == "identity" else np.exp(rng.uniform(-8.0, 8.0, tuple(extents) + (n,)))
+    h = edge_lengths(axes)
+    for k in range(n + 1):
+        got, plain, sq = device_star(axes, m, k), 0.0, 0.0
+        for src, c in got.items():
+            exact = star_quotients(h, m, src, np.longdouble)
+            sq += float(np.mean(((c - exact) / exact) ** 2))
+            plain += float(np.mean(((star_quotients(h, m, src, np.float64) - exact) / exact) ** 2))
+        print(f"star {extents} {kind} k={k}: rms {np.sqrt(sq / len(got)):.3e}, "
+              f"quotients {np.sqrt(plain / len(got)):.3e}", flush=True)
+        assert sq <= 1.02 ** 2 * plain, k
+
+
+@pytest.mark.parametrize("n", [1, 2, 3])
+def test_metric_entries_without_a_finite_measure(n):
+    """zero, infinite, NaN, subnormal and huge entries: what the quotients of
+    products give (zero where the metric is singular or the source measure
+    vanishes)"""
+    rng = np.random.default_rng(n)
+    axes = [np.cumsum(np.concatenate([[0.0], rng.uniform(0.5, 1.5, e - 1)])) for e in [40, 9, 7][:n]]
+    extents = tuple(len(a) for a in axes)
+    m = rng.choice([1.0, 2.5, -3.0, 0.0, np.inf, np.nan, 5e-324, 1e-200, 1e200, 1.7e308], extents + (n,))
+    h = edge_lengths(axes)
+    with np.errstate(all="ignore"):
+        for k in range(n + 1):
+            for src, c in device_star(axes, m, k).items():
+                want = np.abs(star_quotients(h, m, src, np.float64))
+                s = np.sqrt(np.abs(m)) * h
+                measure = np.prod([s[..., a] for a in src], axis=0) if src else np.ones(extents)
+                want = np.where(np.any(m == 0.0, axis=-1) | (measure == 0.0), 0.0, want)
+                np.testing.assert_allclose(c, want, rtol=1e-15 * 8, atol=0.0, err_msg=str(src))
