@@ -320,6 +320,12 @@ static_assert(kWideNT * kWU == kWideNodes, "a workgroup's nodes per pass");
 
 enum WideMode { W_START = 0, W_CG, W_REPLACE };
 
+// a wide problem's direction buffer
+__device__ __forceinline__ float* wide_p(const WideLaunch& L, const WideSlot& W, int buffer)
+{
+    return buffer ? L.p[1] + W.offset2 : L.p[0] + W.offset;
+}
+
 // sums of `count` (≤ kWideNT) pairs in every thread, fixed order
 __device__ __forceinline__ void wide_sums(const double* __restrict__ part, int count, double& a, double& b)
 {
@@ -372,7 +378,7 @@ __global__ __launch_bounds__(kWideNT) void k_wide_init(WideLaunch L)
     const double* b = L.b + W.offset;
     double* x = L.x + W.offset;
     float* r = L.r + W.offset;
-    float* p = L.p[0] + W.offset;
+    float* p = wide_p(L, W, 0);
     const float* dinv = L.dinv32 + W.offset;
     double bb = 0.0, rz = 0.0;
     for (unsigned t = m.index * kWideNodes + threadIdx.x; t < nn; t += W.nb * kWideNodes)
@@ -429,7 +435,7 @@ __global__ __launch_bounds__(kWideNT) void k_wide_a(WideLaunch L, int s)
     const unsigned nn = (unsigned)n * n;
     float* r = L.r + W.offset;
     const float* dinv = L.dinv32 + W.offset;
-    const float* po = L.p[S.pcur] + W.offset;
+    const float* po = wide_p(L, W, S.pcur);
     const float* wx = L.wx32 + W.offset;
     const float* wy = L.wy32 + W.offset;
     const bool jac = L.jacobi != 0;
@@ -531,7 +537,7 @@ __global__ __launch_bounds__(kWideNT) void k_wide_a(WideLaunch L, int s)
     }
 
     const float beta = (float)N.beta;
-    float* pn = L.p[N.pcur] + W.offset;
+    float* pn = wide_p(L, W, N.pcur);
     float* q = L.q + W.offset;
     double pq = 0.0;
     for (unsigned t0 = t_first; t0 < nn;) {
@@ -570,7 +576,7 @@ __global__ __launch_bounds__(kWideNT) void k_wide_b(WideLaunch L, int s)
     const double rz_now = S.rz;
     const unsigned nn = (unsigned)W.n * W.n;
     double* x = L.x + W.offset;
-    const float* p = L.p[S.pcur] + W.offset;
+    const float* p = wide_p(L, W, S.pcur);
     float* r = L.r + W.offset;
     const float* q = L.q + W.offset;
     const float* dinv = L.dinv32 + W.offset;

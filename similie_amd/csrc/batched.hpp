@@ -54,6 +54,7 @@ constexpr int kWideMaxBlocks = 256; // most workgroups per problem (each sums th
 // a wide problem: its arrays, its workgroups and their partial sums
 struct WideSlot {
     int64_t offset;
+    int64_t offset2; // in the second direction buffer
     int32_t n, id;
     int32_t nb;   // workgroups
     int32_t part; // slot of the first one's partials
@@ -76,7 +77,7 @@ struct WideLaunch {
     const double* b;
     double* x;
     float* r;
-    float* p[2];
+    float* p[2]; // direction buffers: of all problems, of the wide ones
     float* q;
     const float* dinv32;
     int jacobi;

@@ -41,7 +41,7 @@ struct sil_batched_poisson_s {
     std::vector<std::pair<int, hipGraphExec_t>> wide_graphs; // by grid size
     int wide_max_it = -1, wide_replace = -1, wide_jacobi = -1;
     double wide_tol = -1.0;
-    float* p2 = nullptr;              // second direction buffer of the wide path
+    float* p2 = nullptr;              // second direction buffer of the wide problems
     hipStream_t side_stream = nullptr; // the persistent kernel's, beside the wide path
     hipEvent_t fork = nullptr, join = nullptr;
     int* queue = nullptr;
@@ -69,7 +69,8 @@ void drop_wide_graphs(sil_batched_poisson h)
 void free_split(sil_batched_poisson h)
 {
     for (void* ptr : {(void*)h->order_dev, (void*)h->slots_dev, (void*)h->full_map_dev, (void*)h->map_dev,
-                      (void*)h->nactive_dev, (void*)h->wide_state, (void*)h->wide_part, (void*)h->wide_done})
+                      (void*)h->nactive_dev, (void*)h->wide_state, (void*)h->wide_part, (void*)h->wide_done,
+                      (void*)h->p2})
         if (ptr) (void)hipFree(ptr);
     h->order_dev = nullptr;
     h->slots_dev = nullptr;
@@ -79,6 +80,7 @@ void free_split(sil_batched_poisson h)
     h->wide_state = nullptr;
     h->wide_part = nullptr;
     h->wide_done = nullptr;
+    h->p2 = nullptr;
     if (h->wide_host) (void)hipHostFree(h->wide_host);
     h->wide_host = nullptr;
     if (h->graph) (void)hipGraphExecDestroy(h->graph);
@@ -92,7 +94,7 @@ void release(sil_batched_poisson h)
     if (!h) return;
     free_split(h);
     for (void* ptr : {(void*)h->problems_dev, (void*)h->queue, (void*)h->wx32, (void*)h->wy32, (void*)h->dinv32,
-                      (void*)h->r, (void*)h->p, (void*)h->p2, (void*)h->q, (void*)h->wx64, (void*)h->wy64,
+                      (void*)h->r, (void*)h->p, (void*)h->q, (void*)h->wx64, (void*)h->wy64,
                       (void*)h->b, (void*)h->x, (void*)h->results_dev})
         if (ptr) (void)hipFree(ptr);
     for (hipEvent_t e : {h->wide_event[0], h->wide_event[1], h->fork, h->join})
@@ -337,11 +339,13 @@ int map_wide(sil_batched_poisson h)
     drop_wide_graphs(h);
     h->slots.clear();
     h->full_map.clear();
+    int64_t offset2 = 0;
     for (int i = 0; i < h->nwide; ++i) {
         const BatchProblem& p = h->problems[h->wide_ids[i]];
         const int64_t nn = (int64_t)p.side * p.side;
         const int nb = (int)std::min<int64_t>(h->nbx, (nn + kWideNodes - 1) / kWideNodes);
-        h->slots.push_back(WideSlot{p.offset, p.side, h->wide_ids[i], nb, (int)h->full_map.size()});
+        h->slots.push_back(WideSlot{p.offset, offset2, p.side, h->wide_ids[i], nb, (int)h->full_map.size()});
+        offset2 += nn;
         for (int b = 0; b < nb; ++b) h->full_map.push_back(WideBlock{i, b});
     }
     if (h->nwide == 0) return SIL_OK;
@@ -360,13 +364,14 @@ int partition(sil_batched_poisson h, int wide_side)
     h->wide_side = wide_side;
     std::vector<int> order;
     h->wide_ids.clear();
-    int64_t max_wide_nn = 0, total_blocks = 0;
+    int64_t max_wide_nn = 0, wide_nodes = 0, total_blocks = 0;
     for (int i = 0; i < h->nprob; ++i) {
         const int side = h->problems[i].side;
         if (side >= wide_side) {
             const int64_t nn = (int64_t)side * side;
             h->wide_ids.push_back(i);
             max_wide_nn = std::max(max_wide_nn, nn);
+            wide_nodes += nn;
             total_blocks += std::min<int64_t>(kWideMaxBlocks, (nn + kWideNodes - 1) / kWideNodes);
         } else {
             order.push_back(i);
@@ -386,7 +391,7 @@ int partition(sil_batched_poisson h, int wide_side)
         (rc = dalloc(&h->nactive_dev, 1)) || (rc = dalloc(&h->wide_state, 2 * nw)) ||
         (rc = dalloc(&h->wide_part, 3 * 2 * nblk)) || (rc = dalloc(&h->wide_done, nw)))
         return rc;
-    if (h->nwide && !h->p2 && (rc = dalloc(&h->p2, h->total))) return rc;
+    if (h->nwide && (rc = dalloc(&h->p2, wide_nodes))) return rc;
     const size_t map_bytes = sizeof(WideBlock) * nblk, done_bytes = sizeof(int) * nw;
     if (hipHostMalloc(&h->wide_host, 2 * (map_bytes + done_bytes + sizeof(int))) != hipSuccess) {
         h->wide_host = nullptr;

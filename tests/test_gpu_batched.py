@@ -145,3 +145,25 @@ def test_wide_and_persistent_paths_take_the_same_iterations(limit, replace, monk
         assert abs(rw[p]["true_relative_residual"] - rp[p]["true_relative_residual"]) <= \
             1e-4 * rp[p]["true_relative_residual"] + 1e-10
     assert np.linalg.norm(xw - xp) <= 1e-4 * np.linalg.norm(xp)
+
+
+def test_second_direction_buffer_is_the_wide_problems_alone():
+    """6000 problems of the persistent kernel and one wide one: a handle holds
+    six FP32 and four FP64 values a node, and the wide path's own arrays for
+    the wide problem only (an FP32 value a node of all would be 194 MB; 64 MB
+    are left for the rounding of some twenty allocations)"""
+    import gc
+
+    from similie_amd.batched import BatchedPoisson2D
+
+    sides = [90] * 6000 + [96]
+    nodes = sum(n * n for n in sides)
+    kappa = torch.ones(nodes, dtype=torch.float64, device="cuda")
+    gc.collect()
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    solver = BatchedPoisson2D(sides, kappa)
+    torch.cuda.synchronize()
+    held = before - torch.cuda.mem_get_info()[0]
+    assert 56 * nodes <= held <= 56 * nodes + (64 << 20), held / nodes
+    del solver
