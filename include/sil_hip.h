@@ -577,8 +577,9 @@ int sil_magnetostatics_cell_inputs(const int32_t* cell_tags, int64_t ncells, con
 
 /* No reference counterpart (the reference runs one Ginkgo solve per
  * operator): many independent Dirichlet-zero 2D Poisson problems of uneven
- * size on unit-spaced square grids, solved in one persistent launch captured
- * in a hipGraph.  Problem p has sides[p]² nodes (x slowest) stored at offset
+ * size on unit-spaced square grids: those of side >= 96 (or what the autotuner
+ * chose) each spread over many workgroups, two kernels a step, and beside them
+ * the others in one persistent launch, a workgroup each.  Problem p has sides[p]² nodes (x slowest) stored at offset
  * sil_batched_poisson2d_offset(h, p) of every concatenated array; kappa is
  * the nodal coefficient (device, concatenated; edge value = mean of its two
  * nodes).  The solve is CG (settings.preconditioner: Jacobi or identity)
@@ -597,6 +598,9 @@ int sil_batched_poisson2d_create(sil_batched_poisson* out, int32_t nproblems, co
 int64_t sil_batched_poisson2d_offset(sil_batched_poisson h, int32_t problem);
 /* workgroup size of the persistent kernel (256, 512 or 1024) */
 int sil_batched_poisson2d_set_block(sil_batched_poisson h, int32_t block);
+/* the size in use: 1024 or 512 by the number of small problems until it is set
+ * or autotuned */
+int32_t sil_batched_poisson2d_block(sil_batched_poisson h);
 /* times every workgroup size on `probe_iterations` iterations of every
  * problem and keeps the fastest */
 int sil_batched_poisson2d_autotune(sil_batched_poisson h, const double* rhs, int32_t probe_iterations,
@@ -616,8 +620,8 @@ typedef struct sil_batch_shape {
 } sil_batch_shape;
 int sil_batched_poisson2d_autotune_shape(sil_batched_poisson h, const double* rhs, int32_t probe_iterations,
                                          sil_batch_shape* chosen);
-/* results: host array of nproblems entries (or NULL); seconds: device time
- * of the graph launch (or NULL) */
+/* results: host array of nproblems entries (or NULL); seconds: the
+ * solve's time on the host's clock, inputs in place to results (or NULL) */
 int sil_batched_poisson2d_solve(sil_batched_poisson h, const double* rhs, double* solution,
                                 const sil_solver_settings* settings, sil_batch_result* results, double* seconds,
                                 void* stream);

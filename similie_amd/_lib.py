@@ -252,6 +252,7 @@ SIGNATURES = {
     "sil_batched_poisson2d_create": (ctypes.c_int, [ctypes.POINTER(_P), _I32, ctypes.POINTER(_I32), _P]),
     "sil_batched_poisson2d_offset": (_I64, [_P, _I32]),
     "sil_batched_poisson2d_set_block": (ctypes.c_int, [_P, _I32]),
+    "sil_batched_poisson2d_block": (_I32, [_P]),
     "sil_batched_poisson2d_autotune": (
         ctypes.c_int,
         [_P, _P, _I32, ctypes.POINTER(_I32), ctypes.POINTER(ctypes.c_double)],

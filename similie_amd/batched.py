@@ -1,4 +1,5 @@
-"""Batched persistent Poisson solves (many uneven 2D problems, one launch).
+"""Batched Poisson solves: many uneven 2D problems, the small ones in one
+persistent launch beside the large ones' kernels.
 
 No reference counterpart: the reference solves one operator per Ginkgo
 call.  See sil_batched_poisson2d_* in include/sil_hip.h.
@@ -30,7 +31,7 @@ class BatchedPoisson2D:
         L.check(L.lib().sil_batched_poisson2d_create(ctypes.byref(h), len(self.sides), arr, L.ptr(kappa)))
         self.handle = h
         self._destroy = L.lib().sil_batched_poisson2d_destroy
-        self.block = 256
+        self.block = int(L.lib().sil_batched_poisson2d_block(self.handle))
 
     def offset(self, p):
         return int(L.lib().sil_batched_poisson2d_offset(self.handle, p))

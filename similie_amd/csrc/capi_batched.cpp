@@ -519,6 +519,8 @@ int sil_batched_poisson2d_set_block(sil_batched_poisson h, int32_t block)
     return SIL_OK;
 }
 
+int32_t sil_batched_poisson2d_block(sil_batched_poisson h) { return h ? h->block : 0; }
+
 int sil_batched_poisson2d_solve(sil_batched_poisson h, const double* rhs, double* solution,
                                 const sil_solver_settings* st, sil_batch_result* results, double* seconds,
                                 void* stream)

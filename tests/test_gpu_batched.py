@@ -167,3 +167,19 @@ def test_second_direction_buffer_is_the_wide_problems_alone():
     held = before - torch.cuda.mem_get_info()[0]
     assert 56 * nodes <= held <= 56 * nodes + (64 << 20), held / nodes
     del solver
+
+
+def test_the_workgroup_size_is_the_one_in_use():
+    """few small problems: 16 wavefronts each; many: eight; set or autotuned:
+    that"""
+    from similie_amd import _lib as L
+    from similie_amd.batched import BatchedPoisson2D
+
+    compute_units = torch.cuda.get_device_properties(0).multi_processor_count
+    for count, block in ((4, 1024), (2 * compute_units, 1024), (2 * compute_units + 1, 512)):
+        solver = BatchedPoisson2D([5] * count, torch.ones(25 * count, dtype=torch.float64, device="cuda"))
+        assert solver.block == block == L.lib().sil_batched_poisson2d_block(solver.handle)
+        solver.set_block(256)
+        assert solver.block == 256 == L.lib().sil_batched_poisson2d_block(solver.handle)
+        chosen, _ = solver.autotune(torch.ones(25 * count, dtype=torch.float64, device="cuda"), probe_iterations=2)
+        assert solver.block == chosen == L.lib().sil_batched_poisson2d_block(solver.handle)
