@@ -912,13 +912,8 @@ __global__ __launch_bounds__(kBlock) void k_p2d_apply(int64_t nx, int64_t ny, co
     }
     T v[5];
     if constexpr (PU) {
-        double beta;
-        if (pu.step.sc) {
-            if (!cg_begin<kBlock>(pu.step, beta)) return;
-        } else {
-            if (*pu.done) return;
-            beta = *pu.beta;
-        }
+        double beta; // (every CG on this operator is a joined one)
+        if (!cg_begin<kBlock>(pu.step, beta)) return;
 #pragma unroll
         for (int q = 0; q < 5; ++q) {
             // arithmetic of p_value
