@@ -183,3 +183,52 @@ def test_the_workgroup_size_is_the_one_in_use():
         assert solver.block == 256 == L.lib().sil_batched_poisson2d_block(solver.handle)
         chosen, _ = solver.autotune(torch.ones(25 * count, dtype=torch.float64, device="cuda"), probe_iterations=2)
         assert solver.block == chosen == L.lib().sil_batched_poisson2d_block(solver.handle)
+
+
+@pytest.mark.parametrize("limit,replace", [(24, 0), (41, 7)])
+def test_wide_problems_that_finish_at_different_times(limit, replace, monkeypatch):
+    """Wide problems whose right-hand sides hold 1, 6, 14 or 22 eigenvectors
+    finish after about as many iterations, and the map of workgroups is
+    rebuilt while a problem of side 517 still runs, whose 256 workgroups take
+    a second, partial pass (267 289 nodes).  The persistent kernel does the
+    same arithmetic with its FP64 sums in another order: the solved problems
+    stop within an iteration of it on a verified residual, the others hold
+    its iterates (FP32 recurrences, 1e-4 as in the test above)."""
+    from similie_amd.batched import BatchedPoisson2D
+    from similie_amd.solvers import StrongFormulationSolverSettings
+
+    rng = np.random.default_rng(4)
+    modes = {96: 1, 160: 1, 161: 6, 200: 6, 130: 14, 201: 14, 162: 22, 97: 22}
+    sides, kap = [517], [np.exp(0.5 * rng.standard_normal((517, 517)))]
+    rhs = [np.pad(rng.standard_normal((515, 515)), 1)]
+    for n, count in modes.items():  # of middle wavelengths: eigenvalues that FP32 products resolve
+        t = np.pi * np.arange(n) / (n - 1)
+        b = np.zeros((n, n))
+        for m in range(1, count + 1):
+            b += rng.uniform(0.5, 1.5) * np.outer(np.sin((n // 8 + 2 * m) * t), np.sin((n // 6 + m) * t))
+        b[0], b[-1], b[:, 0], b[:, -1] = 0.0, 0.0, 0.0, 0.0
+        sides.append(n), kap.append(np.ones((n, n))), rhs.append(b)
+    kappa = torch.from_numpy(np.concatenate([k.ravel() for k in kap])).cuda()
+    b = torch.from_numpy(np.concatenate([r.ravel() for r in rhs])).cuda()
+    st = StrongFormulationSolverSettings(relative_tolerance=1e-5, precision="mixed", preconditioner="identity",
+                                         max_iterations=limit, replace_interval=replace)
+    got = []
+    for side in ("96", "100000"):
+        monkeypatch.setenv("SIL_BATCH_WIDE_SIDE", side)
+        x, results, _ = BatchedPoisson2D(sides, kappa).solve(b, settings=st)
+        got.append((x.cpu().numpy(), results))
+    (xw, rw), (xp, rp) = got
+    print([r["iterations"] for r in rw], [r["iterations"] for r in rp], flush=True)
+    assert len({r["iterations"] for r in rw if r["converged"]}) >= 3 and not rw[0]["converged"]
+    at = 0
+    for p, n in enumerate(sides):
+        xi, xr = xw[at:at + n * n], xp[at:at + n * n]
+        at += n * n
+        assert rw[p]["converged"] == rp[p]["converged"], p
+        if rw[p]["converged"]:
+            assert abs(rw[p]["iterations"] - rp[p]["iterations"]) <= 1, p
+            r = rhs[p] - orc.poisson2d_apply(np.ones(n), np.ones(n), kap[p], xi.reshape(n, n))
+            assert np.linalg.norm(r) <= 1.0001e-5 * np.linalg.norm(rhs[p]), p
+        else:
+            assert rw[p]["iterations"] == rp[p]["iterations"] == limit, p
+        assert np.linalg.norm(xi - xr) <= 1e-4 * np.linalg.norm(xr), p

@@ -152,7 +152,8 @@ def check_every_cell_between_guards():
     import similie_amd.solvers as S
 
     pad = 4096
-    for shape, nonlinear in (((70, 21, 5), True), ((65, 9, 3), False), ((64, 8), True), ((131, 18), False), ((2, 2), True)):
+    for shape, nonlinear in (((70, 21, 5), True), ((65, 9, 3), False), ((64, 8), True), ((131, 18), False),
+                             ((2, 2), True)):
         print(f"guarded post_process shape={shape} nonlinear={nonlinear}", flush=True)
         rng = np.random.default_rng(sum(shape))
         coords = axes(shape, rng)

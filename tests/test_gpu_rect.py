@@ -218,7 +218,8 @@ def device_star(axes, m, k):
     o = torch.empty(extents + (comb(n, n - k),), dtype=torch.float64, device="cuda")
     E.hodge_star(gg, k, o, w)
     o = np.abs(o.cpu().numpy())
-    return {tuple(a for a in range(n) if a not in tgt): o[..., q] for q, tgt in enumerate(combinations(range(n), n - k))}
+    return {tuple(a for a in range(n) if a not in tgt): o[..., q]
+            for q, tgt in enumerate(combinations(range(n), n - k))}
 
 
 @pytest.mark.parametrize("kind", ["identity", "diagonal"])
@@ -262,3 +263,31 @@ def test_metric_entries_without_a_finite_measure(n):
                 measure = np.prod([s[..., a] for a in src], axis=0) if src else np.ones(extents)
                 want = np.where(np.any(m == 0.0, axis=-1) | (measure == 0.0), 0.0, want)
                 np.testing.assert_allclose(c, want, rtol=1e-15 * 8, atol=0.0, err_msg=str(src))
+
+
+@pytest.mark.parametrize("kind", ["identity", "diagonal"])
+@pytest.mark.parametrize("extents,oext,degrees", [([23, 13, 125], [10, 12, 100], (1, 2)),
+                                                  ([23, 13, 125], [1, 13, 124], (1, 2)),
+                                                  ([9, 70, 66], [7, 61, 62], (1, 2)),
+                                                  ([131, 69, 70], [128, 64, 62], (0, 3))])
+def test_march_on_output_domains_well_inside_the_grid(extents, oext, degrees, kind):
+    """output domains several nodes shorter than the grid along each axis: the
+    last tiles and chunks read nodes that none of them writes"""
+    import similie_amd.exterior as E
+
+    rng = np.random.default_rng(sum(extents))
+    axes = [np.cumsum(np.concatenate([[0.0], rng.uniform(0.5, 1.5, e - 1)])) for e in extents]
+    m = metric_of(rng, extents, 3, kind)
+    mk = orc.METRIC_IDENTITY if m is None else orc.METRIC_DIAGONAL
+    og = orc.Geometry(extents, axes=axes, metric_kind=mk, metric=None if m is None else m.reshape(-1, 3))
+    gg = E.Grid(extents, axis_coords=axes, metric=None if m is None else cuda(m), metric_kind=mk)
+    for k in degrees:
+        w = rng.standard_normal(tuple(extents) + (comb(3, k),))
+        ref = orc.laplacian(og, k, w, oext)
+        for order in orders(3):
+            t = stored(w.shape, order)
+            t.copy_(cuda(w))
+            o = stored(tuple(oext) + (comb(3, k),), order)
+            o.fill_(float("nan"))
+            E.laplacian(gg, k, o, t, comp_dim=3)
+            assert close(o, ref), (k, order)

@@ -220,3 +220,30 @@ def test_cg_stops_at_the_iteration_limit(shape, precision):
             ref = _numpy_cg(apply, diag, b, limit)
             tol = 1e-10 if precision == "fp64" else 2e-3
             assert np.linalg.norm(x.cpu().numpy() - ref) <= tol * np.linalg.norm(ref), limit
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_cg_with_more_partial_sums_than_a_workgroup_adds(precision):
+    """From 2049 workgroups of a product on (524 288 nodes of a 2D Poisson
+    grid) α comes from a kernel of its own: the iterates after 1, 2 and 5
+    iterations against plain CG (5 steps of a recurrence that the operator's
+    condition of these few steps amplifies by less than 1e3: 5e3 · u)."""
+    from similie_amd import solvers as S
+
+    rng = np.random.default_rng(21)
+    shape = (1027, 515)
+    assert (np.prod(shape) + 255) // 256 > 2048
+    kappa = torch.from_numpy(np.exp(rng.standard_normal(shape)).reshape(-1)).cuda()
+    op = S.Poisson2D(np.linspace(0.0, 2.0, shape[0]), np.linspace(0.0, 1.0, shape[1]), kappa=kappa)
+    b = np.zeros(shape)
+    b[1:-1, 1:-1] = rng.standard_normal((shape[0] - 2, shape[1] - 2))
+    b = b.reshape(-1)
+    diag = op.diagonal().cpu().numpy()
+    for limit in (1, 2, 5):
+        x, dg = S.minimize_strong_formulation_residual(
+            op, torch.from_numpy(b).cuda(), settings=S.StrongFormulationSolverSettings(
+                max_iterations=limit, relative_tolerance=1e-9, precision=precision))
+        assert dg["iterations"] == limit and dg["converged"] == 0
+        ref = _numpy_cg(lambda v: op.apply(torch.from_numpy(v).cuda()).cpu().numpy(), diag, b, limit)
+        tol = 1e-12 if precision == "fp64" else 3e-4
+        assert np.linalg.norm(x.cpu().numpy() - ref) <= tol * np.linalg.norm(ref), limit

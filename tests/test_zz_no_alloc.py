@@ -95,3 +95,33 @@ def test_noalloc_refuses_what_it_cannot_hold():
                                                                   ctypes.byref(st), ctypes.byref(d), None)
     assert rc == L.SIL_ERR_UNSUPPORTED and b"FP64 only" in L.lib().sil_last_error()
     assert torch.count_nonzero(x) == 0  # nothing ran
+
+
+@pytest.mark.parametrize("kind", ["poisson", "magnetostatics"])
+def test_noalloc_into_a_solution_at_any_address(kind):
+    """a solution (and a right-hand side) 8 bytes off the vector alignment, an
+    odd number of unknowns: the bits of the aligned solve"""
+    from similie_amd import _lib as L
+    from similie_amd import solvers as S
+
+    if kind == "poisson":
+        op, b = poisson(97, 6)
+    else:
+        rng = np.random.default_rng(8)
+        coords = [np.cumsum(rng.uniform(0.5, 1.5, m)) for m in (13, 9, 11)]
+        op = S.MagnetostaticsOperator3D(*coords, torch.from_numpy(rng.uniform(1.0, 3.0, 13 * 9 * 11)).cuda(),
+                                        gauge_penalty=0.5)
+        b = torch.from_numpy(rng.standard_normal(op.size())).cuda()
+    n = b.numel()
+    assert n % 2 == 1
+    st = settings(L, L.PRECOND_JACOBI)
+    x_ref, d_ref, x_new, _ = solve_both(L, op, b, st)
+    assert torch.equal(x_ref, x_new)
+    buf, rhs = torch.full((n + 2,), -7.5, dtype=torch.float64, device="cuda"), torch.zeros_like(torch.cat([b, b[:1]]))
+    rhs[1:].copy_(b)
+    x, d = buf[1:1 + n], L.SolverDiagnostics()
+    assert buf.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 8
+    L.check(L.lib().sil_minimize_strong_formulation_residual_noalloc(op.handle, L.ptr(rhs[1:]), L.ptr(x),
+                                                                     ctypes.byref(st), ctypes.byref(d), None))
+    assert d.as_dict()["iterations"] == d_ref["iterations"] and torch.equal(x, x_ref)
+    assert float(buf[0]) == -7.5 and float(buf[-1]) == -7.5
