@@ -1,16 +1,20 @@
-// Batched persistent solver: many independent 2D Dirichlet Poisson problems
-// of uneven size in one launch.
+// Batched solver: many independent 2D Dirichlet Poisson problems of uneven
+// size at once.
 //
-// No reference counterpart: SimiLie solves one operator per Ginkgo call.  A
-// persistent grid of workgroups pulls problems from a device work queue
-// (largest first); each workgroup runs a whole CG solve for its problem with
-// workgroup-level reductions and barriers only.  The recurrence (r, p, q, and
-// every operator application inside the loop) is FP32 while x, all dot
+// No reference counterpart: SimiLie solves one operator per Ginkgo call.
+// Large problems take the wide path below, two kernels a step over all of
+// them; the others, beside it on a stream of their own, the persistent kernel:
+// its grid of workgroups pulls problems from a device work queue (largest
+// first), each workgroup runs a whole CG solve for its problem with
+// workgroup-level reductions and barriers only.  In both the recurrence (r, p,
+// q, and every operator application inside the loop) is FP32 while x, all dot
 // products and the scalars are FP64; the residual is replaced by the FP64
 // residual b − A x (FP64 edge weights) whenever the recurrence reports
 // convergence or every `replace` iterations, and a problem is declared solved
-// only on that FP64 residual.  The launch (queue reset + solve) is captured
-// into a hipGraph by the host.  Workgroup size is chosen by the autotuner.
+// only on that FP64 residual.  The launches (queue reset + persistent solve;
+// chunks of wide steps) are captured into hipGraphs by the host.  The line
+// between the paths, the workgroups of a wide problem and the persistent
+// kernel's workgroup size are chosen by the autotuner.
 #include <algorithm>
 #include <chrono>
 #include <cmath>

@@ -12,12 +12,13 @@
 // (reduce_all, cg_begin): β, the stopping test ‖r‖2 ≤ tol·‖b‖2 and the
 // iteration counter in K1 of the next iteration, α in K2.  A kernel of one
 // workgroup for each of the two (k_alpha, k_beta, still used where an
-// operator's partials are too many or K1 cannot sum them) took 4.5 µs a time,
-// more than the vectors of a small system.  Every scalar stays in device
-// memory, every kernel returns at once when the solve is over, and a chunk of
-// iterations, ended by a kernel that settles the scalars, is captured once
-// into a hipGraph and replayed; the host reads the flag once per chunk.
-// Partial sums are reduced in a fixed order, so a solve is bit-reproducible.
+// operator's partials are too many, kMaxSharedPartials, or K1 cannot sum them)
+// took 4.5 µs a time, more than the vectors of a small system.  Every scalar
+// stays in device memory, every kernel returns at once when the solve is over,
+// and a chunk of iterations, ended by a kernel that settles the scalars, is
+// captured once into a hipGraph and replayed; the host reads the flag once per
+// chunk.  Partial sums are reduced in a fixed order, so a solve is
+// bit-reproducible.
 //
 // Mixed precision: the recurrence (r, p, q) and every operator application
 // inside the loop run in FP32 while x, all dot products and the scalars are
@@ -70,7 +71,10 @@ constexpr int kUpdBlock = 256;
 constexpr int kUpdBlocks = 2048;
 constexpr int kRedThreads = 1024;
 // most partials of an operator application that every workgroup of the update
-// sums itself
+// sums itself.  (Not in the single-pass iteration, whose three arrays are summed
+// by a wavefront each at any size: a march of so many workgroups gives the
+// update milliseconds of vectors, 5016 partials on 449³ nodes 1738 µs at 5.0
+// TB/s, the rate it has with 1932 on 321³.)
 constexpr int kMaxSharedPartials = 2048;
 
 // workgroups of an update over n rows of `width` bytes: one 16-byte vector a

@@ -32,8 +32,10 @@
 // included (640: 30 wavefronts), where 256 threads walked the tile in three
 // passes on 12; each row leaves in 16-byte pairs; and the curve's brackets
 // are searched in LDS (the whole table there would cost a workgroup a compute
-// unit: 213 µs).  160 × 144 × 128 cells: 178 → 157 (640 threads) → 152
-// (pairs) → 147 µs, 3.2 TB/s of the bytes it cannot do without.
+// unit: 213 µs).  160 × 144 × 128 cells, inputs from HBM: 178 → 157 (640
+// threads) → 152 (pairs) → 147 µs, 3.2 TB/s of the bytes it cannot do without;
+// 107 µs where the pass before read the same 119 MB of inputs and the 256 MB
+// cache in front of HBM still holds them.
 #include <cstdlib>
 
 #include "bh_curve.hpp"

@@ -14,8 +14,8 @@ import oracle_lib as orc
 
 pytestmark = pytest.mark.gpu
 
-# every coefficient is a product of N factors each within about 4 ulp, every
-# result a sum of at most 30 products: 30 · (3·4 + 2) ulp ≈ 1e-13
+# every coefficient is a quotient of products of N factors, within about 4 ulp
+# for each, every result a sum of at most 30 products: 30 · (3·4 + 2) ulp ≈ 1e-13
 TOL = 1e-13
 
 
